@@ -54,260 +54,114 @@ struct BatchArgs {
   uint32_t *ghist;         // per workgroup drain area (16-bit path), zero at rest
   int H;
   int nmi32;     // reference float-order NMI (ISO_COMPAT_NMI32)
-  int list_cap;  // float2 entries per chain list in the dynamic LDS (nmi32)
-  float *stage;  // nmi32: a staging area of nmi32_stage_bytes(H) per workgroup
+  int hist_bytes;         // LDS histogram
+  iso::ChainBufs chains;  // nmi32: the chains' inputs, per task
 };
 
-constexpr int kBBlock = 1024;
-constexpr int kBWaves = kBBlock / 64;
-constexpr int kBRoundVpt = 8;
-constexpr int kBRound = kBBlock * kBRoundVpt;
-constexpr int kBDepth = 1;  // rounds per drain decision (2 spills registers here)
-constexpr int kBSuper = kBRound * kBDepth;
-constexpr uint32_t kBLimit16 = 65535u - kBSuper;
+constexpr int kBBlock = iso::kHistBlock;
 
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
+// Everything a workgroup keeps in LDS, after the histogram.
+template <bool PACK16>
+struct BatchLds {
+  iso::PairLds<PACK16> pair;
+  double red[3][iso::kHistWaves];
+  uint32_t prog[2];
+  int task, flushed;
+};
 
 template <bool PACK16>
-__global__ __launch_bounds__(kBBlock) void hist_batch_kernel(BatchArgs a) {
-  extern __shared__ uint32_t s_hist[];
-  __shared__ uint32_t s_rows[256], s_cols[256];
-  __shared__ double s_red[3][kBWaves];
-  __shared__ int s_task, s_flag[3], s_flushed;
-  __shared__ iso::Nmi32Lds s_nmi;
-  const int tid = threadIdx.x, H = a.H, HH = H * H;
-  const int words = PACK16 ? (HH + 1) >> 1 : HH;
-  uint32_t *gh = a.ghist + (int64_t)blockIdx.x * HH;
-  for (int w = tid; w < words; w += kBBlock) s_hist[w] = 0u;
+__global__ __launch_bounds__(kBBlock) __attribute__((amdgpu_waves_per_eu(PACK16 ? 4 : 8))) void hist_batch_kernel(BatchArgs a) {
+  extern __shared__ uint4 s_dyn[];
+  uint32_t *s_hist = reinterpret_cast<uint32_t *>(s_dyn);
+  BatchLds<PACK16> &s = *reinterpret_cast<BatchLds<PACK16> *>(s_hist + a.H * iso::kRowWords);
+  const int tid = threadIdx.x, H = a.H;
+  const int words = H * iso::kRowWords;
+  uint32_t *gh = a.ghist + (int64_t)blockIdx.x * H * H;
   while (true) {
-    if (tid == 0) s_task = (int)atomicAdd(a.next, 1u);
-    if (tid < 256) { s_rows[tid] = 0u; s_cols[tid] = 0u; }
-    if (tid == 0) { s_flag[0] = s_flag[1] = s_flag[2] = 0; s_flushed = 0; }
+    if (tid == 0) {
+      s.task = (int)atomicAdd(a.next, 1u);
+      s.prog[0] = s.prog[1] = 0u;
+      s.flushed = 0;
+    }
+    iso::clear_hist(s_hist, words);
+    iso::clear_pair_lds(s.pair);
     __syncthreads();
     // wave-uniform (the LDS read is not known to be): the task's pointers
     // then live in scalar registers and the buffer resources built from them
     // need no per-lane waterfall
-    const int ti = __builtin_amdgcn_readfirstlane(s_task);
+    const int ti = __builtin_amdgcn_readfirstlane(s.task);
     if (ti >= a.ntasks) break;
     const BatchTask t = a.tasks[ti];
     const float *f1 = a.fields + t.fi, *f2 = a.fields + t.fj;
     // the pair's bins (JointHistogram.cu:127-129): union range, H bins
-    iso::Binner bin;
+    iso::PairBins<PACK16> bin;
     bin.init(fminf(a.mins[t.mm_i], a.mins[t.mm_j]), fmaxf(a.maxs[t.mm_i], a.maxs[t.mm_j]), H);
-    auto drain = [&]() {
+    for (int64_t b = 0; b < t.processed; b += iso::kMaxSlice) {  // (once)
+      const int len = (int)min(iso::kMaxSlice, t.processed - b);
+      auto accumulate = [&](auto sub) {
+        constexpr bool SUB = decltype(sub)::value;
+        if constexpr (PACK16)
+          iso::accumulate16<SUB, 2>(bin, f1 + b, f2 + b, len, s_hist, s.prog, [&](int i, int j) {
+            atomicAdd(&gh[i * H + j], 32768u);
+            s.flushed = 1;
+          });
+        else
+          iso::accumulate32<SUB, 8>(bin, f1 + b, f2 + b, len, s_hist);
+      };
+      if (__builtin_amdgcn_readfirstlane(bin.subtract)) accumulate(std::true_type());
+      else accumulate(std::false_type());
+      __syncthreads();
+      if (tid == 0) s.prog[0] = s.prog[1] = 0u;
+      __syncthreads();
+    }
+    uint32_t *src = nullptr;  // where the pair's counts are
+    if (PACK16 && s.flushed) {
+      src = gh;
       for (int w = tid; w < words; w += kBBlock) {
-        uint32_t v = s_hist[w];
-        if (v) {
-          if (PACK16) {
-            if (v & 0xffffu) gh[2 * w] += v & 0xffffu;
-            if (v >> 16) gh[2 * w + 1] += v >> 16;
-          } else {
-            gh[w] += v;
-          }
-          s_hist[w] = 0u;
-        }
+        const uint32_t v = s_hist[w];
+        const int r = w / iso::kRowWords, c = 2 * (w % iso::kRowWords);
+        if (v & 0xffffu) atomicAdd(&gh[r * H + c], v & 0xffffu);
+        if (v >> 16) atomicAdd(&gh[r * H + c + 1], v >> 16);
       }
-    };
-    if constexpr (PACK16) {
-      // The round structure of hist_nmi_kernel's 16-bit path: flag rotation
-      // over three slots, kBDepth rounds per drain decision, buffer loads
-      // bounded by the pair's end, and each round's registers refilled with
-      // the next super-round's values as soon as they are binned.
-      const int64_t end = t.processed;
-      uint32_t voff[kBRoundVpt];
-#pragma unroll
-      for (int u = 0; u < kBRoundVpt; ++u) voff[u] = 4u * (uint32_t)(u * kBBlock + tid);
-      auto rsrc = [&](const float *f, int64_t b) {
-        const int64_t left = end - b;
-        const int n = left <= 0 ? 0 : (left >= kBRound ? kBRound : (int)left);
-        return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(left > 0 ? f + b : f), 0,
-                                                 4 * n, iso::kBufferWord3);
-      };
-      float x[kBDepth][kBRoundVpt], y[kBDepth][kBRoundVpt];
-      auto load_round = [&](float (&xr)[kBRoundVpt], float (&yr)[kBRoundVpt], int64_t b) {
-        const auto r1 = rsrc(f1, b), r2 = rsrc(f2, b);
-#pragma unroll
-        for (int u = 0; u < kBRoundVpt; ++u) {
-          xr[u] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r1, voff[u], 0, 0));
-          yr[u] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r2, voff[u], 0, 0));
-        }
-      };
-#pragma unroll
-      for (int r = 0; r < kBDepth; ++r) load_round(x[r], y[r], (int64_t)r * kBRound);
-      auto super_round = [&](auto full_tag, int64_t base) {
-        constexpr bool FULL = decltype(full_tag)::value;
-        const int rem = FULL ? kBSuper : (int)(end - base);
-        bool hot = false;
-#pragma unroll
-        for (int r = 0; r < kBDepth; ++r) {
-          uint32_t e[kBRoundVpt], old[kBRoundVpt], sh[kBRoundVpt];
-          iso::joint_bins(bin, x[r], y[r], e);
-          load_round(x[r], y[r], base + kBSuper + (int64_t)r * kBRound);
-#pragma unroll
-          for (int u = 0; u < kBRoundVpt; ++u) {  // atomics back to back, returns examined after
-            const int o = (r * kBRoundVpt + u) * kBBlock;
-            old[u] = 0u;
-            sh[u] = 0u;
-            if (FULL || o + tid < rem) {
-              sh[u] = (e[u] & 1u) << 4;
-              old[u] = atomicAdd(&s_hist[e[u] >> 1], 1u << sh[u]);
-            }
-          }
-#pragma unroll
-          for (int u = 0; u < kBRoundVpt; ++u) hot |= ((old[u] >> sh[u]) & 0xffffu) >= kBLimit16;
-        }
-        return hot;
-      };
-      int fb = 0;
-      for (int64_t base = 0; base < end; base += kBSuper) {
-        const bool hot = base + kBSuper <= end
-                             ? super_round(std::integral_constant<bool, true>(), base)
-                             : super_round(std::integral_constant<bool, false>(), base);
-        const int fn = fb == 2 ? 0 : fb + 1;
-        if (hot) s_flag[fb] = 1;
-        if (tid == 0) s_flag[fn] = 0;
-        iso::lds_barrier();
-        if (s_flag[fb]) {
-          drain();  // this workgroup owns its drain area: plain adds
-          if (tid == 0) s_flushed = 1;
-          __syncthreads();
-        }
-        fb = fn;
-      }
-    } else {
-      // 8 values per lane and field per step through bounded buffer loads,
-      // the next step's loaded as soon as this step's are binned (as in
-      // hist_nmi_kernel's 32-bit path)
-      constexpr int kVpt = 8, kStep = kVpt * kBBlock;
-      const int64_t end = t.processed;
-      uint32_t voff[kVpt];
-#pragma unroll
-      for (int u = 0; u < kVpt; ++u) voff[u] = 4u * (uint32_t)(u * kBBlock + tid);
-      float x[kVpt], y[kVpt];
-      auto load = [&](int64_t b) {
-        const int64_t left = end - b;
-        const int n = left <= 0 ? 0 : (left >= kStep ? kStep : (int)left);
-        const auto r1 = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<float *>(left > 0 ? f1 + b : f1), 0, 4 * n, iso::kBufferWord3);
-        const auto r2 = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<float *>(left > 0 ? f2 + b : f2), 0, 4 * n, iso::kBufferWord3);
-#pragma unroll
-        for (int u = 0; u < kVpt; ++u) {
-          x[u] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r1, voff[u], 0, 0));
-          y[u] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r2, voff[u], 0, 0));
-        }
-      };
-      load(0);
-      for (int64_t b = 0; b < end; b += kStep) {
-        uint32_t e[kVpt];
-        iso::joint_bins(bin, x, y, e);
-        load(b + kStep);
-        if (b + kStep <= end) {
-#pragma unroll
-          for (int u = 0; u < kVpt; ++u) atomicAdd(&s_hist[e[u]], 1u);
-        } else {
-          const int rem = (int)(end - b);
-#pragma unroll
-          for (int u = 0; u < kVpt; ++u)
-            if (u * kBBlock + tid < rem) atomicAdd(&s_hist[e[u]], 1u);
-        }
-      }
-    }
-    __syncthreads();
-    const bool use_global = s_flushed;
-    if (use_global) {
-      drain();
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
       __syncthreads();
     }
+    // H made opaque here, so the tail's bin addresses are not hoisted out of
+    // the task loop (they would stay live, and spill, across the histogram)
+    int Hv = H;
+    asm volatile("" : "+v"(Hv));
     if (a.nmi32) {
-      // the reference's float order (iso_nmi.hpp) with this workgroup's own
-      // staging area; its windows overwrite the histogram's LDS, which is
-      // cleared again afterwards
-      // H made opaque here, so the tail's bin addresses are not hoisted out of
-      // the task loop (they would stay live, and spill, across the histogram)
-      int Hv = H;
-      asm volatile("" : "+v"(Hv));
-      auto count_at = [&](int e) -> uint32_t {
-        if (use_global) return gh[e];
-        return PACK16 ? (s_hist[e >> 1] >> ((e & 1) << 4)) & 0xffffu : s_hist[e];
-      };
-      auto take_at = [&](int e) -> uint32_t {
-        if (!use_global) return PACK16 ? (s_hist[e >> 1] >> ((e & 1) << 4)) & 0xffffu : s_hist[e];
-        const uint32_t c = gh[e];
-        gh[e] = 0u;  // zero bins already are
-        return c;
-      };
-      float *map = a.maps[t.job];
-      // this workgroup's own staging area (the grid is persistent)
-      auto claim = [&]() -> float * {
-        return (float *)((char *)a.stage + (size_t)blockIdx.x * iso::nmi32_stage_bytes(H));
-      };
-      auto release = [&]() {};
-      float *out_ij = map + (int64_t)t.map_i * t.n + t.map_j;
-      float *out_ji = map + (int64_t)t.map_j * t.n + t.map_i;
+      // the chains of the reference's float order, folded by fold_batch_kernel
       const bool mirror = t.map_i != t.map_j;
-      // the counts stay in registers (16 bits each with the packed
-      // histogram), unless the pair drained to the global one or an odd H
-      // puts a lane's bins across three packed words
-      if (PACK16 && (use_global || (H & 1)))
-        iso::nmi32_pair<16, 4, false>(count_at, s_hist, take_at, true, Hv, t.F, mirror, s_rows,
-                                      s_cols, claim, release, (float2 *)s_hist, a.list_cap,
-                                      s_nmi, out_ij, out_ji);
+      if (PACK16 && src)
+        iso::emit_chains<PACK16, PACK16>(s_hist, a.hist_bytes, src, Hv, mirror, s.pair, a.chains, ti);
       else
-        iso::nmi32_pair<PACK16 ? 16 : 8, PACK16 ? 4 : 2, true>(
-            count_at, s_hist, take_at, use_global, Hv, t.F, mirror, s_rows, s_cols, claim,
-            release, (float2 *)s_hist, a.list_cap, s_nmi, out_ij, out_ji);
-      for (int w = tid; w < words; w += kBBlock) s_hist[w] = 0u;
+        iso::emit_chains<PACK16, false>(s_hist, a.hist_bytes, nullptr, Hv, mirror, s.pair, a.chains,
+                                        ti);
+    } else {
+      iso::list_bins<PACK16>(s_hist, src, Hv, s.pair);
       __syncthreads();
-      continue;
-    }
-    double sxy = 0.0;
-    for (int e = tid; e < HH; e += kBBlock) {
-      uint32_t c;
-      if (use_global) {
-        c = gh[e];
-        gh[e] = 0u;
-      } else {
-        c = PACK16 ? (s_hist[e >> 1] >> ((e & 1) << 4)) & 0xffffu : s_hist[e];
+      const double v = iso::nmi64_pair<PACK16>(s_hist, src, Hv, t.F, s.pair, s.red);
+      if (tid == 0) {
+        float *map = a.maps[t.job];
+        map[(int64_t)t.map_i * t.n + t.map_j] = map[(int64_t)t.map_j * t.n + t.map_i] =
+            (v != v) ? 0.0f : (float)v;
       }
-      if (c) {
-        const double dc = (double)c;
-        sxy += dc * log(dc);
-        atomicAdd(&s_rows[e / H], c);
-        atomicAdd(&s_cols[e % H], c);
-      }
-    }
-    __syncthreads();
-    // LDS back to zero for the next task
-    for (int w = tid; w < words; w += kBBlock) s_hist[w] = 0u;
-    double sx = 0.0, sy = 0.0;
-    if (tid < H) {
-      const uint32_t r = s_rows[tid], c = s_cols[tid];
-      if (r) sx = (double)r * log((double)r);
-      if (c) sy = (double)c * log((double)c);
-    }
-    sxy = wave_sum(sxy);
-    sx = wave_sum(sx);
-    sy = wave_sum(sy);
-    if ((tid & 63) == 0) { s_red[0][tid >> 6] = sxy; s_red[1][tid >> 6] = sx; s_red[2][tid >> 6] = sy; }
-    __syncthreads();
-    if (tid == 0) {
-      double txy = 0, tx = 0, ty = 0;
-      for (int q = 0; q < kBWaves; ++q) { txy += s_red[0][q]; tx += s_red[1][q]; ty += s_red[2][q]; }
-      const double dN = (double)t.F, lnN = log(dN);
-      const double hx = lnN - tx / dN, hy = lnN - ty / dN, hxy = lnN - txy / dN;
-      const double val = 2.0 * (hx + hy - hxy) / (hx + hy);
-      const float out = (val != val) ? 0.0f : (float)val;
-      float *map = a.maps[t.job];
-      map[(int64_t)t.map_i * t.n + t.map_j] = out;
-      map[(int64_t)t.map_j * t.n + t.map_i] = out;
     }
     __syncthreads();
   }
+}
+
+// The float-order NMI of every task of a hist_batch_kernel launch.
+__global__ __launch_bounds__(64 * iso::kFoldWaves) void fold_batch_kernel(BatchArgs a) {
+  __shared__ iso::FoldLds s_fold;
+  const int64_t t0 = (int64_t)blockIdx.x * iso::kFoldPairs;
+  iso::fold_chains(a.chains, a.H, t0, a.ntasks, [&](int64_t i) {
+    const BatchTask t = a.tasks[i];
+    float *map = a.maps[t.job];
+    return iso::FoldOut{t.map_i != t.map_j, t.F, map + (int64_t)t.map_i * t.n + t.map_j,
+                        map + (int64_t)t.map_j * t.n + t.map_i};
+  }, s_fold);
 }
 
 }  // namespace
@@ -438,42 +292,54 @@ int iso_ism_batch(iso_ctx *ctx, iso_ism_job *jobs, int njobs, int extractor, int
   const int nt = (int)tasks.size();
   if (nt > 0) {
     const bool pack16 = H > 128;
-    const int per_cu = 1;  // one 1024-lane workgroup per CU (registers)
+    const int per_cu = pack16 ? 1 : 2;  // 1024-lane workgroups per CU (LDS)
     const int groups = std::min(nt, per_cu * ctx->cu_count);
     const bool nmi32 = (flags & ISO_COMPAT_NMI32) != 0;
-    // the float-order NMI lays its chain lists out in the histogram's LDS
-    const size_t hist_lds = 4 * (pack16 ? ((size_t)H * H + 1) / 2 : (size_t)H * H);
-    const size_t lds = nmi32 ? std::max<size_t>(hist_lds, 16384) : hist_lds;
+    const size_t hist_bytes = sizeof(uint32_t) * (size_t)H * iso::kRowWords;
+    const size_t lds = hist_bytes + (pack16 ? sizeof(BatchLds<true>) : sizeof(BatchLds<false>));
     if (pack16)
       ISO_HIP_CHECK(ctx, hipFuncSetAttribute((const void *)hist_batch_kernel<true>,
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, 131072));
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     else
       ISO_HIP_CHECK(ctx, hipFuncSetAttribute((const void *)hist_batch_kernel<false>,
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, 65536));
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     BatchArgs ba;
     ba.fields = (const float *)fields;
     ba.mins = d_mins;
     ba.maxs = d_maxs;
-    ba.ntasks = nt;
     ba.H = H;
     ba.nmi32 = nmi32 ? 1 : 0;
-    ba.list_cap = (int)(lds / 16);
-    auto launch = [&]() -> int {
-      ISO_TRY(iso::fill_u32(ctx, ba.next, 0u, 1));
-      if (pack16)
-        hipLaunchKernelGGL(hist_batch_kernel<true>, dim3(groups), dim3(kBBlock), lds, ctx->stream, ba);
-      else
-        hipLaunchKernelGGL(hist_batch_kernel<false>, dim3(groups), dim3(kBBlock), lds, ctx->stream, ba);
-      ISO_HIP_CHECK(ctx, hipGetLastError());
+    ba.hist_bytes = (int)hist_bytes;
+    // tasks of a launch: what the memory for the chains' inputs holds (a graph
+    // keeps its own; the tasks' largest field comes first)
+    const bool graph = (flags & ISO_BATCH_GRAPH) != 0;
+    const size_t per = nmi32 ? iso::chain_task_bytes(H, tasks[0].F) : 1;
+    const int most = (int)std::min<size_t>(
+        nt, std::max<size_t>(1, nmi32 ? ((size_t)(graph ? 1 : 4) << 30) / per : (size_t)nt));
+    auto launch = [&](const BatchTask *d_tasks) -> int {
+      for (int i0 = 0; i0 < nt; i0 += most) {
+        ba.tasks = d_tasks + i0;
+        ba.ntasks = std::min(most, nt - i0);
+        ISO_TRY(iso::fill_u32(ctx, ba.next, 0u, 1));
+        if (pack16)
+          hipLaunchKernelGGL(hist_batch_kernel<true>, dim3(groups), dim3(kBBlock), lds, ctx->stream, ba);
+        else
+          hipLaunchKernelGGL(hist_batch_kernel<false>, dim3(groups), dim3(kBBlock), lds, ctx->stream, ba);
+        if (nmi32)
+          hipLaunchKernelGGL(fold_batch_kernel,
+                             dim3((unsigned)((ba.ntasks + iso::kFoldPairs - 1) / iso::kFoldPairs)),
+                             dim3(64 * iso::kFoldWaves), 0, ctx->stream, ba);
+        ISO_HIP_CHECK(ctx, hipGetLastError());
+      }
       return ISO_OK;
     };
     const size_t tbytes = sizeof(BatchTask) * (size_t)nt, mbytes = sizeof(float *) * (size_t)njobs;
     const size_t hbytes = sizeof(uint32_t) * (size_t)groups * H * H;
-    const size_t sbytes = nmi32 ? (size_t)groups * iso::nmi32_stage_bytes(H) : 0;
-    ba.stage = nullptr;
-    if (flags & ISO_BATCH_GRAPH) {
+    const size_t cbytes = nmi32 ? per * (size_t)most + 512 : 0;
+    if (nmi32) ISO_TRY(iso::nmi_logs(ctx, &ba.chains.logs));
+    if (graph) {
       // the graph owns one buffer: tasks | maps | queue head | drain area |
-      // NMI staging; its key is the layout: the tasks, the launch shape and
+      // chains' inputs; its key is the layout: the tasks, the launch shape and
       // the inputs' addresses
       uint64_t key = 1469598103934665603ull;
       auto mix = [&](const void *p, size_t n) {
@@ -492,8 +358,8 @@ int iso_ism_batch(iso_ctx *ctx, iso_ism_job *jobs, int njobs, int extractor, int
       for (auto &e : ctx->graphs)
         if (e.key == key) ge = &e;
       const size_t o_maps = (tbytes + 255) & ~(size_t)255, o_head = o_maps + ((mbytes + 255) & ~(size_t)255);
-      const size_t o_hist = o_head + 256, o_stage = o_hist + ((hbytes + 255) & ~(size_t)255);
-      const size_t need = o_stage + sbytes;
+      const size_t o_hist = o_head + 256, o_chains = o_hist + ((hbytes + 255) & ~(size_t)255);
+      const size_t need = o_chains + cbytes;
       if (!ge) {
         if (ctx->graphs.size() >= 8) {  // keep a few layouts: drop the oldest
           ISO_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
@@ -509,23 +375,22 @@ int iso_ism_batch(iso_ctx *ctx, iso_ism_job *jobs, int njobs, int extractor, int
         char *gb = (char *)e.buf;
         ISO_HIP_CHECK(ctx, hipMemcpyAsync(gb, tasks.data(), tbytes, hipMemcpyHostToDevice, ctx->stream));
         ISO_TRY(iso::fill_u32(ctx, gb + o_hist, 0u, hbytes / 4));  // drain area: zero at rest
-        ba.tasks = (const BatchTask *)gb;
         ba.maps = (float *const *)(gb + o_maps);
         ba.next = (uint32_t *)(gb + o_head);
         ba.ghist = (uint32_t *)(gb + o_hist);
-        if (nmi32) ba.stage = (float *)(gb + o_stage);
-        hipGraph_t graph = nullptr;
+        if (nmi32) iso::chain_carve(ba.chains, gb + o_chains, most, H, tasks[0].F);
+        hipGraph_t captured = nullptr;
         ISO_HIP_CHECK(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-        const int rc = launch();
-        const hipError_t ce = hipStreamEndCapture(ctx->stream, &graph);
+        const int rc = launch((const BatchTask *)gb);
+        const hipError_t ce = hipStreamEndCapture(ctx->stream, &captured);
         if (rc != ISO_OK) {
-          if (graph) (void)hipGraphDestroy(graph);
+          if (captured) (void)hipGraphDestroy(captured);
           (void)hipFree(e.buf);
           return rc;
         }
         ISO_HIP_CHECK(ctx, ce);
-        const hipError_t ie = hipGraphInstantiate(&e.exec, graph, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(graph);
+        const hipError_t ie = hipGraphInstantiate(&e.exec, captured, nullptr, nullptr, 0);
+        (void)hipGraphDestroy(captured);
         if (ie != hipSuccess) {
           (void)hipFree(e.buf);
           ISO_HIP_CHECK(ctx, ie);
@@ -547,19 +412,18 @@ int iso_ism_batch(iso_ctx *ctx, iso_ism_job *jobs, int njobs, int extractor, int
       ISO_TRY(iso::ws_get(ctx, WS_PIPE_F, mbytes, false, &dmaps));
       ISO_TRY(iso::ws_get(ctx, WS_HIST_GLOBAL, hbytes, true, &gh));
       if (nmi32) {
-        void *st = nullptr;
-        ISO_TRY(iso::ws_get(ctx, WS_NMI_STAGE, sbytes, false, &st));
-        ba.stage = (float *)st;
+        void *c = nullptr;
+        ISO_TRY(iso::ws_get(ctx, WS_NMI_CHAINS, cbytes, false, &c));
+        iso::chain_carve(ba.chains, c, most, H, tasks[0].F);
       }
       ISO_HIP_CHECK(ctx, hipMemcpyAsync(dt, tasks.data(), tbytes, hipMemcpyHostToDevice,
                                         ctx->stream));
       ISO_HIP_CHECK(ctx, hipMemcpyAsync(dmaps, maps.data(), mbytes, hipMemcpyHostToDevice,
                                         ctx->stream));
-      ba.tasks = (const BatchTask *)dt;
       ba.next = (uint32_t *)dq;
       ba.maps = (float *const *)dmaps;
       ba.ghist = (uint32_t *)gh;
-      ISO_TRY(launch());
+      ISO_TRY(launch((const BatchTask *)dt));
     }
   }
   ISO_HIP_CHECK(ctx, hipEventRecord(ev[2], ctx->stream));

@@ -12,23 +12,32 @@
 //     voxel slice of it when there are too few pairs to fill 256 CUs); the
 //     pair's joint histogram is privatised in LDS (32-bit counters for
 //     H <= 128: 64 KB; 16-bit counters packed two per dword for H <= 256:
-//     128 KB of the 160 KB LDS);
-//   - bins are computed exactly: q = (v-min) * (1/step) is within H*2^-23 of
-//     the true quotient, so whenever frac(q) is at least H*2^-19 away from an
-//     integer, trunc(q) equals the reference's trunc((v-min)/step); the rare
-//     remaining values take the IEEE division;
-//   - 16-bit counters never wrap: after every 8192-voxel round the workgroup
-//     checks a flag raised by any counter above 65535-8192 and, if set,
-//     drains LDS into a 32-bit global histogram;
-//   - slices of one pair (and drained pairs) merge in a global 32-bit
-//     histogram; the last slice to arrive (acq/rel counter) evaluates NMI
-//     and restores the zeros, so the buffer is zero at rest;
-//   - NMI is fused into the same kernel; only the float result leaves the
-//     chip.  With ISO_COMPAT_NMI32 it is the reference's float evaluation
-//     in the reference's order (iso_nmi.hpp); without it, the same quantity
-//     from the exact integer counts in double (sum c ln c);
-//   - workgroup ids are remapped so consecutive pairs (sharing field i) run
-//     on the same XCD and hit its L2.
+//     128 KB of the 160 KB LDS), 128 words to a row whatever H is;
+//   - bins are computed exactly in fixed point, and 16-bit counters hand on
+//     32,768 of their count before they can wrap (iso_bins.hpp);
+//   - slices of one pair (and what 16-bit counters handed on) merge in a global
+//     32-bit histogram; the last slice to arrive (acq/rel counter) takes the sum
+//     back into its LDS and restores the zeros, so the buffer is zero at rest;
+//   - with ISO_COMPAT_NMI32 the NMI is the reference's float evaluation in the
+//     reference's order: the workgroup writes the pair's nonzero counts out in
+//     both chain orders and a second kernel folds the chains of all pairs
+//     (iso_nmi.hpp); without it, the same quantity from the exact integer
+//     counts in double (sum c ln c), in the same kernel;
+//   - pairs come in tiles of 4 x 8 fields (12 fields for 32 pairs), and
+//     workgroup ids are remapped so that a tile's pairs run on one XCD at a time
+//     and share their fields in its L2 (row by row, 33 fields for 32 pairs, the
+//     launch read 13.6 GB past the L2s on the 600x248x248 front at 100
+//     isovalues, tiled 10.3 GB; those reads reach 7 TB/s, also where the
+//     256 MB cache holds them).
+//
+// 600x248x248 front, 100 isovalues, 256 bins (5,050 pairs of 576,600 voxels):
+// 3.04 -> 2.0 ms + 0.09 ms for the chains.  The counting's floor is its vector
+// instructions, 11 per pair of values at 4 cycles per wave: 0.9 ms; on top come
+// the rare exact divisions, LDS conflicts between lanes that meet in a counter
+// (2.4e8 cycles over the CUs), the pairs' starts and the lists (0.3 ms), which
+// one workgroup per CU cannot hide.  128 bins (2,016 pairs of 2^20 voxels, two
+// workgroups per CU): 1.55 -> 1.3 ms, at 9.4 GB past the L2s bound by those
+// reads; 256 isovalues of 60,000 voxels (32,896 pairs): 4.9 -> 2.1 ms.
 #include "iso_internal.hpp"
 #include "iso_bins.hpp"
 #include "iso_nmi.hpp"
@@ -42,15 +51,13 @@
 
 namespace {
 
-constexpr int kBlock = 1024;
+constexpr int kBlock = iso::kHistBlock;
 constexpr int kWaves = kBlock / 64;
-constexpr int kRoundVpt = 8;                     // voxels per lane per 16-bit round
-constexpr int kRound = kBlock * kRoundVpt;       // voxels per round
-// DEPTH (a template parameter, picked by the autotuner): with 16-bit
-// counters, the rounds between drain decisions (a counter grows by at most
-// DEPTH * kRound between them, which the drain threshold leaves room for);
-// with 32-bit counters, the values per lane and field loaded per step.
+// Pairs of a tile of the pair matrix (4 x 8), which is also the workgroups of
+// 16-bit counters that an XCD runs at once (one per CU, 32 CUs).
+constexpr int kTileRows = 4, kTileCols = 8, kTilePairs = kTileRows * kTileCols;
 constexpr int kMaxTasksPerLaunch = 16384;  // one launch per 128-isovalue ISM (no tail wave)
+constexpr size_t kMaxChainBytes = (size_t)4 << 30;  // chains' inputs of a launch
 
 struct HistArgs {
   const float *fields;
@@ -73,336 +80,196 @@ struct HistArgs {
   uint32_t *cols;
   int nxcd;
   int nmi32;     // reference float-order NMI (ISO_COMPAT_NMI32)
-  int list_cap;  // float2 entries per chain list in the dynamic LDS (nmi32)
-  float *stage;         // nmi32: nslots staging areas of nmi32_stage_bytes(H)
-  uint32_t *slot_bits;  // nmi32: free-slot bitmap, zero at rest
-  int slot_words;       // nmi32: bitmap words per XCD
-  int slots_per_word;   // nmi32: staging slots behind each bitmap word
+  int hist_bytes;         // LDS histogram
+  iso::ChainBufs chains;  // nmi32: the chains' inputs, per task
 };
 
-using iso::Binner;
-
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+// A wave-uniform value in a scalar register, however it was computed (integer
+// divisions run on the vector unit): the fields' pointers that come from it then
+// stay scalar, and their buffer loads need no per-lane waterfall.
+__device__ __forceinline__ int scalar(int v) {
+  asm volatile("" : "+v"(v));
+  return __builtin_amdgcn_readfirstlane(v);
 }
 
-using iso::lds_barrier;
-using iso::kBufferWord3;
-
+// Everything a workgroup keeps in LDS, the histogram first: at address 0 its
+// atomics need no base added.
 template <bool PACK16>
-__device__ __forceinline__ uint32_t lds_count(const uint32_t *s, int e) {
-  if (PACK16) return (s[e >> 1] >> ((e & 1) << 4)) & 0xffffu;
-  return s[e];
-}
+struct HistLds {
+  iso::PairLds<PACK16> pair;
+  double red[3][kWaves];
+  uint32_t prog[2];
+  int flushed, last;
+};
 
-template <bool PACK16, int DEPTH>
+// STEP (picked by the autotuner): rounds of 8 values per lane and field on their
+// way (16-bit counters), values per step (32-bit ones).
+template <bool PACK16, int STEP>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(PACK16 ? 4 : 8))) void hist_nmi_kernel(HistArgs a) {
-  extern __shared__ uint32_t s_hist[];
-  __shared__ uint32_t s_rows[256];
-  __shared__ uint32_t s_cols[256];
-  __shared__ double s_red[3][kWaves];
-  __shared__ int s_flag[3], s_flushed, s_last;
-  __shared__ uint32_t s_slot;
-  __shared__ iso::Nmi32Lds s_nmi;
+  extern __shared__ uint4 s_dyn[];
+  uint32_t *s_hist = reinterpret_cast<uint32_t *>(s_dyn);
+  HistLds<PACK16> &s = *reinterpret_cast<HistLds<PACK16> *>(s_hist + a.H * iso::kRowWords);
 
   const int tid = threadIdx.x;
   const int H = a.H;
   const int HH = H * H;
-  const int words = PACK16 ? (HH + 1) >> 1 : HH;
+  const int words = H * iso::kRowWords;
 
-  const uint32_t G = gridDim.x;
-  const uint32_t L = iso_xcd_remap(blockIdx.x, G, (uint32_t)a.nxcd);
-  const int task = (int)(L / (uint32_t)a.slices);
-  const int slice = (int)(L % (uint32_t)a.slices);
+  // Workgroups that run on an XCD at the same time take the pairs of one tile
+  // of the pair matrix, slice by slice, so each value read serves several of
+  // them from the XCD's L2.
+  const uint32_t L = iso_xcd_remap(blockIdx.x, gridDim.x, (uint32_t)a.nxcd);
+  const uint32_t per = (uint32_t)(kTilePairs * a.slices), tile = L / per, rem = L - tile * per;
+  const uint32_t pairs = min((uint32_t)kTilePairs, (uint32_t)a.ntasks - tile * kTilePairs);
+  const int task = scalar((int)(tile * kTilePairs + rem % pairs)), slice = scalar((int)(rem / pairs));
   const int2 tk = a.tasks[task];
   const int fi = tk.x, fj = tk.y;
 
-  for (int w = tid; w < words; w += kBlock) s_hist[w] = 0u;
-  if (tid < 256) { s_rows[tid] = 0u; s_cols[tid] = 0u; }
-  if (tid == 0) { s_flag[0] = s_flag[1] = s_flag[2] = 0; s_flushed = 0; s_last = 0; }
+  iso::clear_hist(s_hist, words);
+  iso::clear_pair_lds(s.pair);
+  if (tid == 0) { s.prog[0] = s.prog[1] = 0u; s.flushed = 0; s.last = 0; }
 
-  Binner bin;
+  iso::PairBins<PACK16> bin;
   {
     float mi = a.mins[fi], mj = a.mins[fj];
     float xi = a.maxs[fi], xj = a.maxs[fj];
     bin.init(mi < mj ? mi : mj, xi > xj ? xi : xj, H);
   }
-  const float *f1 = a.fields + (int64_t)fi * a.F;
-  const float *f2 = a.fields + (int64_t)fj * a.F;
   const int64_t begin = (int64_t)slice * a.chunk;
-  int64_t end = begin + a.chunk;
-  if (end > a.processed) end = a.processed;
+  const int len = (int)max((int64_t)0, min(a.chunk, a.processed - begin));
+  const float *f1 = a.fields + (int64_t)fi * a.F + begin;
+  const float *f2 = a.fields + (int64_t)fj * a.F + begin;
   uint32_t *gh = a.ghist + (int64_t)task * HH;
   __syncthreads();
 
-  auto drain = [&]() {
-    // LDS -> global 32-bit histogram of this task, leaves LDS zero
-    for (int w = tid; w < words; w += kBlock) {
-      uint32_t v = s_hist[w];
-      if (v) {
-        if (PACK16) {
-          uint32_t lo = v & 0xffffu, hi = v >> 16;
-          if (lo) atomicAdd(&gh[2 * w], lo);
-          if (hi) atomicAdd(&gh[2 * w + 1], hi);
-        } else {
-          atomicAdd(&gh[w], v);
-        }
-        s_hist[w] = 0u;
-      }
-    }
+  auto accumulate = [&](auto sub) {
+    constexpr bool SUB = decltype(sub)::value;
+    if constexpr (PACK16)
+      iso::accumulate16<SUB, STEP>(bin, f1, f2, len, s_hist, s.prog, [&](int i, int j) {
+        atomicAdd(&gh[i * H + j], 32768u);
+        s.flushed = 1;
+      });
+    else
+      iso::accumulate32<SUB, STEP>(bin, f1, f2, len, s_hist);
   };
-
-  if constexpr (PACK16) {
-    // Round r raises flag r%3; it is read after the round's barrier and
-    // cleared by thread 0 in round r+2 before that round's barrier, so no
-    // wave of a later round can touch it while a slow wave still reads it.
-    // A super-round is DEPTH rounds of 8 values per lane, loaded during the
-    // previous one: the rounds' atomics (8 back to back before any return
-    // value is examined), then one LDS-only barrier for the drain decision.
-    constexpr int kSuperRound = kRound * DEPTH;
-    constexpr uint32_t kLimit16 = 65535u - kSuperRound;  // drain threshold
-    int fb = 0;
-    // Loads go through buffer resources based at one round of the slice
-    // whose record count stops at the slice's end: a value past it reads as
-    // 0 without a memory access, so no load needs a bound.  A round's values
-    // are binned, then the same registers take the next super-round's values
-    // for that round, so those loads are in flight over this super-round's
-    // remaining atomics and its barrier.
-    uint32_t voff[kRoundVpt];
-#pragma unroll
-    for (int u = 0; u < kRoundVpt; ++u) voff[u] = 4u * (uint32_t)(u * kBlock + tid);
-    auto rsrc = [&](const float *f, int64_t b) {
-      const int64_t left = end - b;
-      const int n = left <= 0 ? 0 : (left >= kRound ? kRound : (int)left);
-      return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(left > 0 ? f + b : f), 0,
-                                               4 * n, kBufferWord3);
-    };
-    float x[DEPTH][kRoundVpt], y[DEPTH][kRoundVpt];
-    auto load_round = [&](float (&xr)[kRoundVpt], float (&yr)[kRoundVpt], int64_t b) {
-      const auto r1 = rsrc(f1, b), r2 = rsrc(f2, b);
-#pragma unroll
-      for (int u = 0; u < kRoundVpt; ++u) {
-        xr[u] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r1, voff[u], 0, 0));
-        yr[u] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r2, voff[u], 0, 0));
-      }
-    };
-#pragma unroll
-    for (int r = 0; r < DEPTH; ++r) load_round(x[r], y[r], begin + (int64_t)r * kRound);
-    // FULL: a whole super-round inside the slice, so no per-voxel bound
-    auto super_round = [&](auto full_tag, int64_t base) {
-      constexpr bool FULL = decltype(full_tag)::value;
-      const int rem = FULL ? kSuperRound : (int)(end - base);
-      bool hot = false;
-#pragma unroll
-      for (int r = 0; r < DEPTH; ++r) {
-        uint32_t e[kRoundVpt], old[kRoundVpt], sh[kRoundVpt];
-        iso::joint_bins(bin, x[r], y[r], e);
-        load_round(x[r], y[r], base + kSuperRound + (int64_t)r * kRound);
-#pragma unroll
-        for (int u = 0; u < kRoundVpt; ++u) {
-          const int o = (r * kRoundVpt + u) * kBlock;
-          old[u] = 0u;
-          sh[u] = 0u;
-          if (FULL || o + tid < rem) {
-            sh[u] = (e[u] & 1u) << 4;
-            old[u] = atomicAdd(&s_hist[e[u] >> 1], 1u << sh[u]);
-          }
-        }
-#pragma unroll
-        for (int u = 0; u < kRoundVpt; ++u) hot |= ((old[u] >> sh[u]) & 0xffffu) >= kLimit16;
-      }
-      return hot;
-    };
-    for (int64_t base = begin; base < end; base += kSuperRound) {
-      const bool hot = base + kSuperRound <= end
-                           ? super_round(std::integral_constant<bool, true>(), base)
-                           : super_round(std::integral_constant<bool, false>(), base);
-      const int fn = fb == 2 ? 0 : fb + 1;
-      if (hot) s_flag[fb] = 1;
-      if (tid == 0) s_flag[fn] = 0;
-      lds_barrier();
-      if (s_flag[fb]) {
-        drain();
-        if (tid == 0) s_flushed = 1;
-        lds_barrier();
-      }
-      fb = fn;
-    }
-  } else {
-    // DEPTH values per lane and field per step through bounded buffer loads
-    // (as in the 16-bit path); the next step's values load as soon as this
-    // step's are binned.  32-bit counters cannot wrap within a slice.
-    constexpr int kStep = DEPTH * kBlock;
-    uint32_t voff[DEPTH];
-#pragma unroll
-    for (int u = 0; u < DEPTH; ++u) voff[u] = 4u * (uint32_t)(u * kBlock + tid);
-    float x[DEPTH], y[DEPTH];
-    auto load = [&](int64_t b) {
-      const int64_t left = end - b;
-      const int n = left <= 0 ? 0 : (left >= kStep ? kStep : (int)left);
-      const auto r1 = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(left > 0 ? f1 + b : f1),
-                                                        0, 4 * n, kBufferWord3);
-      const auto r2 = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(left > 0 ? f2 + b : f2),
-                                                        0, 4 * n, kBufferWord3);
-#pragma unroll
-      for (int u = 0; u < DEPTH; ++u) {
-        x[u] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r1, voff[u], 0, 0));
-        y[u] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r2, voff[u], 0, 0));
-      }
-    };
-    load(begin);
-    for (int64_t b = begin; b < end; b += kStep) {
-      uint32_t e[DEPTH];
-      iso::joint_bins(bin, x, y, e);
-      load(b + kStep);
-      if (b + kStep <= end) {
-#pragma unroll
-        for (int u = 0; u < DEPTH; ++u) atomicAdd(&s_hist[e[u]], 1u);
-      } else {
-        const int rem = (int)(end - b);
-#pragma unroll
-        for (int u = 0; u < DEPTH; ++u)
-          if (u * kBlock + tid < rem) atomicAdd(&s_hist[e[u]], 1u);
-      }
-    }
-  }
+  if (__builtin_amdgcn_readfirstlane(bin.subtract)) accumulate(std::true_type());
+  else accumulate(std::false_type());
   __syncthreads();
 
-  const bool use_global = a.slices > 1 || s_flushed;
+  const bool use_global = a.slices > 1 || s.flushed;
   if (use_global) {
-    drain();
+    // LDS -> global 32-bit histogram of this task
+    for (int w = tid; w < words; w += kBlock) {
+      const uint32_t v = s_hist[w];
+      if (v) {
+        const int r = w / iso::kRowWords, c = w % iso::kRowWords;
+        if (PACK16) {
+          const uint32_t lo = v & 0xffffu, hi = v >> 16;
+          if (lo) atomicAdd(&gh[r * H + 2 * c], lo);
+          if (hi) atomicAdd(&gh[r * H + 2 * c + 1], hi);
+        } else {
+          atomicAdd(&gh[r * H + c], v);
+        }
+      }
+    }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
     __syncthreads();
     if (a.slices > 1) {
       if (tid == 0) {
         uint32_t old = __hip_atomic_fetch_add(&a.arrive[task], 1u, __ATOMIC_ACQ_REL,
                                               __HIP_MEMORY_SCOPE_AGENT);
-        s_last = (old == (uint32_t)a.slices - 1);
+        s.last = (old == (uint32_t)a.slices - 1);
       }
       __syncthreads();
-      if (!s_last) return;
+      if (!s.last) return;
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    }
+  }
+  // the merged counts back into LDS, unless one needs more than its counter
+  uint32_t *src = nullptr;  // where the pair's counts are, if not in LDS
+  if (use_global) {
+    bool fits = true;
+    for (int w = tid; w < words; w += kBlock) {
+      const int r = w / iso::kRowWords, c = (PACK16 ? 2 : 1) * (w % iso::kRowWords);
+      uint32_t v = c < H ? iso::pair_count<PACK16>(nullptr, gh, H, r, c) : 0u;
+      if (PACK16) {
+        const uint32_t hi = c + 1 < H ? iso::pair_count<PACK16>(nullptr, gh, H, r, c + 1) : 0u;
+        fits &= (v | hi) <= 0xffffu;
+        v |= hi << 16;
+      }
+      s_hist[w] = v;
+    }
+    if (PACK16) fits = __syncthreads_and(fits);
+    else __syncthreads();
+    if (fits) {
+      for (int e = tid; e < HH; e += kBlock) gh[e] = 0u;  // zero at rest
+    } else {
+      src = gh;
     }
   }
 
   const bool mirror = !a.multi && fi != fj;
   const int mj = a.multi ? fj - a.n : fj;
-  uint32_t *jout = a.joint ? a.joint + ((int64_t)fi * a.n + mj) * HH : nullptr;
-  uint32_t *jtr = (a.joint && mirror) ? a.joint + ((int64_t)fj * a.n + fi) * HH : nullptr;
-  auto write_marginals = [&]() {
-    if (tid < H && a.rows) {
-      const uint32_t r = s_rows[tid], c = s_cols[tid];
-      int64_t o = ((int64_t)fi * a.n + mj) * H + tid;
-      a.rows[o] = r;
-      a.cols[o] = c;
-      if (mirror) {
-        int64_t o2 = ((int64_t)fj * a.n + fi) * H + tid;
-        a.rows[o2] = c;
-        a.cols[o2] = r;
-      }
+  if (a.joint) {
+    // the joint histogram out (and its transpose for the mirrored entry),
+    // before the NMI reuses the LDS
+    uint32_t *jout = a.joint + ((int64_t)fi * a.n + mj) * HH;
+    uint32_t *jtr = mirror ? a.joint + ((int64_t)fj * a.n + fi) * HH : nullptr;
+    for (int e = tid; e < HH; e += kBlock) {
+      const uint32_t c = iso::pair_count<PACK16>(s_hist, src, H, e / H, e % H);
+      jout[e] = c;
+      if (jtr) jtr[(e % H) * H + e / H] = c;
     }
-  };
-
-  // ---- fused NMI in the reference's float order ----
+  }
   if (a.nmi32) {
-    if (jout) {
-      // the joint histogram out (and its transpose for the mirrored entry),
-      // before the NMI tail reuses the LDS
-      for (int e = tid; e < HH; e += kBlock) {
-        const uint32_t c = use_global ? gh[e] : lds_count<PACK16>(s_hist, e);
-        jout[e] = c;
-        if (jtr) jtr[(e % H) * H + e / H] = c;
-      }
-    }
-    auto count_at = [&](int e) -> uint32_t {
-      return use_global ? gh[e] : lds_count<PACK16>(s_hist, e);
-    };
-    auto take_at = [&](int e) -> uint32_t {
-      if (!use_global) return lds_count<PACK16>(s_hist, e);
-      const uint32_t c = gh[e];
-      gh[e] = 0u;  // restore zero at rest (zero bins already are)
-      return c;
-    };
-    // a staging slot of this XCD, claimed only when the chain lists do not
-    // fit in LDS
-    auto claim = [&]() -> float * {
-      if (tid == 0) s_slot = iso::nmi32_claim(a.slot_bits, a.slot_words, a.nxcd);
-      __syncthreads();
-      const uint32_t slot = s_slot;
-      // only the low slots_per_word bits of each word have staging behind them
-      const size_t stage_idx = (size_t)(slot >> 5) * (size_t)a.slots_per_word + (slot & 31u);
-      return (float *)((char *)a.stage + stage_idx * iso::nmi32_stage_bytes(H));
-    };
-    auto release = [&]() {
-      if (tid == 0) iso::nmi32_release(a.slot_bits, s_slot);
-    };
-    float *out_ij = a.map + (int64_t)fi * a.n + mj, *out_ji = a.map + (int64_t)fj * a.n + fi;
-    // the counts stay in registers (16 bits each with the packed histogram),
-    // unless the pair merged in the global one (where they may need 32) or
-    // an odd H puts a lane's bins across three packed words
-    if (PACK16 && (use_global || (H & 1)))
-      iso::nmi32_pair<16, 4, false>(count_at, s_hist, take_at, true, H, a.F, mirror, s_rows,
-                                    s_cols, claim, release, (float2 *)s_hist, a.list_cap, s_nmi,
-                                    out_ij, out_ji);
-    else if (PACK16)
-      iso::nmi32_pair<16, 4, true>(count_at, s_hist, take_at, false, H, a.F, mirror, s_rows,
-                                   s_cols, claim, release, (float2 *)s_hist, a.list_cap, s_nmi,
-                                   out_ij, out_ji);
+    // ---- the chains of the reference's float order, folded by fold_kernel
+    if (PACK16 && src)
+      iso::emit_chains<PACK16, PACK16>(s_hist, a.hist_bytes, src, H, mirror, s.pair, a.chains, task);
     else
-      iso::nmi32_pair<8, 2, true>(count_at, s_hist, take_at, use_global, H, a.F, mirror, s_rows,
-                                  s_cols, claim, release, (float2 *)s_hist, a.list_cap, s_nmi,
-                                  out_ij, out_ji);
-    write_marginals();
-    if (tid == 0 && use_global && a.slices > 1) a.arrive[task] = 0u;
-    return;
+      iso::emit_chains<PACK16, false>(s_hist, a.hist_bytes, nullptr, H, mirror, s.pair, a.chains,
+                                      task);
+  } else {
+    // ---- fused NMI from exact counts ----
+    iso::list_bins<PACK16>(s_hist, src, H, s.pair);
+    __syncthreads();
+    const double v = iso::nmi64_pair<PACK16>(s_hist, src, H, a.F, s.pair, s.red);
+    if (tid == 0) {
+      const float out = (v != v) ? 0.0f : (float)v;
+      a.map[(int64_t)fi * a.n + mj] = out;
+      if (mirror) a.map[(int64_t)fj * a.n + fi] = out;
+    }
   }
+  if (tid < H && a.rows) {  // (every form of the NMI ends its sums with a barrier)
+    const uint32_t r = s.pair.rows[tid], c = s.pair.cols[tid];
+    const int64_t o = ((int64_t)fi * a.n + mj) * H + tid;
+    a.rows[o] = r;
+    a.cols[o] = c;
+    if (mirror) {
+      const int64_t o2 = ((int64_t)fj * a.n + fi) * H + tid;
+      a.rows[o2] = c;
+      a.cols[o2] = r;
+    }
+  }
+  if (tid == 0 && use_global && a.slices > 1) a.arrive[task] = 0u;
+}
 
-  // ---- fused NMI from exact counts ----
-  double sxy = 0.0;
-  for (int e = tid; e < HH; e += kBlock) {
-    uint32_t c;
-    if (use_global) {
-      c = gh[e];
-      gh[e] = 0u;  // restore zero at rest
-    } else {
-      c = lds_count<PACK16>(s_hist, e);
-    }
-    if (c) {
-      double dc = (double)c;
-      sxy += dc * log(dc);
-      atomicAdd(&s_rows[e / H], c);
-      atomicAdd(&s_cols[e % H], c);
-    }
-    if (jout) jout[e] = c;
-    if (jtr) jtr[(e % H) * H + e / H] = c;
-  }
-  __syncthreads();
-  double sx = 0.0, sy = 0.0;
-  if (tid < H) {
-    uint32_t r = s_rows[tid], c = s_cols[tid];
-    if (r) sx = (double)r * log((double)r);
-    if (c) sy = (double)c * log((double)c);
-  }
-  write_marginals();
-  sxy = wave_sum(sxy);
-  sx = wave_sum(sx);
-  sy = wave_sum(sy);
-  const int wv = tid >> 6;
-  if ((tid & 63) == 0) { s_red[0][wv] = sxy; s_red[1][wv] = sx; s_red[2][wv] = sy; }
-  __syncthreads();
-  if (tid == 0) {
-    double txy = 0, tx = 0, ty = 0;
-    for (int k = 0; k < kWaves; ++k) { txy += s_red[0][k]; tx += s_red[1][k]; ty += s_red[2][k]; }
-    double dN = (double)a.F, lnN = log(dN);
-    double hx = lnN - tx / dN, hy = lnN - ty / dN, hxy = lnN - txy / dN;
-    double v = 2.0 * (hx + hy - hxy) / (hx + hy);
-    float out = (v != v) ? 0.0f : (float)v;
-    a.map[(int64_t)fi * a.n + mj] = out;
-    if (mirror) a.map[(int64_t)fj * a.n + fi] = out;
-    if (use_global && a.slices > 1) a.arrive[task] = 0u;
-  }
+// The float-order NMI of every task of a hist_nmi_kernel launch: kFoldPairs
+// tasks per workgroup.
+__global__ __launch_bounds__(64 * iso::kFoldWaves) void fold_kernel(HistArgs a) {
+  __shared__ iso::FoldLds s_fold;
+  const int64_t t0 = (int64_t)blockIdx.x * iso::kFoldPairs;
+  iso::fold_chains(a.chains, a.H, t0, a.ntasks, [&](int64_t t) {
+    const int2 tk = a.tasks[t];
+    const int mj = a.multi ? tk.y - a.n : tk.y;
+    return iso::FoldOut{!a.multi && tk.x != tk.y, a.F, a.map + (int64_t)tk.x * a.n + mj,
+                        a.map + (int64_t)tk.y * a.n + tk.x};
+  }, s_fold);
+}
+
+// logf of the counts 1 to kLogs - 1, 0 for 0
+__global__ void logs_kernel(float *logs) {
+  const int c = blockIdx.x * blockDim.x + threadIdx.x;
+  if (c < iso::kLogs) logs[c] = c ? iso::logf_cr((float)c) : 0.0f;
 }
 
 // ---- per-field (min, max), DistanceField::getInterval semantics ----
@@ -485,6 +352,21 @@ int field_interval(iso_ctx *ctx, const float *d_fields, int nfields, int64_t F, 
   return ISO_OK;
 }
 
+int nmi_logs_fill(iso_ctx *ctx, float *d_logs) {
+  hipLaunchKernelGGL(logs_kernel, dim3(kLogs / 256), dim3(256), 0, ctx->stream, d_logs);
+  ISO_HIP_CHECK(ctx, hipGetLastError());
+  return ISO_OK;
+}
+
+int nmi_logs(iso_ctx *ctx, const float **out) {
+  const bool first = !ctx->ws[WS_NMI_LOGS].ptr;
+  void *p = nullptr;
+  ISO_TRY(ws_get(ctx, WS_NMI_LOGS, sizeof(float) * kLogs, false, &p));
+  if (first) ISO_TRY(nmi_logs_fill(ctx, (float *)p));
+  *out = (const float *)p;
+  return ISO_OK;
+}
+
 // Launches the histogram+NMI kernel over a device task list.
 int hist_nmi_tasks(iso_ctx *ctx, const float *d_fields, int n, int64_t F, int H, int multi,
                    uint32_t flags, const float *d_mins, const float *d_maxs, float *d_map,
@@ -493,20 +375,16 @@ int hist_nmi_tasks(iso_ctx *ctx, const float *d_fields, int n, int64_t F, int H,
   if (ntasks <= 0) return ISO_OK;
   const bool pack16 = H > 128;
   const bool nmi32 = (flags & ISO_COMPAT_NMI32) != 0;
-  // float-order NMI: a staging slot per workgroup that fits on the device
-  // at once (one per CU with 16-bit counters, two with 32-bit ones), in
-  // whole bitmap words per XCD (slots are claimed on the claimant's XCD)
   HistBufs b;
-  const int nxcd = std::max(ctx->xcd_count, 1);
-  const int per_xcd = ((pack16 ? 1 : 2) * ctx->cu_count + nxcd - 1) / nxcd;
-  b.slot_words = (per_xcd + 31) / 32;
-  const size_t nslots = (size_t)b.slot_words * 32 * nxcd;
+  int most = kMaxTasksPerLaunch;
   if (nmi32) {
-    void *stage = nullptr, *bits = nullptr;
-    ISO_TRY(ws_get(ctx, WS_NMI_STAGE, nslots * nmi32_stage_bytes(H), false, &stage));
-    ISO_TRY(ws_get(ctx, WS_NMI_SLOTS, 4 * (size_t)b.slot_words * nxcd, true, &bits));
-    b.stage = (float *)stage;
-    b.slot_bits = (uint32_t *)bits;
+    // the chains' inputs, at most kMaxChainBytes of them (a launch's tasks)
+    const size_t per = chain_task_bytes(H, F);
+    most = (int)std::max<size_t>(1, std::min<size_t>(most, kMaxChainBytes / per));
+    void *c = nullptr;
+    ISO_TRY(ws_get(ctx, WS_NMI_CHAINS, per * (size_t)std::min(most, ntasks) + 512, false, &c));
+    chain_carve(b.chains, c, std::min(most, ntasks), H, F);
+    ISO_TRY(nmi_logs(ctx, &b.chains.logs));
   }
   int64_t processed = F;
   if (flags & ISO_COMPAT_HIST_CHUNKS) {
@@ -514,8 +392,8 @@ int hist_nmi_tasks(iso_ctx *ctx, const float *d_fields, int n, int64_t F, int H,
     if (F > 0 && F % C == 0) processed = F - C;
   }
   auto run = [&](int variant) -> int {
-    for (int t0 = 0; t0 < ntasks; t0 += kMaxTasksPerLaunch) {
-      int nt = ntasks - t0 < kMaxTasksPerLaunch ? ntasks - t0 : kMaxTasksPerLaunch;
+    for (int t0 = 0; t0 < ntasks; t0 += most) {
+      const int nt = std::min(ntasks - t0, most);
       void *gh = nullptr, *arr = nullptr;
       ISO_TRY(ws_get(ctx, WS_HIST_GLOBAL, sizeof(uint32_t) * (size_t)nt * H * H, true, &gh));
       ISO_TRY(ws_get(ctx, WS_HIST_ARRIVE, sizeof(uint32_t) * (size_t)nt, true, &arr));
@@ -528,13 +406,14 @@ int hist_nmi_tasks(iso_ctx *ctx, const float *d_fields, int n, int64_t F, int H,
   };
   const uint64_t key = ((uint64_t)H << 32) | ((uint64_t)ceil_log2((uint64_t)processed) << 16) |
                        (uint64_t)ceil_log2((uint64_t)ntasks);
-  return tune_pick(ctx, kTuneHist, key, 2, 1, pack16 ? "hist16 rounds/sync {1,2}" : "hist32 loads/step {4,8}", run);
+  return tune_pick(ctx, kTuneHist, key, 2, 1,
+                   pack16 ? "hist16 rounds ahead {1,2}" : "hist32 loads/step {4,8}", run);
 }
 
-// One launch of the histogram + NMI kernel over nt tasks with the caller's
+// One launch of the histogram + NMI kernels over nt tasks with the caller's
 // buffers (ghist: nt * H * H words and arrive: nt words, both zero at rest;
-// for ISO_COMPAT_NMI32 the staging slots and their bitmap).  Launch variant
-// 0 or 1 (the autotuner's choices).
+// for ISO_COMPAT_NMI32 the chains' inputs of nt tasks and the logarithms).
+// Launch variant 0 or 1 (the autotuner's choices).
 int hist_launch(iso_ctx *ctx, const float *d_fields, int n, int64_t F, int H, int multi,
                 uint32_t flags, const float *d_mins, const float *d_maxs, float *d_map,
                 const int2 *d_tasks, int nt, uint32_t *d_joint, uint32_t *d_rows,
@@ -542,19 +421,17 @@ int hist_launch(iso_ctx *ctx, const float *d_fields, int n, int64_t F, int H, in
   if (nt <= 0) return ISO_OK;
   const bool pack16 = H > 128;
   const bool nmi32 = (flags & ISO_COMPAT_NMI32) != 0;
-  const size_t words = pack16 ? ((size_t)H * H + 1) / 2 : (size_t)H * H;
-  // the float-order NMI reads its chain lists back through the histogram's
-  // LDS: at least 16 KB, windows of 1024 entries per list
-  const size_t lds = nmi32 ? std::max<size_t>(words * 4, 16384) : words * 4;
+  const size_t hist_bytes = sizeof(uint32_t) * (size_t)H * kRowWords;
+  const size_t lds = hist_bytes + (pack16 ? sizeof(HistLds<true>) : sizeof(HistLds<false>));
   int64_t processed = F;
   if (flags & ISO_COMPAT_HIST_CHUNKS) {
     const int64_t C = 1000000;
     if (F > 0 && F % C == 0) processed = F - C;
   }
-  // variants: 16-bit counters with 1 or 2 rounds per drain decision,
-  // 32-bit counters with 4 or 8 values per step (the autotuner picks; with
-  // the prefetch, 16 would take 96 registers and one workgroup per CU).
-  // The LDS limit is raised once per process, whatever thread gets here.
+  // variants: 16-bit counters with 1 or 2 rounds of 8 values on their way,
+  // 32-bit counters with 4 or 8 values per step (the autotuner picks; 16 would
+  // take too many registers for two workgroups per CU).  The LDS limit is
+  // raised once per process, whatever thread gets here.
   static std::once_flag attr_once;
   static hipError_t attr_err = hipSuccess;
   std::call_once(attr_once, [] {
@@ -563,16 +440,28 @@ int hist_launch(iso_ctx *ctx, const float *d_fields, int n, int64_t F, int H, in
                            (const void *)hist_nmi_kernel<true, 1>,
                            (const void *)hist_nmi_kernel<true, 2>};
     for (int v = 0; v < 4 && attr_err == hipSuccess; ++v)
-      attr_err = hipFuncSetAttribute(kern[v], hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     v < 2 ? 65536 : 131072);
+      attr_err = hipFuncSetAttribute(
+          kern[v], hipFuncAttributeMaxDynamicSharedMemorySize,
+          v < 2 ? 65536 + (int)sizeof(HistLds<false>) : 131072 + (int)sizeof(HistLds<true>));
   });
   ISO_HIP_CHECK(ctx, attr_err);
-  // enough workgroups to fill the chip, but at least 16K voxels per slice
-  int want = (2 * ctx->cu_count + nt - 1) / nt;
-  int64_t max_slices = processed / 16384;
-  if (max_slices < 1) max_slices = 1;
-  int slices = want < max_slices ? want : (int)max_slices;
-  if (slices < 1) slices = 1;
+  // Slices per pair, where the pairs alone leave CUs idle (one workgroup per CU
+  // with 16-bit counters, two with 32-bit ones): as few rounds of voxels as
+  // possible, a slice counting another 32K voxels' time for its start and the
+  // merge (10 us at 3 voxels per ns), with at least 16K voxels each.  136 pairs
+  // of 64^3 fields, 128 bins: 3 slices in one round 155 us, 4 in two 190 us.
+  // With a round or more of pairs, slices would only add merges (2,016 pairs of
+  // 128^3 fields, 256 bins: 3.7 ms, cut up to even the last round out 7.0 ms).
+  const int64_t cap = (int64_t)(pack16 ? 1 : 2) * ctx->cu_count;
+  int64_t slices = 1, best = INT64_MAX;
+  for (int64_t k = 1; nt < cap && k <= std::max<int64_t>(1, processed / 16384); ++k) {
+    const int64_t cost = (nt * k + cap - 1) / cap * (processed / k + (k > 1 ? 32768 : 0));
+    if (cost < best) {
+      best = cost;
+      slices = k;
+    }
+  }
+  slices = std::max(slices, (processed + kMaxSlice - 1) / kMaxSlice);
   const int64_t chunk = (processed + slices - 1) / slices;
   HistArgs a;
   a.fields = d_fields;
@@ -580,7 +469,7 @@ int hist_launch(iso_ctx *ctx, const float *d_fields, int n, int64_t F, int H, in
   a.processed = processed;
   a.tasks = d_tasks;
   a.ntasks = nt;
-  a.slices = slices;
+  a.slices = (int)slices;
   a.chunk = chunk;
   a.mins = d_mins;
   a.maxs = d_maxs;
@@ -595,37 +484,30 @@ int hist_launch(iso_ctx *ctx, const float *d_fields, int n, int64_t F, int H, in
   a.cols = d_cols;
   a.nxcd = ctx->xcd_count;
   a.nmi32 = nmi32 ? 1 : 0;
-  a.list_cap = (int)(lds / 16);
-  a.stage = b.stage;
-  a.slot_bits = b.slot_bits;
-  a.slot_words = b.slot_words;
-  a.slots_per_word = b.slots_per_word;
+  a.hist_bytes = (int)hist_bytes;
+  a.chains = b.chains;
   dim3 grid((unsigned)(nt * slices));
-  if (pack16) {
-    if (variant == 0)
-      hipLaunchKernelGGL((hist_nmi_kernel<true, 1>), grid, dim3(kBlock), lds, ctx->stream, a);
-    else
-      hipLaunchKernelGGL((hist_nmi_kernel<true, 2>), grid, dim3(kBlock), lds, ctx->stream, a);
-  } else {
-    if (variant == 0)
-      hipLaunchKernelGGL((hist_nmi_kernel<false, 4>), grid, dim3(kBlock), lds, ctx->stream, a);
-    else
-      hipLaunchKernelGGL((hist_nmi_kernel<false, 8>), grid, dim3(kBlock), lds, ctx->stream, a);
-  }
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(kBlock), lds, ctx->stream, a);
+  };
+  if (pack16) variant == 0 ? launch(hist_nmi_kernel<true, 1>) : launch(hist_nmi_kernel<true, 2>);
+  else variant == 0 ? launch(hist_nmi_kernel<false, 4>) : launch(hist_nmi_kernel<false, 8>);
+  ISO_HIP_CHECK(ctx, hipGetLastError());
+  if (nmi32)
+    hipLaunchKernelGGL(fold_kernel, dim3((unsigned)((nt + kFoldPairs - 1) / kFoldPairs)),
+                       dim3(64 * kFoldWaves), 0, ctx->stream, a);
   ISO_HIP_CHECK(ctx, hipGetLastError());
   return ISO_OK;
 }
 
-// Unordered pairs (i <= j) row by row, or all n*n (i, n+j) for multi.
+// Unordered pairs (i <= j), or all n*n pairs (i, n + j) for multi, in tiles.
 void build_tasks(int n, int multi, std::vector<int2> &t) {
   t.clear();
-  if (multi) {
-    for (int i = 0; i < n; ++i)
-      for (int j = 0; j < n; ++j) t.push_back(make_int2(i, n + j));
-  } else {
-    for (int i = 0; i < n; ++i)
-      for (int j = i; j < n; ++j) t.push_back(make_int2(i, j));
-  }
+  for (int i0 = 0; i0 < n; i0 += kTileRows)
+    for (int j0 = multi ? 0 : i0; j0 < n; j0 += kTileCols)
+      for (int i = i0; i < std::min(i0 + kTileRows, n); ++i)
+        for (int j = multi ? j0 : std::max(i, j0); j < std::min(j0 + kTileCols, n); ++j)
+          t.push_back(make_int2(i, multi ? n + j : j));
 }
 
 }  // namespace iso

@@ -13,26 +13,29 @@
 // visits the bins column by column, and its hX, hY are this pair's hY, hX
 // (their sum is the same float).
 //
-// On the GPU the chains are serial (one lane each) but short: only the
-// nonzero bins take part (about 1,500 of 65,536 for the 600x248x248 front at
-// 256 bins).  The whole workgroup first writes the nonzero counts in chain
-// order to a staging area in global memory; positions come from counts of
-// nonzero bins: a row-major position is the row's base (exclusive prefix of
-// the nonzero bins per row) plus the nonzero bins before it in its row (a
-// ballot prefix across the wave); a column-major position is the column's
-// base plus the nonzero bins above it in its column (per-wave column counts
-// and their prefix over the waves before).  Then the lists come back into
-// LDS window by window (coalesced), each lane taking the logarithms of the
-// counts it brings in, and one lane per chain folds the terms (c, logf(c)).
+// The chains are serial, so they are folded where many run side by side: the
+// histogram workgroup only writes a pair's nonzero counts out in both chain
+// orders, with the marginals, and fold_kernel (iso_hist.hip, iso_batch.hip)
+// folds the chains of all pairs of a launch, eight to a wave.  Folded by four
+// lanes of the histogram workgroup, the chains of 3,000 to 6,000 bins that
+// 128-bin maps have kept a whole CU waiting.
+//
+// A pair's counts lie over the workgroup's lanes as the histogram's rows do (a
+// wave has 16 or 8 consecutive rows, a lane 4 or 2 columns of them), so a bin's
+// place in row-major order is the number of bins in the rows before plus a
+// ballot prefix in its row, and in column-major order the number in the columns
+// before plus those in the rows above: a prefix over the waves, then counted up
+// row by row.
 #pragma once
 
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
 
-namespace iso {
+#include "iso_bins.hpp"
+#include "iso_internal.hpp"
 
-constexpr int kNmiBlock = 1024;  // lanes of the histogram workgroups
+namespace iso {
 
 // logf, correctly rounded for the counts it is applied to: the double
 // logarithm of the value, rounded once to float.  For every integer from 1
@@ -43,446 +46,623 @@ constexpr int kNmiBlock = 1024;  // lanes of the histogram workgroups
 // field has more than 16.2 million samples.
 __device__ __forceinline__ float logf_cr(float x) { return (float)log((double)x); }
 
+// Where a launch leaves what the chains need, per pair task: a header (number
+// of nonzero bins; 1 if a count needs 32 bits), the counts row by row and,
+// list_bytes after it, column by column (16 bits each, or 32), and the
+// marginals (H column sums, then H row sums).
+struct ChainBufs {
+  uint2 *head = nullptr;
+  unsigned char *lists = nullptr;  // 2 * list_bytes per task
+  size_t list_bytes = 0;           // a multiple of 16
+  uint32_t *marg = nullptr;        // 2 * H words per task
+  const float *logs = nullptr;     // logf of 0 (taken as 0) to kLogs - 1
+};
+constexpr int kLogs = 65536;
+
+// Room for one list: every nonzero bin, at most one per voxel, 32 bits each.
+__host__ __device__ inline size_t chain_list_bytes(int H, int64_t F) {
+  const int64_t n = (int64_t)H * H < F ? (int64_t)H * H : F;
+  return ((size_t)n * 4 + 15) & ~(size_t)15;
+}
+
+// Takes a launch's ChainBufs out of p (chain_task_bytes per task + 512).
+inline void chain_carve(ChainBufs &b, void *p, int64_t ntasks, int H, int64_t F) {
+  auto up = [](size_t n) { return (n + 255) & ~(size_t)255; };
+  char *q = (char *)p;
+  b.head = (uint2 *)q;
+  q += up(sizeof(uint2) * (size_t)ntasks);
+  b.marg = (uint32_t *)q;
+  q += up(2 * sizeof(uint32_t) * (size_t)H * (size_t)ntasks);
+  b.lists = (unsigned char *)q;
+  b.list_bytes = chain_list_bytes(H, F);
+}
+
+// Device bytes of ChainBufs per task (without the logarithms).
+__host__ __device__ inline size_t chain_task_bytes(int H, int64_t F) {
+  return sizeof(uint2) + 2 * chain_list_bytes(H, F) + 2 * sizeof(uint32_t) * (size_t)H;
+}
+
 // number of set bits of m in the lanes below this one
 __device__ __forceinline__ uint32_t lanes_below(uint64_t m) {
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
 }
 
-// LDS the float-order NMI uses beside the histogram kernels' own.
-struct Nmi32Lds {
-  uint8_t colpre[16][256];  // per wave: nonzero bins of column j in its 16 rows,
-                            // then those in the rows of the waves before it
-  uint32_t rowbase[256];    // nonzero bins per row, then their exclusive prefix
-  uint32_t colbase[256];    // exclusive prefix of the nonzero bins per column
-  // the marginals' chain terms (c, logf(c)), (0, 0) where c == 0
-  alignas(16) float2 mrow[256];
-  alignas(16) float2 mcol[256];
-  float2 mslack[16];  // read past mcol by the chain fold, never folded
+// LDS the NMI uses beside the histogram: nonzero bins per wave and column (then
+// those in the waves before), nonzero bins in the rows (columns) before, the
+// marginals and, for the double form, a list of nonzero bins (row << 8 | column).
+template <bool PACK16>
+struct PairLds {
+  static constexpr int kH = PACK16 ? 256 : 128;    // most bins per axis
+  static constexpr int kRows = kH / kHistWaves;    // rows of a wave
+  static constexpr int kCols = kH / 64;            // columns of a lane
+  static constexpr int kBins = 3072;  // most listed bins, 3 per lane
+  union {
+    uint8_t colpre[kHistWaves][kH];
+    uint16_t bins[kBins];
+  };
+  uint32_t rowbase[kH], colbase[kH];
+  uint32_t rows[kH], cols[kH];
+  uint32_t nbins, big;
   uint32_t wtot[8];
-  float acc[4];
 };
 
-// Staging of one workgroup: 2 * H * H float counts (row-major list, then
-// column-major list).
-__host__ __device__ constexpr size_t nmi32_stage_bytes(int H) {
-  return (size_t)2 * H * H * sizeof(float);
+// Clears the marginals and counters; a barrier comes before their use.
+template <bool PACK16>
+__device__ __forceinline__ void clear_pair_lds(PairLds<PACK16> &s) {
+  if (threadIdx.x < PairLds<PACK16>::kH) s.rows[threadIdx.x] = s.cols[threadIdx.x] = 0u;
+  if (threadIdx.x == 0) s.nbins = s.big = 0u;
 }
 
-// Terms per block of the chain fold: the lists in LDS are padded with (0, 0)
-// to a multiple of it, and fmaf(-0, 0, acc) is acc exactly.
-constexpr int kChainBlock = 16;
+// The count of bin (i, j): from the LDS histogram or, when gh is not null, from
+// the H x H counts there (read past this CU's cache: atomics put them there).
+template <bool PACK16>
+__device__ __forceinline__ uint32_t pair_count(const uint32_t *s_hist, const uint32_t *gh, int H,
+                                               int i, int j) {
+  if (gh) return __hip_atomic_load(&gh[i * H + j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return lds_count<PACK16>(s_hist, i, j);
+}
 
-// acc = fmaf(-c, t, acc) over the terms (c, t) = v[0], ..., v[n-1] in order.
-// v is 16-byte aligned; from n up to the next multiple of kChainBlock it
-// holds (0, 0), and the kChainBlock entries after that are readable (read,
-// never folded).  One lane runs it: blocks of 2 Q terms in two register
-// buffers of Q float4, each block's 16-byte LDS reads issued one block
-// ahead of its fold, no predication: per term one fma and half a read.
-template <int Q>
-__device__ __forceinline__ float fma_chain(const float2 *v, int n, float acc) {
-  static_assert(kChainBlock % (2 * Q) == 0, "block");
-  const float4 *p = reinterpret_cast<const float4 *>(v);
-  const int nq = ((n + kChainBlock - 1) / kChainBlock) * (kChainBlock / 2);
-  if (nq == 0) return acc;
-  float4 a[Q], b[Q];
-  auto load = [&](float4(&r)[Q], int q0) {
+// Bins of a lane in a row: two words of the LDS histogram.
+template <bool PACK16>
+constexpr int kSlotBins = PACK16 ? 4 : 2;
+
+// Slot k of the histogram is words 2 (k % 64) and + 1 of row k / 64; lane t of
+// the workgroup has slots t + 1024 q, q < kSlots.
+template <bool PACK16>
+constexpr int kSlots = PairLds<PACK16>::kH * 64 / kHistBlock;
+
+template <bool PACK16>
+__device__ __forceinline__ uint32_t slot_count(uint2 v, int c) {
+  if (PACK16) return ((c < 2 ? v.x : v.y) >> (16 * (c & 1))) & 0xffffu;
+  return c == 0 ? v.x : v.y;
+}
+
+// Counts the nonzero bins of the LDS histogram (or of gh) and lists the first
+// kBins of them, in any order.  The caller's barrier comes after; the number is
+// then s.nbins.
+template <bool PACK16>
+__device__ __attribute__((always_inline)) void list_bins(const uint32_t *s_hist, const uint32_t *gh,
+                                                         int H, PairLds<PACK16> &s) {
+  using L = PairLds<PACK16>;
+  constexpr int kPer = kSlotBins<PACK16>;
+  const int l = threadIdx.x & 63;
+  // kPer bits per slot of the lane: which of its bins are not zero
+  uint64_t nz = 0ull;
 #pragma unroll
-    for (int u = 0; u < Q; ++u) r[u] = p[q0 + u];
-  };
-  auto fold = [&](const float4(&r)[Q]) {
+  for (int q = 0; q < kSlots<PACK16>; ++q) {
+    const int k = q * kHistBlock + (int)threadIdx.x;
+    if (k >= H * 64) break;
+    uint2 v = make_uint2(0u, 0u);
+    if (!gh) v = reinterpret_cast<const uint2 *>(s_hist)[k];
 #pragma unroll
-    for (int u = 0; u < Q; ++u) {
-      acc = fmaf(-r[u].x, r[u].y, acc);
-      acc = fmaf(-r[u].z, r[u].w, acc);
+    for (int c = 0; c < kPer; ++c) {
+      const int j = (k & 63) * kPer + c;
+      const uint32_t n = !gh ? slot_count<PACK16>(v, c)
+                         : j < H ? pair_count<PACK16>(s_hist, gh, H, k >> 6, j) : 0u;
+      nz |= (uint64_t)(n != 0u) << (kPer * q + c);
     }
-  };
-  // reads stay below nq + Q float4: nq + 2 Q terms
-  load(a, 0);
-  load(b, Q);
-  for (int q = 0;; q += 2 * Q) {
-    fold(a);
-    if (q + Q >= nq) break;
-    load(a, q + 2 * Q);
-    fold(b);
-    if (q + 2 * Q >= nq) break;
-    load(b, q + 3 * Q);
   }
-  return acc;
+  const uint32_t n = (uint32_t)__popcll(nz);
+  // the lane's place in the wave's run, the wave's in the list
+  uint32_t incl = n;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t t = __shfl_up(incl, o, 64);
+    if (l >= o) incl += t;
+  }
+  const uint32_t tot = __shfl(incl, 63, 64);
+  uint32_t base = 0u;
+  if (tot && l == 0) base = atomicAdd(&s.nbins, tot);
+  uint32_t at = __builtin_amdgcn_readfirstlane(base) + incl - n;
+  // a list that is full already serves nobody
+  if (__builtin_amdgcn_readfirstlane(base) + tot > (uint32_t)L::kBins) return;
+  while (nz) {
+    const int b = __ffsll((unsigned long long)nz) - 1;
+    nz &= nz - 1ull;
+    const int k = (b / kPer) * kHistBlock + (int)threadIdx.x;
+    s.bins[at++] = (uint16_t)((k >> 6) << 8 | ((k & 63) * kPer + b % kPer));
+  }
 }
 
-// Bins a lane covers: lane (w, l) of the 16 waves holds bins (RW w + r,
-// CL l + c), r < RW, c < CL, so 16 RW rows and 64 CL columns must cover H
-// (RW 16, CL 4 up to 256 bins; RW 8, CL 2 up to 128, a quarter of the
-// registers).
-template <int RW, int CL>
-struct Nmi32Tile {
-  static_assert(RW * CL <= 64 && 16 * RW <= 256 && 64 * CL <= 256, "tile");
-  static constexpr int kBits = RW * CL;
-  // bits c, c + CL, c + 2 CL, ... of a lane's mask: column c of its tile
-  static constexpr uint64_t col_mask(int c) {
-    uint64_t m = 0;
-    for (int r = 0; r < RW; ++r) m |= 1ull << (CL * r + c);
-    return m;
+// f(i, j, count) for every nonzero bin of a pair whose bins are not listed.
+template <bool PACK16, class F>
+__device__ __forceinline__ void each_bin(const uint32_t *s_hist, const uint32_t *gh, int H, F f) {
+  constexpr int kPer = kSlotBins<PACK16>;
+  for (int k = threadIdx.x; k < H * 64; k += kHistBlock) {
+#pragma unroll
+    for (int c = 0; c < kPer; ++c) {
+      const int j = (k & 63) * kPer + c;
+      if (j < H) {
+        const uint32_t v = pair_count<PACK16>(s_hist, gh, H, k >> 6, j);
+        if (v) f(k >> 6, j, v);
+      }
+    }
   }
-  static constexpr uint64_t kRowBits = (1ull << CL) - 1ull;
-};
+}
 
-// The pair's joint counts are count_at(e), e = row * H + col (row from the
-// first field), H <= 16 RW and H <= 64 CL; with KEEP and the 64-bin tiles
-// they are read instead from `packed`, the LDS histogram of 16-bit counts two
-// to a word (H even).  KEEP: the counts stay in the lanes' registers from the
-// structure pass to the placement.  take_at(e) returns the count of a nonzero
-// bin; it is called once per nonzero bin, after every read of the counts,
-// where they are not kept or need_take is set (it may restore a zero behind
-// it).  Called by every lane of a 1024-lane workgroup, with uniform flags.
-// s_rows / s_cols: 256 zeroed LDS words, left holding the marginals (row
-// sums, column sums).  win: LDS room for 2 * cap float2, 16-byte aligned,
-// cap >= 2 kChainBlock, that no lane reads once every lane has passed the
-// first barrier in here.  With KEEP, when both chain lists fit there, they
-// are built in it directly; otherwise claim_stage() (called by every lane)
-// returns a global staging area of nmi32_stage_bytes(H) for them, and
-// release_stage() (every lane) hands it back after its last read.  Lane 0
-// writes the map entry (i, j) to *out_ij and, with mirror, the entry (j, i)
-// to *out_ji.  N is the field size.
-template <int RW, int CL, bool KEEP, class CountAt, class TakeAt, class Claim, class Release>
-__device__ __attribute__((always_inline)) void nmi32_pair(
-    CountAt count_at, const uint32_t *packed, TakeAt take_at, bool need_take, int H, int64_t N,
-    bool mirror, uint32_t *s_rows, uint32_t *s_cols, Claim claim_stage, Release release_stage,
-    float2 *win, int cap, Nmi32Lds &s, float *out_ij, float *out_ji) {
-  using T = Nmi32Tile<RW, CL>;
-  static_assert(RW == 8 || RW == 16, "rows per wave");
-  constexpr int kLogRW = RW == 16 ? 4 : 3;
-  // chain buffers: 2 x 8 float4 with the 256-bin tiles, 2 x 4 float4 with
-  // the smaller ones (whose kernels fit more workgroups per CU)
-  constexpr int CQ = RW >= 16 ? 8 : 4;
-  // KEEP: a lane's counts are kept from the structure pass to the placement,
-  // two 16-bit counts per register for the 64-bin tiles, one per register
-  // for the smaller ones
-  constexpr bool kPack = RW * CL > 16;
-  constexpr int kRegs = KEEP ? (kPack ? RW * CL / 2 : RW * CL) : 1;
+// Writes a pair's chain inputs out (task t of b).  The joint counts are in the
+// LDS histogram (hist_bytes of it, overwritten) or, with GH, in gh (H x H 32-bit
+// counts, set back to zero here).  s.rows and s.cols are zero and are left
+// holding the marginals.  mirror: the column-by-column list is wanted too.
+// Called by every lane of a 1024-lane workgroup with uniform arguments, after a
+// barrier.
+//
+// The counts wait in registers while their LDS takes the lists, so the lists
+// leave in coalesced stores (scattered 2-byte stores of some 4,000 bins to both
+// lists would cost the L2 8,000 transactions per pair).  Counts past 16 bits
+// (rare) go out one by one.
+template <bool PACK16, bool GH>
+__device__ __attribute__((always_inline)) void emit_chains(uint32_t *s_hist, int hist_bytes,
+                                                           uint32_t *gh, int H, bool mirror,
+                                                           PairLds<PACK16> &s, const ChainBufs &b,
+                                                           int64_t t) {
+  using L = PairLds<PACK16>;
+  constexpr int kH = L::kH, R = L::kRows, C = L::kCols;
+  constexpr int kLogR = PACK16 ? 4 : 3;
+  int tid = threadIdx.x;
   // the lane id made opaque: inside a persistent task loop, addresses derived
   // from it must not be hoisted out of the loop (they would stay live across
   // the histogram phase and spill)
-  int tid = threadIdx.x;
   asm volatile("" : "+v"(tid));
-  const int w = tid >> 6, l = tid & 63;
-  // bit CL r + c of `nzm` says whether bin (RW w + r, CL l + c) is nonzero
-  uint64_t nzm = 0ull;
-  // per row r: nonzero bins of the lanes below in the row, a byte each (at
-  // most CL * 63)
-  uint32_t rowpre[(RW + 3) / 4];
-  uint32_t reg[kRegs];
+  const int l = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int i0 = R * w, j0 = C * l;  // the lane's bins: rows i0 + r, columns j0 + c
+  uint2 slot[R];                     // the lane's two words of each row
 #pragma unroll
-  for (int q = 0; q < (RW + 3) / 4; ++q) rowpre[q] = 0u;
-  {
-    // without KEEP, the lane's row sums are kept instead
-    uint32_t csum[CL], rsum[KEEP ? 1 : RW];
+  for (int r = 0; r < R; ++r) {
+    slot[r] = make_uint2(0u, 0u);
+    if (!GH && i0 + r < H) slot[r] = reinterpret_cast<const uint2 *>(s_hist)[(i0 + r) * 64 + l];
+  }
+  auto count = [&](int r, int c) -> uint32_t {
+    if (GH)
+      return i0 + r < H && j0 + c < H ? pair_count<PACK16>(nullptr, gh, H, i0 + r, j0 + c) : 0u;
+    if (PACK16) return ((c < 2 ? slot[r].x : slot[r].y) >> (16 * (c & 1))) & 0xffffu;
+    return c == 0 ? slot[r].x : slot[r].y;
+  };
+  uint32_t csum[C], cnz[C], rsum[R], all = 0u;
 #pragma unroll
-    for (int c = 0; c < CL; ++c) csum[c] = 0u;
+  for (int c = 0; c < C; ++c) csum[c] = cnz[c] = 0u;
 #pragma unroll
-    for (int r = 0; r < RW; ++r) {
-      const int i = RW * w + r;
-      uint32_t n = 0u, rs = 0u;
-      if constexpr (KEEP && kPack) {
-        // the lane's 4 bins of row i are 16-bit halves of two words of the
-        // packed histogram (H even); halves past the row's end read as 0
-        uint32_t w0 = 0u, w1 = 0u;
-        if (i < H && CL * l < H) {
-          const int b = (i * H + CL * l) >> 1;
-          w0 = packed[b];
-          if (CL * l + 2 < H) w1 = packed[b + 1];
-        }
-        reg[2 * r] = w0;
-        reg[2 * r + 1] = w1;
-      }
+  for (int r = 0; r < R; ++r) {
+    uint32_t rs = 0u, n = 0u;
+    if (i0 + r < H) {
 #pragma unroll
-      for (int c = 0; c < CL; ++c) {
-        const int j = CL * l + c;
-        const int k = r * CL + c;
-        uint32_t v;
-        if constexpr (KEEP && kPack) {
-          v = (reg[k >> 1] >> (16 * (k & 1))) & 0xffffu;
-        } else {
-          v = (i < H && j < H) ? count_at(i * H + j) : 0u;
-          if (KEEP) reg[KEEP && !kPack ? k : 0] = v;
-        }
+      for (int c = 0; c < C; ++c) {
+        const uint32_t v = count(r, c);
         csum[c] += v;
+        cnz[c] += v != 0u;
         rs += v;
-        if (v) {
-          nzm |= 1ull << k;
-          ++n;
-        }
-      }
-      if (!KEEP) rsum[KEEP ? 0 : r] = rs;
-      // the lane's count n <= CL < 8, bit-sliced over three ballots
-      const uint64_t b0 = __ballot(n & 1u), b1 = __ballot(n & 2u), b2 = __ballot(n & 4u);
-      if (l == 0)
-        s.rowbase[i] =
-            (uint32_t)__popcll(b0) + 2u * (uint32_t)__popcll(b1) + 4u * (uint32_t)__popcll(b2);
-      const uint32_t pre = lanes_below(b0) + 2u * lanes_below(b1) + 4u * lanes_below(b2);
-      rowpre[r >> 2] |= pre << (8 * (r & 3));
-    }
-    // row sums over the wave's 64 lanes by halving exchanges: across lane
-    // bit 32, 16, ... a lane keeps the half of its rows that the bit selects
-    // and adds its partner's copy of that half (RW - 1 shuffles), then the
-    // low lane bits are summed; lane l ends with row l >> (6 - log2 RW).  The
-    // lane's own row sums come from its counts as the first exchange needs
-    // them.
-    auto own_row = [&](int r) -> uint32_t {
-      if (!KEEP) return rsum[r];
-      uint32_t t = 0u;
-#pragma unroll
-      for (int c = 0; c < CL; ++c) {
-        const int k = r * CL + c;
-        t += kPack ? (reg[KEEP ? k >> 1 : 0] >> (16 * (k & 1))) & 0xffffu : reg[KEEP ? k : 0];
-      }
-      return t;
-    };
-    uint32_t rsv[RW / 2];
-#pragma unroll
-    for (int t = 0; t < RW / 2; ++t) {
-      const bool up = (l & 32) != 0;
-      const uint32_t lo = own_row(t), hi = own_row(RW / 2 + t);
-      rsv[t] = (up ? hi : lo) + __shfl_xor(up ? lo : hi, 32, 64);
-    }
-#pragma unroll
-    for (int st = 1; st < kLogRW; ++st) {
-      const int half = RW >> (st + 1), sbit = 32 >> st;
-      const bool up = (l & sbit) != 0;
-#pragma unroll
-      for (int t = 0; t < half; ++t) {
-        const uint32_t give = up ? rsv[t] : rsv[half + t];
-        const uint32_t keep = up ? rsv[half + t] : rsv[t];
-        rsv[t] = keep + __shfl_xor(give, sbit, 64);
+        all |= v;
+        n += (uint32_t)__popcll(__ballot(v != 0u));
       }
     }
-    uint32_t tot = rsv[0];
+    rsum[r] = rs;
+    if (l == 0) s.rowbase[i0 + r] = n;
+  }
+  if (__ballot(all > 0xffffu) && l == 0) s.big = 1u;
+  // row sums over the wave's 64 lanes by halving exchanges: across lane bit 32,
+  // 16, ... a lane keeps the half of its rows that the bit selects and adds its
+  // partner's copy of that half (R - 1 shuffles), then the low lane bits are
+  // summed; lane l ends with row l >> (6 - kLogR)
 #pragma unroll
-    for (int o = 32 >> kLogRW; o > 0; o >>= 1) tot += __shfl_xor(tot, o, 64);
-    {
-      const int i = RW * w + (l >> (6 - kLogRW));
-      if ((l & ((64 >> kLogRW) - 1)) == 0 && i < H) s_rows[i] = tot;
+  for (int st = 0; st < kLogR; ++st) {
+    const int half = R >> (st + 1), sbit = 32 >> st;
+    const bool up = (l & sbit) != 0;
+#pragma unroll
+    for (int k = 0; k < half; ++k) {
+      const uint32_t give = up ? rsum[k] : rsum[half + k];
+      const uint32_t keep = up ? rsum[half + k] : rsum[k];
+      rsum[k] = keep + __shfl_xor(give, sbit, 64);
     }
+  }
+  uint32_t tot = rsum[0];
 #pragma unroll
-    for (int c = 0; c < CL; ++c) {
-      if (csum[c]) atomicAdd(&s_cols[CL * l + c], csum[c]);
-      s.colpre[w][CL * l + c] = (uint8_t)__popcll(nzm & T::col_mask(c));
-    }
-    // rows and columns beyond the tiles count no bins
+  for (int o = 32 >> kLogR; o > 0; o >>= 1) tot += __shfl_xor(tot, o, 64);
+  if ((l & ((64 >> kLogR) - 1)) == 0) s.rows[i0 + (l >> (6 - kLogR))] = tot;
 #pragma unroll
-    for (int c = CL; c < 4; ++c) s.colpre[w][64 * CL + (4 - CL) * l + (c - CL)] = 0;
-    if (16 * RW < 256 && tid >= 16 * RW && tid < 256) s.rowbase[tid] = 0u;
+  for (int c = 0; c < C; ++c) {
+    if (csum[c]) atomicAdd(&s.cols[j0 + c], csum[c]);
+    s.colpre[w][j0 + c] = (uint8_t)cnz[c];
   }
   __syncthreads();
-  // column bases (waves 0-3), row bases (waves 4-7), marginal logs (8-15)
+  // column bases (waves 0-3) and row bases (waves 4-7); the marginals out
   uint32_t mine = 0u, incl = 0u;
   if (tid < 512) {
-    if (tid < 256) {
-      uint32_t run = 0u;
-      for (int q = 0; q < 16; ++q) {
-        const uint32_t v = s.colpre[q][tid];
-        s.colpre[q][tid] = (uint8_t)run;  // at most 15 RW
-        run += v;
+    const int q = tid & 255;
+    if (q < kH) {
+      if (tid < 256) {
+#pragma unroll
+        for (int v = 0; v < kHistWaves; ++v) {
+          const uint32_t n = s.colpre[v][q];
+          s.colpre[v][q] = (uint8_t)mine;  // at most 15 R
+          mine += n;
+        }
+      } else {
+        mine = s.rowbase[q];
       }
-      mine = run;
-    } else {
-      mine = s.rowbase[tid - 256];
     }
     incl = mine;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
-      const uint32_t t = __shfl_up(incl, o, 64);
-      if (l >= o) incl += t;
+      const uint32_t u = __shfl_up(incl, o, 64);
+      if (l >= o) incl += u;
     }
     if (l == 63) s.wtot[w] = incl;
-  } else if (tid < 768) {
-    const int q = tid - 512;
-    const uint32_t c = q < H ? s_cols[q] : 0u;
-    s.mcol[q] = c ? make_float2((float)c, logf_cr((float)c)) : make_float2(0.0f, 0.0f);
   } else {
-    const int q = tid - 768;
-    const uint32_t c = q < H ? s_rows[q] : 0u;
-    s.mrow[q] = c ? make_float2((float)c, logf_cr((float)c)) : make_float2(0.0f, 0.0f);
+    const int q = tid & 255;
+    if (q < H) b.marg[(2 * t + (tid < 768 ? 0 : 1)) * H + q] = tid < 768 ? s.cols[q] : s.rows[q];
   }
   __syncthreads();
+  const uint32_t nz = s.wtot[4] + s.wtot[5] + s.wtot[6] + s.wtot[7];
+  const bool wide = s.big != 0u;
   if (tid < 512) {
     uint32_t off = 0u;
     for (int q = tid < 256 ? 0 : 4; q < w; ++q) off += s.wtot[q];
-    if (tid < 256)
-      s.colbase[tid] = incl - mine + off;
-    else
-      s.rowbase[tid - 256] = incl - mine + off;
+    const int q = tid & 255;
+    if (q < kH) (tid < 256 ? s.colbase : s.rowbase)[q] = incl - mine + off;
   }
-  const uint32_t nz = s.wtot[4] + s.wtot[5] + s.wtot[6] + s.wtot[7];
+  if (tid == 0) b.head[t] = make_uint2(nz, wide ? 1u : 0u);
   __syncthreads();
-
-  // each list's room in win: capw terms, a multiple of kChainBlock (the
-  // mirror list starts 16-byte aligned at win + capw); a list is folded from
-  // at most capw - kChainBlock terms at a time, so its padding and the fold's
-  // read-ahead stay inside its room
-  const int capw = cap / kChainBlock * kChainBlock;
-  const int step = capw - kChainBlock;
-  // both lists straight into win when they fit and the registers hold the
-  // counts; else through the global staging area, window by window
-  const bool direct = KEEP && (int)nz <= step;
-  float *stage = direct ? nullptr : claim_stage();
-  const uint32_t HH = (uint32_t)(H * H);
-  // positions in chain order, row by row of the lane's tile: a row's nonzero
-  // bins are consecutive in the row-major list from the row's base plus the
-  // lanes before; in the column-major list column j continues from its base
-  // plus the bins above in earlier waves, counted up row by row here
-  {
-    uint32_t colrun[CL];
+  unsigned char *la = b.lists + 2 * (size_t)t * b.list_bytes, *lb = la + b.list_bytes;
+  // each list's room in LDS, whole 16-byte pieces
+  const uint32_t room = (2u * nz + 15u) & ~15u;
+  const bool staged = !GH && !wide && 2u * room <= (uint32_t)hist_bytes;
+  uint16_t *wa = reinterpret_cast<uint16_t *>(s_hist), *wb = wa + room / 2;
+  uint32_t col[C];  // the lane's columns' next places
 #pragma unroll
-    for (int c = 0; c < CL; ++c) colrun[c] = s.colbase[CL * l + c] + s.colpre[w][CL * l + c];
+  for (int c = 0; c < C; ++c) col[c] = s.colbase[j0 + c] + s.colpre[w][j0 + c];
 #pragma unroll
-    for (int r = 0; r < RW; ++r) {
-      const uint32_t bits = (uint32_t)(nzm >> (CL * r)) & (uint32_t)T::kRowBits;
-      if (bits) {
-        const int i = RW * w + r;
-        uint32_t pa = s.rowbase[i] + ((rowpre[r >> 2] >> (8 * (r & 3))) & 0xffu);
+  for (int r = 0; r < R; ++r) {
+    if (i0 + r >= H) continue;
+    uint32_t v[C];
+    uint64_t m[C];
+    uint64_t any = 0ull;
 #pragma unroll
-        for (int c = 0; c < CL; ++c) {
-          if (bits & (1u << c)) {
-            const int e = i * H + CL * l + c;
-            const int k = r * CL + c;
-            uint32_t v;
-            if (KEEP && direct) {
-              v = kPack ? (reg[KEEP ? k >> 1 : 0] >> (16 * (k & 1))) & 0xffffu : reg[KEEP ? k : 0];
-              if (need_take) (void)take_at(e);
-            } else {
-              v = take_at(e);
-            }
-            const float p = (float)v;
-            // positions are a permutation of [0, nz); the bounds only keep a
-            // wrong count from writing past the lists
-            if (direct) {
-              if (pa < nz) win[pa] = make_float2(p, 0.0f);
-              if (mirror && colrun[c] < nz) win[capw + colrun[c]] = make_float2(p, 0.0f);
-            } else {
-              if (pa < HH) stage[pa] = p;
-              if (mirror && colrun[c] < HH) stage[HH + colrun[c]] = p;
-            }
-            ++pa;
-            ++colrun[c];
-          }
+    for (int c = 0; c < C; ++c) {
+      v[c] = count(r, c);
+      m[c] = __ballot(v[c] != 0u);
+      any |= m[c];
+    }
+    if (any == 0ull) continue;
+    uint32_t row = s.rowbase[i0 + r];
+#pragma unroll
+    for (int c = 0; c < C; ++c) row += lanes_below(m[c]);
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      if (v[c]) {
+        // places are permutations of [0, nz); the bounds only keep a wrong
+        // count from writing past the lists
+        if (staged) {
+          if (row < nz) wa[row] = (uint16_t)v[c];
+          if (mirror && col[c] < nz) wb[col[c]] = (uint16_t)v[c];
+        } else if (wide) {
+          if (row < nz) reinterpret_cast<uint32_t *>(la)[row] = v[c];
+          if (mirror && col[c] < nz) reinterpret_cast<uint32_t *>(lb)[col[c]] = v[c];
+        } else {
+          if (row < nz) reinterpret_cast<uint16_t *>(la)[row] = (uint16_t)v[c];
+          if (mirror && col[c] < nz) reinterpret_cast<uint16_t *>(lb)[col[c]] = (uint16_t)v[c];
         }
+        if (GH) gh[(i0 + r) * H + j0 + c] = 0u;  // zero at rest (zero bins already are)
+        ++row;
+        ++col[c];
       }
     }
   }
+  if (!staged) return;
   __syncthreads();
+  const uint4 *src = reinterpret_cast<const uint4 *>(s_hist);
+  const int n16 = (int)(room / 16u);
+  for (int k = tid; k < (mirror ? 2 : 1) * n16; k += kHistBlock)
+    reinterpret_cast<uint4 *>(k < n16 ? la : lb)[k < n16 ? k : k - n16] = src[k];
+}
 
-  // one lane per chain: (i, j) on wave 0, (j, i) on wave 1, the column and
-  // row marginals on waves 2 and 3
-  float acc_ij = 0.0f, acc_ji = 0.0f, hx = 0.0f, hy = 0.0f;
-  auto fold = [&](int len, bool first) {
-    if (tid == 0) {
-      acc_ij = fma_chain<CQ>(win, len, acc_ij);
-    } else if (tid == 64) {
-      if (mirror) acc_ji = fma_chain<CQ>(win + capw, len, acc_ji);
-    } else if (tid == 128) {
-      // zero column sums, and the entries from H to 256, are (0, 0) no-ops
-      if (first) hx = fma_chain<CQ>(s.mcol, H, hx);
-    } else if (tid == 192) {
-      if (first) hy = fma_chain<CQ>(s.mrow, H, hy);
+// ---- the chains -------------------------------------------------------------
+constexpr int kFoldPairs = 2;                // pairs of a workgroup
+constexpr int kFoldChains = 4 * kFoldPairs;  // (i, j), (j, i), columns, rows of each
+constexpr int kFoldBlock = 256;              // terms of a chain per step
+constexpr int kFoldWaves = 3;                // the first folds, the others lay terms out
+// terms of a chain's row in LDS, padded so that the chains' 16-byte reads meet
+// different banks
+constexpr int kFoldRow = kFoldBlock + 2;
+
+struct FoldLds {
+  alignas(16) float2 terms[2][kFoldChains][kFoldRow];
+};
+
+// Task t's outputs for fold_chains.
+struct FoldOut {
+  bool mirror;
+  int64_t N;
+  float *ij, *ji;
+};
+
+// The NMI of pair tasks t0 and t0 + 1 (below ntasks), by a workgroup of 3 waves.
+// out(t) gives task t's outputs.
+//
+// Chain c of the 8 is pair c / 4's (i, j), (j, i), column or row chain.  Lane c
+// of the first wave folds it, acc = fmaf(-c, logf(c), acc), in order, 256 terms
+// a step from one of two LDS buffers, while the other waves lay the next 256 of
+// every chain out in the other; their counts are read three steps ahead and
+// their logarithms looked up two steps ahead.  Past a chain's end the terms are
+// (0, 0), and fmaf(-0, 0, acc) is acc exactly.
+//
+// The fold is a chain of dependent multiply-adds (about 1.2 us a step); by one
+// wave alone, the counts, look-ups and stores between its folds took twice as
+// long again (600x248x248 front, up to 9,400 terms: 140 us for 5,050 pairs, 3.3
+// us a step).
+template <class Out>
+__device__ __attribute__((always_inline)) void fold_chains(const ChainBufs &b, int H, int64_t t0,
+                                                           int64_t ntasks, Out out, FoldLds &s) {
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // length of pair p's chain k (0 where there is none)
+  auto length = [&](int p, int k) -> int {
+    if (t0 + p >= ntasks) return 0;
+    if (k >= 2) return H;
+    if (k == 1 && !out(t0 + p).mirror) return 0;
+    return __builtin_amdgcn_readfirstlane((int)b.head[t0 + p].x);
+  };
+  int most = H;
+#pragma unroll
+  for (int p = 0; p < kFoldPairs; ++p) most = max(most, length(p, 0));
+  const int steps = (most + kFoldBlock - 1) / kFoldBlock;
+
+  if (w == 0) {  // ---- the folds
+    float acc = 0.0f;
+    for (int q = 0; q < steps; ++q) {
+      __syncthreads();
+      if (lane < kFoldChains) {
+        // 16 terms at a time, the next 16 on their way: a read's latency is
+        // about that of 16 dependent multiply-adds
+        const float4 *row = reinterpret_cast<const float4 *>(s.terms[q & 1][lane]);
+        constexpr int kQ = 8;
+        float4 r0[kQ], r1[kQ];
+        auto get = [&](float4(&r)[kQ], int k) {
+#pragma unroll
+          for (int u = 0; u < kQ; ++u) r[u] = row[k + u];
+        };
+        auto fold = [&](const float4(&r)[kQ]) {
+#pragma unroll
+          for (int u = 0; u < kQ; ++u) {
+            acc = fmaf(-r[u].x, r[u].y, acc);
+            acc = fmaf(-r[u].z, r[u].w, acc);
+          }
+        };
+        get(r0, 0);
+        for (int k = 0; k < kFoldBlock / 2; k += 2 * kQ) {
+          get(r1, k + kQ);
+          __builtin_amdgcn_sched_barrier(0);
+          fold(r0);
+          if (k + 2 * kQ < kFoldBlock / 2) get(r0, k + 2 * kQ);
+          __builtin_amdgcn_sched_barrier(0);
+          fold(r1);
+        }
+      }
+    }
+    // lanes 4 p .. 4 p + 3 hold pair p's chains
+    const int p = (lane >> 2) & (kFoldPairs - 1);
+    const float hji = __shfl(acc, 4 * p + 1, 64), hx = __shfl(acc, 4 * p + 2, 64),
+                hy = __shfl(acc, 4 * p + 3, 64);
+    if (lane < kFoldChains && (lane & 3) == 0 && t0 + p < ntasks) {
+      const FoldOut o = out(t0 + p);
+      const float fN = (float)o.N;
+      const float lN = logf_cr(fN);
+      const float fx = hx / fN + lN, fy = hy / fN + lN;
+      const float sxy = fx + fy;
+      float fxy = acc / fN + lN;
+      float v = 2.0f * (sxy - fxy) / sxy;
+      *o.ij = v != v ? 0.0f : v;
+      if (o.mirror) {
+        fxy = hji / fN + lN;
+        v = 2.0f * (sxy - fxy) / sxy;
+        *o.ji = v != v ? 0.0f : v;
+      }
+    }
+    return;
+  }
+
+  // ---- the terms: wave w has list chains w - 1, w + 1, ... of the 4 (pair lc /
+  // 2's row-major or column-major list) and, in the first step, the marginals'
+  // chains of the same numbers
+  constexpr int kLists = 2 * kFoldPairs, kOwn = (kLists + kFoldWaves - 2) / (kFoldWaves - 1);
+  int len[kOwn];
+  bool wide[kOwn];
+  const unsigned char *src[kOwn];
+#pragma unroll
+  for (int u = 0; u < kOwn; ++u) {
+    const int lc = w - 1 + u * (kFoldWaves - 1);
+    len[u] = lc < kLists ? length(lc >> 1, lc & 1) : 0;
+    const int64_t t = t0 + (len[u] ? lc >> 1 : 0);
+    wide[u] = __builtin_amdgcn_readfirstlane((int)b.head[t].y) != 0;
+    src[u] = b.lists + (2 * (size_t)t + (lc & 1)) * b.list_bytes;
+  }
+  struct Counts {
+    uint32_t v[kOwn][4];
+  };
+  // this lane's counts of step q: entries k .. k + 3 of each chain, k = 256 q +
+  // 4 lane, 0 past the chain's end (a list's room is whole 16-byte pieces, so
+  // the four of its last entry can be read)
+  auto load = [&](Counts &n, int q) {
+#pragma unroll
+    for (int u = 0; u < kOwn; ++u) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) n.v[u][c] = 0u;
+      if (q * kFoldBlock < len[u]) {
+        const int k = q * kFoldBlock + 4 * lane, i = k < len[u] ? k : 0;
+        uint32_t x[4];
+        if (wide[u]) {
+          const uint4 y = reinterpret_cast<const uint4 *>(src[u])[i >> 2];
+          x[0] = y.x; x[1] = y.y; x[2] = y.z; x[3] = y.w;
+        } else {
+          const uint2 y = reinterpret_cast<const uint2 *>(src[u])[i >> 2];
+          x[0] = y.x & 0xffffu; x[1] = y.x >> 16; x[2] = y.y & 0xffffu; x[3] = y.y >> 16;
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) n.v[u][c] = k + c < len[u] ? x[c] : 0u;
+      }
     }
   };
-  if (direct) {
-    // the logarithms in place; (0, 0) from nz to the next kChainBlock
-    const int nzp = ((int)nz + kChainBlock - 1) / kChainBlock * kChainBlock;
-    for (int q = tid; q < nzp; q += kNmiBlock) {
-      if (q < (int)nz) {
-        win[q].y = logf_cr(win[q].x);
-        if (mirror) win[capw + q].y = logf_cr(win[capw + q].x);
-      } else {
-        win[q] = make_float2(0.0f, 0.0f);
-        if (mirror) win[capw + q] = make_float2(0.0f, 0.0f);
+  struct Logs {
+    float t[kOwn][4];
+  };
+  auto look_up = [&](const Counts &n, Logs &g, int q) {
+#pragma unroll
+    for (int u = 0; u < kOwn; ++u)
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        g.t[u][c] = q * kFoldBlock < len[u] ? b.logs[min(n.v[u][c], (uint32_t)kLogs - 1u)] : 0.0f;
+  };
+  // rows past their chain's end are zeroed in both buffers and left
+  auto put = [&](const Counts &n, Logs &g, int q) {
+#pragma unroll
+    for (int u = 0; u < kOwn; ++u) {
+      const int lc = w - 1 + u * (kFoldWaves - 1);
+      if (lc >= kLists || (q - 2) * kFoldBlock >= len[u]) continue;
+      if (wide[u]) {  // counts past the table
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          if (n.v[u][c] >= (uint32_t)kLogs) g.t[u][c] = logf_cr((float)n.v[u][c]);
+      }
+      float4 *row = reinterpret_cast<float4 *>(&s.terms[q & 1][4 * (lc >> 1) + (lc & 1)][4 * lane]);
+      row[0] = make_float4((float)n.v[u][0], g.t[u][0], (float)n.v[u][1], g.t[u][1]);
+      row[1] = make_float4((float)n.v[u][2], g.t[u][2], (float)n.v[u][3], g.t[u][3]);
+    }
+  };
+  auto log_of = [&](uint32_t v) -> float {
+    float t = b.logs[min(v, (uint32_t)kLogs - 1u)];
+    if (v >= (uint32_t)kLogs) t = logf_cr((float)v);
+    return t;
+  };
+  // the marginals: one step (H <= 256), then zeros in both buffers
+  auto put_marginals = [&](int q) {
+#pragma unroll
+    for (int u = 0; u < kOwn; ++u) {
+      const int lc = w - 1 + u * (kFoldWaves - 1);
+      if (lc >= kLists) continue;
+      const int n = q == 0 ? length(lc >> 1, 2 + (lc & 1)) : 0;
+      const uint32_t *m = b.marg + (2 * (t0 + (n ? lc >> 1 : 0)) + (lc & 1)) * H;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int k = 64 * c + lane;
+        const uint32_t v = k < n ? m[k] : 0u;
+        s.terms[q & 1][4 * (lc >> 1) + 2 + (lc & 1)][k] = make_float2((float)v, k < n ? log_of(v) : 0.0f);
       }
     }
+  };
+  Counts n0, n1, n2, n3;
+  Logs g0, g1, g2;
+  load(n0, 0);
+  load(n1, 1);
+  load(n2, 2);
+  look_up(n0, g0, 0);
+  look_up(n1, g1, 1);
+  put(n0, g0, 0);
+  put_marginals(0);
+  for (int q = 0; q < steps; ++q) {
     __syncthreads();
-    fold((int)nz, true);
+    if (q + 1 < steps) {
+      // n1, g1: step q + 1; n2: q + 2
+      load(n3, q + 3);
+      look_up(n2, g2, q + 2);
+      put(n1, g1, q + 1);
+      if (q < 2) put_marginals(q + 1);
+      n1 = n2;
+      g1 = g2;
+      n2 = n3;
+    }
+  }
+}
+
+__device__ __forceinline__ double wave_sum(double v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  return v;
+}
+
+// NMI of a pair in double from the exact counts (arguments as for emit_chains;
+// the histogram's LDS is left as it is); the value is lane 0's, NaN included.
+template <bool PACK16>
+__device__ __attribute__((always_inline)) double nmi64_pair(const uint32_t *s_hist, uint32_t *gh,
+                                                            int H, int64_t N, PairLds<PACK16> &s,
+                                                            double (&s_red)[3][kHistWaves]) {
+  using L = PairLds<PACK16>;
+  const int tid = threadIdx.x;
+  double sxy = 0.0, sx = 0.0, sy = 0.0;
+  auto fold = [&](int i, int j, uint32_t c) {
+    const double dc = (double)c;
+    sxy += dc * log(dc);
+    atomicAdd(&s.rows[i], c);
+    atomicAdd(&s.cols[j], c);
+    if (gh) gh[i * H + j] = 0u;  // zero at rest
+  };
+  if (s.nbins <= (uint32_t)L::kBins) {
+    for (uint32_t k = tid; k < s.nbins; k += kHistBlock) {
+      const int i = s.bins[k] >> 8, j = s.bins[k] & 255;
+      fold(i, j, pair_count<PACK16>(s_hist, gh, H, i, j));
+    }
   } else {
-    // window by window through LDS, each entry's logarithm taken by the lane
-    // that brings it in
-    for (uint32_t w0 = 0;; w0 += (uint32_t)step) {
-      const uint32_t w1 = w0 + (uint32_t)step < nz ? w0 + (uint32_t)step : nz;
-      const int len = w0 < nz ? (int)(w1 - w0) : 0;
-      const int lenp = (len + kChainBlock - 1) / kChainBlock * kChainBlock;
-      for (int q = tid; q < lenp; q += kNmiBlock) {
-        float2 t = make_float2(0.0f, 0.0f), u = t;
-        if (q < len) {
-          const float c = stage[w0 + q];
-          t = make_float2(c, logf_cr(c));
-          if (mirror) {
-            const float d = stage[HH + w0 + q];
-            u = make_float2(d, logf_cr(d));
-          }
-        }
-        win[q] = t;
-        if (mirror) win[capw + q] = u;
-      }
-      __syncthreads();
-      fold(len, w0 == 0);
-      __syncthreads();
-      if (w1 >= nz) break;
-    }
-    release_stage();
+    each_bin<PACK16>(s_hist, gh, H, fold);
   }
-  if (tid == 64) s.acc[1] = acc_ji;
-  if (tid == 128) s.acc[2] = hx;
-  if (tid == 192) s.acc[3] = hy;
   __syncthreads();
+  if (tid < H) {
+    const uint32_t r = s.rows[tid], c = s.cols[tid];
+    if (r) sx = (double)r * log((double)r);
+    if (c) sy = (double)c * log((double)c);
+  }
+  sxy = wave_sum(sxy);
+  sx = wave_sum(sx);
+  sy = wave_sum(sy);
+  const int w = tid >> 6;
+  if ((tid & 63) == 0) { s_red[0][w] = sxy; s_red[1][w] = sx; s_red[2][w] = sy; }
+  __syncthreads();
+  double v = 0.0;
   if (tid == 0) {
-    const float fN = (float)N;
-    const float lN = logf_cr(fN);
-    const float fx = s.acc[2] / fN + lN, fy = s.acc[3] / fN + lN;
-    const float sxy = fx + fy;
-    float fxy = acc_ij / fN + lN;
-    float v = 2.0f * (sxy - fxy) / sxy;
-    *out_ij = v != v ? 0.0f : v;
-    if (mirror) {
-      fxy = s.acc[1] / fN + lN;
-      v = 2.0f * (sxy - fxy) / sxy;
-      *out_ji = v != v ? 0.0f : v;
-    }
+    double txy = 0, tx = 0, ty = 0;
+    for (int k = 0; k < kHistWaves; ++k) { txy += s_red[0][k]; tx += s_red[1][k]; ty += s_red[2][k]; }
+    const double dN = (double)N, lnN = log(dN);
+    const double hx = lnN - tx / dN, hy = lnN - ty / dN, hxy = lnN - txy / dN;
+    v = 2.0 * (hx + hy - hxy) / (hx + hy);
   }
+  return v;
 }
 
-// Staging slots of a launch whose workgroups are not persistent: a bitmap of
-// free slots (zero at rest), `words` 32-bit words per XCD.  A workgroup only
-// claims slots of the XCD it runs on (the hardware XCC id): each XCD has its
-// own write-back L2, not coherent with the others within a kernel, so a slot
-// written on one XCD and then reused on another could have the first XCD's
-// dirty lines written back over the second's data.  Within one XCD the next
-// holder's stores land in the same L2 lines.  Each XCD has at least as many
-// slots as workgroups of the kernel that fit on its CUs at once, so a claim
-// finds a free bit on its first sweep; a workgroup that holds a slot never
-// waits, so a claim that found none still ends once one is released.
-__device__ __forceinline__ uint32_t nmi32_claim(uint32_t *bits, int words, int nxcd) {
-  // s_getreg of HW_REG_XCC_ID (register 20), bits [3:0]
-  const uint32_t xcd = (uint32_t)__builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) %
-                       (uint32_t)nxcd;
-  for (;;) {
-    for (int k = 0; k < words; ++k) {
-      const int w = (int)xcd * words + k;
-      uint32_t v = __hip_atomic_load(&bits[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      while (~v) {
-        const uint32_t bit = 1u << (__ffs(~v) - 1);
-        const uint32_t old = atomicOr(&bits[w], bit);
-        if (!(old & bit)) return (uint32_t)w * 32u + (uint32_t)(__ffs(bit) - 1);
-        v = old | bit;
-      }
-    }
-    __builtin_amdgcn_s_sleep(8);
-  }
-}
+// logf of the counts 0 to kLogs - 1: the context's table, filled on
+// first use, or into the caller's memory.
+int nmi_logs(iso_ctx *ctx, const float **out);
+int nmi_logs_fill(iso_ctx *ctx, float *d_logs);
 
-// Called by one lane after the workgroup's last read of the slot has returned
-// (the window copies end in LDS stores of the loaded values).  The next
-// holder writes before it reads, and its writes depend on the claimed index,
-// so relaxed atomics order the hand-over.
-__device__ __forceinline__ void nmi32_release(uint32_t *bits, uint32_t slot) {
-  atomicAnd(&bits[slot >> 5], ~(1u << (slot & 31u)));
-}
+// Device buffers one launch of the histogram + NMI kernels works in: merged
+// 32-bit histograms and slice arrival counters per task (zero at rest) and,
+// for the reference-order NMI, the chains' inputs.
+struct HistBufs {
+  uint32_t *ghist = nullptr;
+  uint32_t *arrive = nullptr;
+  ChainBufs chains;
+};
+
+// One launch over tasks d_tasks[0, nt) with the caller's buffers; variant
+// 0 or 1 is the kernel shape (the autotuner's two candidates).
+int hist_launch(iso_ctx *ctx, const float *d_fields, int n, int64_t F, int H, int multi,
+                uint32_t flags, const float *d_mins, const float *d_maxs, float *d_map,
+                const int2 *d_tasks, int nt, uint32_t *d_joint, uint32_t *d_rows,
+                uint32_t *d_cols, const HistBufs &b, int variant);
 
 }  // namespace iso

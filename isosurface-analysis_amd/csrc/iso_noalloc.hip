@@ -1,12 +1,12 @@
 // iso_hist_nmi_noalloc: the joint-histogram + NMI entry point for callers
 // that cannot allocate device memory (code under HIP graph capture, tight
 // serving loops, harnesses that forbid hipMalloc).  It computes exactly what
-// iso_hist_nmi computes, with the same kernel; its working memory -- the
+// iso_hist_nmi computes, with the same kernels; its working memory -- the
 // pair task list, the merged 32-bit histograms and slice arrival counters,
-// and the staging slots of the reference-order NMI -- lives in one
+// and the reference-order NMI's logarithms and chain inputs -- lives in one
 // file-scope device array, `scratch`, of 64 MiB per device, held until the
 // process ends.  Pairs go through in launches of as many tasks as the array
-// holds at once (127 at 256 bins), so any number of fields fits.
+// holds at once (84 at 256 bins), so any number of fields fits.
 //
 // Host code never uses the array's name as an address: at set-up (the
 // context's creation, else this entry point's first call on a device) the
@@ -22,7 +22,6 @@
 namespace {
 
 constexpr size_t kScratchBytes = (size_t)64 << 20;
-constexpr int kSlotsPerXcd = 4;      // reference-order NMI staging slots per XCD
 constexpr int kMaxFields = 65535;    // n(n+1)/2 pair tasks stay below 2^31
 constexpr int kMaxDevices = 64;
 
@@ -108,35 +107,34 @@ int iso_hist_nmi_noalloc(iso_ctx *ctx, const float *d_fields, int n, int64_t F, 
   ISO_TRY(scratch_of(ctx, &base));
   char *p = (char *)base;
   const bool nmi32 = (flags & ISO_COMPAT_NMI32) != 0;
-  const int nxcd = std::max(ctx->xcd_count, 1);
-  // layout: slot bitmap (one word per XCD) | staging slots | tasks | arrive | histograms
+  // layout: logarithms | tasks | arrive | chains' inputs | histograms
   iso::HistBufs b;
   size_t off = 0;
+  size_t per_task = sizeof(int2) + 4 + 4 * (size_t)H * H;
   if (nmi32) {
-    // one bitmap word per XCD with kSlotsPerXcd slots behind it (the other
-    // bits are set below and never claimed)
-    b.slot_words = 1;
-    b.slots_per_word = kSlotsPerXcd;
-    b.slot_bits = (uint32_t *)(p + off);
-    off += align256(4 * (size_t)nxcd);
-    b.stage = (float *)(p + off);
-    off += align256((size_t)nxcd * kSlotsPerXcd * iso::nmi32_stage_bytes(H));
+    ISO_TRY(iso::nmi_logs_fill(ctx, (float *)p));
+    b.chains.logs = (const float *)p;
+    off += align256(sizeof(float) * iso::kLogs);
+    per_task += iso::chain_task_bytes(H, F);
   }
-  const size_t per_task = sizeof(int2) + 4 + 4 * (size_t)H * H;
-  if (off + 3 * 256 + per_task > kScratchBytes)
+  constexpr size_t kPad = 5 * 256;  // what rounding the parts up takes
+  if (off + kPad + per_task > kScratchBytes)
     return iso::fail(ctx, ISO_ERR_UNSUPPORTED, "iso_hist_nmi_noalloc: %d bins exceed the %zu-byte scratch",
                      H, kScratchBytes);
-  const int T = (int)std::min<size_t>((kScratchBytes - off - 3 * 256) / per_task, 16384);
+  const int T = (int)std::min<size_t>((kScratchBytes - off - kPad) / per_task, 16384);
   int2 *tasks = (int2 *)(p + off);
   off += align256(sizeof(int2) * (size_t)T);
   b.arrive = (uint32_t *)(p + off);
   off += align256(4 * (size_t)T);
+  if (nmi32) {
+    iso::chain_carve(b.chains, p + off, T, H, F);
+    off += align256(iso::chain_task_bytes(H, F) * (size_t)T + 512);
+  }
   b.ghist = (uint32_t *)(p + off);
   // what the kernels expect zero at rest (a previous call may have ended
-  // early); slots beyond kSlotsPerXcd in each XCD's word stay taken
+  // early)
   ISO_TRY(iso::fill_u32(ctx, b.arrive, 0u, (size_t)T));
   ISO_TRY(iso::fill_u32(ctx, b.ghist, 0u, (size_t)T * H * H));
-  if (nmi32) ISO_TRY(iso::fill_u32(ctx, b.slot_bits, ~((1u << kSlotsPerXcd) - 1u), (size_t)nxcd));
   const int64_t ntasks = multi ? (int64_t)n * n : (int64_t)n * (n + 1) / 2;
   for (int64_t t0 = 0; t0 < ntasks; t0 += T) {
     const int nt = (int)std::min<int64_t>(T, ntasks - t0);
