@@ -85,6 +85,18 @@ __device__ __forceinline__ void sample_coords(const iso::SampleGrid &g, int x, i
 
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
+// min with the lane 32 (or 16) away, and with the lane R before in its row of 16
+template <int O>
+__device__ __forceinline__ uint32_t min_swapped(uint32_t v) {
+  const auto p = O == 32 ? __builtin_amdgcn_permlane32_swap(v, v, false, false)
+                         : __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  return min((uint32_t)p[0], (uint32_t)p[1]);
+}
+template <int R>
+__device__ __forceinline__ uint32_t min_rotated(uint32_t v) {
+  return min(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x120 + R, 0xf, 0xf, true));
+}
+
 // number of set bits of m in lanes below this one
 __device__ __forceinline__ int lane_rank(uint64_t m) {
   return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
@@ -935,13 +947,13 @@ __global__ __launch_bounds__(kTrBlock) __attribute__((amdgpu_waves_per_eu(SPL >=
   static_assert(BUCKET <= 64, "one point per lane");
   __shared__ int s_stack[kTrWaves][64];  // one deferred node per level at most
   // the points being scanned by each wave; slots from BUCKET on stay at +inf
-  // (a packed scan reads up to 63 slots past the leaf)
-  __shared__ float4 s_pts[kTrWaves][BUCKET + 64];
+  // (a packed scan for one sample reads two rows of 64)
+  __shared__ float4 s_pts[kTrWaves][128];
   // packed samples of a compacted scan: at most one per lane
   constexpr int kPack = kCompact * SPL < 64 ? kCompact * SPL : 64;
   __shared__ float4 s_cand[kTrWaves][kPack];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  s_pts[w][BUCKET + lane] = make_float4(INFINITY, 0.f, 0.f, 0.f);
+  for (int i = BUCKET + lane; i < 128; i += 64) s_pts[w][i] = make_float4(INFINITY, 0.f, 0.f, 0.f);
   const uint32_t nbricks = (uint32_t)bx * by * bz;
   const uint32_t total = nbricks * (uint32_t)S;
   // Tickets: the first nbig are chunks of `chunk` bricks, the next nhalf
@@ -1008,64 +1020,88 @@ __global__ __launch_bounds__(kTrBlock) __attribute__((amdgpu_waves_per_eu(SPL >=
       }
     }
 
+    // which samples of each lane find bound d below their best: one mask per
+    // sample slot, kept as it is (a mask rebuilt from a bool that crosses a
+    // branch costs two more vector instructions)
+    auto wanted = [&](const float (&d)[SPL], uint64_t (&m)[SPL]) {
+      uint64_t any = 0;
+#pragma unroll
+      for (int q = 0; q < SPL; ++q) any |= m[q] = __ballot(d[q] < best[q]);
+      return any != 0;
+    };
     // points [first, first + cnt), cnt <= BUCKET: one coalesced load, through
     // this wave's LDS slots, read back at a uniform address (a broadcast), four
-    // per step.  Slots past cnt hold a point at +inf, whose d2 is +inf, so the
-    // last step needs no mask.  d2 is never NaN, so fminf keeps the smaller.
-    // d: each sample's bound for the leaf's box.
-    auto scan = [&](int first, int cnt, const float (&d)[SPL]) {
-      const Pt pv = pts[first + (lane < cnt ? lane : 0)];
-      if (lane < BUCKET)
-        s_pts[w][lane] = lane < cnt ? make_float4(pv.x, pv.y, pv.z, 0.f)
-                                    : make_float4(INFINITY, 0.f, 0.f, 0.f);
-      uint64_t mq[SPL];
+    // per step.  Slots past cnt hold a point at x = +inf, whose d2 is +inf or
+    // NaN, so the last step needs no mask (the lanes past cnt load the points
+    // that follow; the array ends in 64 spare ones).  The d2 of the leaf's own
+    // points is never NaN, so fminf keeps the smaller.
+    // mq: the samples whose bound for the leaf's box is below their best.
+    auto scan = [&](int first, int cnt, const uint64_t (&mq)[SPL]) {
+      const Pt pv = (pts + first)[lane];
       int pc = 0;
 #pragma unroll
-      for (int q = 0; q < SPL; ++q) {
-        mq[q] = __ballot(d[q] < best[q]);
-        pc += (int)__popcll(mq[q]);
-      }
+      for (int q = 0; q < SPL; ++q) pc += (int)__popcll(mq[q]);
       if (pc <= kPack) {
         if (pc == 0) return;
-        int rank0 = 0;
+        int rank[SPL], rank0 = 0;
 #pragma unroll
         for (int q = 0; q < SPL; ++q) {
-          if ((mq[q] >> lane) & 1u)
-            s_cand[w][rank0 + lane_rank(mq[q])] = make_float4(sx, sy, sz[q], 0.f);
+          rank[q] = rank0 + lane_rank(mq[q]);
+          if (__builtin_amdgcn_inverse_ballot_w64(mq[q]))
+            s_cand[w][rank[q]] = make_float4(sx, sy, sz[q], 0.f);
           rank0 += (int)__popcll(mq[q]);
         }
+        if (lane < BUCKET)
+          s_pts[w][lane] = make_float4(lane < cnt ? pv.x : INFINITY, pv.y, pv.z, 0.f);
         const int lg = pc <= 1 ? 0 : 32 - __builtin_clz((unsigned)(pc - 1));  // P = 1 << lg
         const int j = lane & ((1 << lg) - 1), step = 64 >> lg;
-        // The partial minima are kept as bit patterns: a d2 is never NaN or
-        // -0 (a sum of squares, +inf at the padding), so its bits order as
-        // its values and an integer min needs no NaN canonicalisation; the
-        // exchanges are plain ds_bpermute (lanes wrap mod 64, no bound test).
+        // The partial minima are kept as bit patterns: a d2 is a sum of
+        // squares, so its bits order as its values (NaN, at the padding, above
+        // +inf) and an integer min needs no NaN canonicalisation.  Two rows a
+        // step; a row past cnt is padding.
         uint32_t part = 0x7f800000u;  // +inf
         if (j < pc) {
           const float4 c = s_cand[w][j];
           const float4 *row = &s_pts[w][lane >> lg];
-          for (int i0 = 0; i0 < cnt; i0 += step) {  // a uniform trip count; +inf past cnt
-            const float4 p = row[i0];
-            part = min(part, __float_as_uint(d2_point(c.x, c.y, c.z, p.x, p.y, p.z)));
+          for (int i0 = 0; i0 < cnt; i0 += 2 * step) {  // a uniform trip count
+            const float4 p0 = row[i0], p1 = row[i0 + step];
+            part = min(part, min(__float_as_uint(d2_point(c.x, c.y, c.z, p0.x, p0.y, p0.z)),
+                                 __float_as_uint(d2_point(c.x, c.y, c.z, p1.x, p1.y, p1.z))));
           }
         }
-        const int lane4 = lane << 2;
-        for (int o = 1 << lg; o < 64; o <<= 1)
-          part = min(part, (uint32_t)__builtin_amdgcn_ds_bpermute(lane4 ^ (o << 2), (int)part));
-        rank0 = 0;
+        // min over the lanes of each sample, which are P apart: the lane
+        // swaps across 32 and 16, then rotations within rows of 16
+        if (lg < 6) {
+          part = min_swapped<32>(part);
+          if (lg < 5) {
+            part = min_swapped<16>(part);
+            if (lg < 4) {
+              part = min_rotated<8>(part);
+              if (lg < 3) {
+                part = min_rotated<4>(part);
+                if (lg < 2) {
+                  part = min_rotated<2>(part);
+                  if (lg < 1) part = min_rotated<1>(part);
+                }
+              }
+            }
+          }
+        }
 #pragma unroll
         for (int q = 0; q < SPL; ++q) {
-          const float v = __uint_as_float(
-              (uint32_t)__builtin_amdgcn_ds_bpermute((rank0 + lane_rank(mq[q])) << 2, (int)part));
-          if ((mq[q] >> lane) & 1u) best[q] = fminf(best[q], v);
-          rank0 += (int)__popcll(mq[q]);
+          const uint32_t v = (uint32_t)__builtin_amdgcn_ds_bpermute(rank[q] << 2, (int)part);
+          // a wanting sample's best is >= 0: its bits order as its value
+          if (__builtin_amdgcn_inverse_ballot_w64(mq[q]))
+            best[q] = __uint_as_float(min(__float_as_uint(best[q]), v));
         }
         return;
       }
+      if (lane < BUCKET)
+        s_pts[w][lane] = make_float4(lane < cnt ? pv.x : INFINITY, pv.y, pv.z, 0.f);
       for (int i0 = 0; i0 < cnt; i0 += 4) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const float4 p = s_pts[w][(i0 + i) & (BUCKET - 1)];
+          const float4 p = s_pts[w][i0 + i];
           // d2_point with the x and y part shared by the lane's samples
           const float dx = sx - p.x, dy = sy - p.y;
           const float pxy = __builtin_fmaf(dy, dy, dx * dx);
@@ -1077,26 +1113,21 @@ __global__ __launch_bounds__(kTrBlock) __attribute__((amdgpu_waves_per_eu(SPL >=
         }
       }
     };
-    // does any sample of any lane find bound d below its best?
-    // (one ballot per comparison: a ballot of an OR-ed bool costs two more
-    // vector instructions to rebuild the mask)
-    auto wanted = [&](const float (&d)[SPL]) {
-      uint64_t m = 0;
-#pragma unroll
-      for (int q = 0; q < SPL; ++q) m |= __ballot(d[q] < best[q]);
-      return m != 0;
-    };
     int all = 0;  // valid samples of the brick
+    uint64_t vm[SPL];
 #pragma unroll
-    for (int q = 0; q < SPL; ++q) all += __popcll(__ballot(valid[q]));
+    for (int q = 0; q < SPL; ++q) {
+      vm[q] = __ballot(valid[q]);
+      all += __popcll(vm[q]);
+    }
 
     int node = uniform(root_of[ne_set[seg]]);
     if (node < 0) {
       if (node != kNoRoot) {  // the set is one leaf
-        float z[SPL];
+        uint64_t m[SPL];
 #pragma unroll
-        for (int q = 0; q < SPL; ++q) z[q] = 0.0f;
-        scan((int)base, n, z);
+        for (int q = 0; q < SPL; ++q) m[q] = __ballot(0.0f < best[q]);
+        scan((int)base, n, m);
       }
     } else {
       int sp = 0;
@@ -1111,16 +1142,19 @@ __global__ __launch_bounds__(kTrBlock) __attribute__((amdgpu_waves_per_eu(SPL >=
           dl[q] = d2_box_z(sz[q], r.lmin, r.lmax, lxy);
           dr[q] = d2_box_z(sz[q], r.rmin, r.rmax, rxy);
         }
-        bool nl = wanted(dl), nr = wanted(dr);
+        uint64_t ml[SPL], mr[SPL];
+        bool nl = wanted(dl, ml), nr = wanted(dr, mr);
         if (left < 0 || right < 0) {
-          bool scanned = false;
-          if (left < 0 && nl) { scan(first, -left - 1 - first, dl); scanned = true; }
-          if (right < 0 && nr) { scan(-right - 1, last + 2 + right, dr); scanned = true; }
-          if (left < 0) nl = false;
-          if (right < 0) nr = false;
-          if (scanned) {  // the leaf's points may already rule the sibling out
-            if (nl) nl = wanted(dl);
-            if (nr) nr = wanted(dr);
+          // a leaf's points may already rule its sibling out
+          if (left < 0 && nl) {
+            scan(first, -left - 1 - first, ml);
+            if (nr) nr = wanted(dr, mr);
+            nl = false;
+          }
+          if (right < 0 && nr) {
+            scan(-right - 1, last + 2 + right, mr);
+            if (nl) nl = wanted(dl, ml);
+            nr = false;
           }
         }
         int next;
@@ -1128,7 +1162,7 @@ __global__ __launch_bounds__(kTrBlock) __attribute__((amdgpu_waves_per_eu(SPL >=
           // nearer child first: the one most samples find closer
           int closer = 0;
 #pragma unroll
-          for (int q = 0; q < SPL; ++q) closer += __popcll(__ballot(valid[q] && dl[q] <= dr[q]));
+          for (int q = 0; q < SPL; ++q) closer += __popcll(__ballot(dl[q] <= dr[q]) & vm[q]);
           const bool left_first = closer * 2 >= all;
           s_stack[w][sp++] = left_first ? right : left;
           next = left_first ? left : right;
@@ -1279,7 +1313,8 @@ int df_pool(iso_ctx *ctx, const void *d_xyz, bool is_int, int64_t ntot, const ui
   uint32_t *keys = (uint32_t *)ca, *vals = (uint32_t *)ia;
   uint32_t *sk = nullptr;
   void *sorted = nullptr, *scodes = nullptr;
-  ISO_TRY(ws_get(ctx, WS_DF_LEAVES, sizeof(Pt) * (size_t)ntot, false, &sorted));
+  // 64 spare points: a leaf is loaded by a whole wave
+  ISO_TRY(ws_get(ctx, WS_DF_LEAVES, sizeof(Pt) * ((size_t)ntot + 64), false, &sorted));
   // sorted-point path: keys, sort, normalised points in key order
   auto prep_sorted = [&]() -> int {
     keys = (uint32_t *)ca;
