@@ -23,13 +23,14 @@
 //   - the workgroup loops over only the isovalues inside the [min,max] of its
 //     samples (block culling), so one read of the volume serves all k
 //     isovalues of an ISM;
-//   - output slots come from one atomic per wave per isovalue (wave prefix
-//     sum in registers); the vertex set is exact, its order unspecified.
+//   - a count pass and a scan give every (block, isovalue, wave) its place in
+//     the output; the vertex set is exact, its order unspecified.
 #include "iso_internal.hpp"
 
 #include <algorithm>
 #include <cstring>
 #include <numeric>
+#include <type_traits>
 #include <vector>
 
 namespace iso {
@@ -135,7 +136,6 @@ struct McArgs {
 };
 
 constexpr int kMcPriv = 64;   // copies of the per-slot counters (blocks spread over them)
-constexpr int kMcAcc = 256;   // per-block LDS accumulators for the first isovalues of its range
 
 __device__ __forceinline__ uint64_t hash64(uint64_t z) {
   z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
@@ -193,260 +193,354 @@ __device__ __forceinline__ bool cell_ok(const McArgs &a, int cx, int cy, int cz)
   return lin < a.ncls;
 }
 
+// f over the lanes of the wave: rotations within rows of 16, then the lanes 16
+// and 32 away
+template <class F>
+__device__ __forceinline__ float wave_fold(float v, F f) {
+  auto rot = [](float x, auto r) {
+    const int i = __float_as_int(x);
+    return __int_as_float(__builtin_amdgcn_update_dpp(i, i, 0x120 + decltype(r)::value, 0xf, 0xf, true));
+  };
+  v = f(v, rot(v, std::integral_constant<int, 1>()));
+  v = f(v, rot(v, std::integral_constant<int, 2>()));
+  v = f(v, rot(v, std::integral_constant<int, 4>()));
+  v = f(v, rot(v, std::integral_constant<int, 8>()));
+  const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = f(__uint_as_float(p[0]), __uint_as_float(p[1]));
+  const auto q = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return f(__uint_as_float(q[0]), __uint_as_float(q[1]));
+}
+
+__device__ __forceinline__ void wave_minmax(float &lo, float &hi) {
+  lo = wave_fold(lo, [](float a, float b) { return fminf(a, b); });
+  hi = wave_fold(hi, [](float a, float b) { return fmaxf(a, b); });
+}
+
+// isovalues that values in [lo, hi] can cross, lo < iso <= hi: [first, second)
+__device__ __forceinline__ int2 iso_range(const float *isos, int k, float lo, float hi) {
+  int b0 = 0, b1 = 0;
+  for (int i = threadIdx.x & 63; __ballot(i < k); i += 64) {
+    const float v = i < k ? isos[i] : 0.0f;
+    b0 += __popcll(__ballot(i < k && !(v > lo)));
+    b1 += __popcll(__ballot(i < k && !(v > hi)));
+  }
+  return make_int2(b0, lo <= hi ? b1 : b0);
+}
+
+// exclusive prefix sum over the first 32 lanes, and their sum
+__device__ __forceinline__ uint32_t prefix32(uint32_t v, uint32_t &sum) {
+  const int lane = threadIdx.x & 63;
+  uint32_t inc = v;
+#pragma unroll
+  for (int o = 1; o < 32; o <<= 1) {
+    const uint32_t u = __shfl_up(inc, o, 64);
+    if (lane >= o) inc += u;
+  }
+  sum = (uint32_t)__builtin_amdgcn_readlane((int)inc, 31);
+  return inc - v;
+}
+
+constexpr int kMcF = 17, kMcM = 5;  // samples of a block: 16 x 4 x 4 and one more per axis
+constexpr int kMcQueue = 256;       // crossings of a wave waiting to be worked out
+
 // EMIT = false: count pass (claims grid-point vertices, per-block totals,
 // per-slot counts and, when STATS, cell statistics).  EMIT = true: the same
 // decisions again, grid-point vertices taken by their recorded owner,
 // vertices written from the block's scanned base.  No pool counter is shared
 // between blocks.
+//
+// A wave goes over its isovalues with one compare per sample: a crossing of a
+// lane's edge is a bit where two masks differ, and the crossings go into the
+// wave's queue, isovalue by isovalue.  64 at a time they are worked out with
+// every lane busy (divisions, orientations, grid points).  Most lanes of a wave
+// cross no given isovalue, so working the edges out isovalue by isovalue ran
+// the divisions of all five candidates for a few lanes each.
+// Bound by the vector instructions (3.7 cycles each): the queueing about half
+// of them, the working out a third, the rest the block's start.  418M vertices
+// of 64 isovalues over 512^3 sines: count 6.6 -> 4.0 ms, emit 9.1 -> 4.1 (6.7 GB
+// written, 1.6 TB/s); 174M of 100 over the 600x248x248 front: 1.17 -> 0.98 and
+// 1.63 -> 1.21; one isovalue of the front 340 -> 238 and 298 -> 66 us (blocks
+// without a vertex leave at once).  Several blocks per workgroup with the next
+// one's samples under way (2, 4, 8): front 2.38, sines 8.7 ms, no gain.
+// A vertex's place is its number in the wave's order plus, per isovalue, what
+// turns that order (wave, isovalue) into the block's (isovalue, wave), so that
+// an isovalue's vertices of a block are one run of the pool.
 template <bool EMIT, bool STATS>
 __global__ __launch_bounds__(kMcBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) void mc_kernel(McArgs a) {
+  __shared__ float s_v[kMcF * kMcM * kMcM];
+  __shared__ uint32_t s_queue[kMcWaves][kMcQueue];
   __shared__ uint8_t s_nv[256];
-  __shared__ float s_lo[kMcBlock / 64], s_hi[kMcBlock / 64];
-  __shared__ int s_range[2];
-  // per (isovalue of the round, wave): vertices, active cells, case vertices, offsets
-  __shared__ uint32_t s_wt[kMcRound][kMcWaves], s_wa[kMcRound][kMcWaves];
-  __shared__ uint32_t s_wv[kMcRound][kMcWaves], s_off[kMcRound][kMcWaves];
-  // per isovalue of the block's range (first kMcAcc): vertices, active cells, case vertices
-  __shared__ uint32_t s_accv[kMcAcc], s_acca[kMcAcc], s_acct[kMcAcc];
-  __shared__ uint32_t s_run;  // vertices of the block so far
-  const int tid = threadIdx.x, w = tid >> 6;
-  s_nv[tid] = a.nverts[tid];
+  __shared__ float s_lo[kMcWaves], s_hi[kMcWaves];
+  // count pass, per (isovalue of the round, wave), of two rounds in turn:
+  // vertices, active cells, case vertices; corrections to the vertices
+  __shared__ uint32_t s_wt[2][kMcRound][kMcWaves], s_wa[2][kMcRound][kMcWaves];
+  __shared__ uint32_t s_wv[2][kMcRound][kMcWaves];
+  __shared__ int s_fix[kMcWaves][kMcRound];
+  __shared__ uint32_t s_run;  // count pass: vertices of the block so far
+  if (EMIT && a.block_total[blockIdx.x] == 0u) return;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if (STATS) s_nv[tid] = a.nverts[tid];
   if (!EMIT) {
-    for (int i = tid; i < kMcAcc; i += kMcBlock) { s_accv[i] = 0u; s_acca[i] = 0u; s_acct[i] = 0u; }
+    if (tid < kMcWaves * kMcRound) (&s_fix[0][0])[tid] = 0;
+    if (tid == 0) s_run = 0u;
   }
-  if (tid == 0) s_run = 0u;
 
   // A block owns a brick of 16 x 4 x 4 grid points, 16 along the memory-fast
-  // axis: a small brick spans a narrower value range than a 256-point line,
-  // so fewer isovalues reach it.
-  int px, py, pz;
+  // axis (z, or x when zfast is 0): a small brick spans a narrower value range
+  // than a 256-point line, so fewer isovalues reach it.
+  int px, py, pz;  // the block's first grid point
   {
-    const int f = tid & 15, m1 = (tid >> 4) & 3, m2 = tid >> 6;
-    const int64_t b = blockIdx.x;
-    if (a.zfast) {  // z fastest: brick 4 (x) x 4 (y) x 16 (z)
-      const int nbz = (a.npz + 15) >> 4, nby = (a.npy + 3) >> 2;
-      pz = (int)(b % nbz) * 16 + f;
-      py = (int)((b / nbz) % nby) * 4 + m1;
-      px = (int)(b / ((int64_t)nbz * nby)) * 4 + m2;
-    } else {  // x fastest: brick 16 (x) x 4 (y) x 4 (z)
-      const int nbx = (a.npx + 15) >> 4, nby = (a.npy + 3) >> 2;
-      px = (int)(b % nbx) * 16 + f;
-      py = (int)((b / nbx) % nby) * 4 + m1;
-      pz = (int)(b / ((int64_t)nbx * nby)) * 4 + m2;
+    const uint32_t nbf = (uint32_t)((a.zfast ? a.npz : a.npx) + 15) >> 4;
+    const uint32_t nby = (uint32_t)(a.npy + 3) >> 2, b = blockIdx.x;
+    const int f = (int)(b % nbf) * 16, m = (int)(b / nbf / nby) * 4;
+    py = (int)(b / nbf % nby) * 4;
+    px = a.zfast ? m : f;
+    pz = a.zfast ? f : m;
+  }
+  const int ex = a.zfast ? 4 : 16, ez = a.zfast ? 16 : 4;  // the brick's extent
+  {
+    float lo = 3.4e38f, hi = -3.4e38f;
+    const uint32_t sm = (uint32_t)(a.zfast ? a.sx : a.sz), sy = (uint32_t)a.sy;
+    const bool inside = px + (a.zfast ? kMcM : kMcF) <= a.gx && py + kMcM <= a.gy &&
+                        pz + (a.zfast ? kMcF : kMcM) <= a.gz;
+    const float *corner = a.vol + (px * a.sx + py * a.sy + pz * a.sz);
+#pragma unroll
+    for (uint32_t i = tid; i < kMcF * kMcM * kMcM; i += kMcBlock) {
+      const uint32_t row = (i * 241u) >> 12, f = i - row * kMcF;  // i / 17 below 425
+      const uint32_t m2 = (row * 205u) >> 10, m1 = row - m2 * kMcM;  // row / 5 below 25
+      float v;
+      if (inside) {
+        v = corner[f + m1 * sy + m2 * sm];  // below 5 / 2 x the grid points in all
+      } else {
+        const int x = min(px + (int)(a.zfast ? m2 : f), a.gx - 1), y = min(py + (int)m1, a.gy - 1);
+        const int z = min(pz + (int)(a.zfast ? f : m2), a.gz - 1);
+        v = a.vol[x * a.sx + y * a.sy + z * a.sz];
+      }
+      s_v[i] = v;
+      lo = fminf(lo, v);
+      hi = fmaxf(hi, v);
     }
+    wave_minmax(lo, hi);
+    if (lane == 0) { s_lo[w] = lo; s_hi[w] = hi; }
   }
-  const bool live = px < a.npx && py < a.npy && pz < a.npz;
-  if (!live) { px = 0; py = 0; pz = 0; }
-  // the eight corner samples of the cell at P, reference corner order
-  float s[8];
+  __syncthreads();
+  int j0, j1;
   {
-    const int x0 = min(px, a.gx - 1), x1 = min(px + 1, a.gx - 1);
-    const int y0 = min(py, a.gy - 1), y1 = min(py + 1, a.gy - 1);
-    const int z0 = min(pz, a.gz - 1), z1 = min(pz + 1, a.gz - 1);
-    const float *v = a.vol;
-    s[0] = v[x0 * a.sx + y0 * a.sy + z0 * a.sz];
-    s[1] = v[x1 * a.sx + y0 * a.sy + z0 * a.sz];
-    s[2] = v[x1 * a.sx + y1 * a.sy + z0 * a.sz];
-    s[3] = v[x0 * a.sx + y1 * a.sy + z0 * a.sz];
-    s[4] = v[x0 * a.sx + y0 * a.sy + z1 * a.sz];
-    s[5] = v[x1 * a.sx + y0 * a.sy + z1 * a.sz];
-    s[6] = v[x1 * a.sx + y1 * a.sy + z1 * a.sz];
-    s[7] = v[x0 * a.sx + y1 * a.sy + z1 * a.sz];
-  }
-  // which cells around P exist and are classified (isovalue independent)
-  const bool c000 = live && cell_ok(a, px, py, pz);
-  const bool c001 = live && cell_ok(a, px, py, pz - 1);
-  const bool c010 = live && cell_ok(a, px, py - 1, pz);
-  const bool c011 = live && cell_ok(a, px, py - 1, pz - 1);
-  const bool c100 = live && cell_ok(a, px - 1, py, pz);
-  const bool c101 = live && cell_ok(a, px - 1, py, pz - 1);
-  const bool c110 = live && cell_ok(a, px - 1, py - 1, pz);
-  const bool xp = c000 || c001, xm = c010 || c011;   // x edge: + / - orientation present
-  const bool yp = c100 || c101, ym = c000 || c001;   // y edge
-  const bool zp = c000 || c100 || c010 || c110;      // z edge (always +)
-  const bool any = xp || xm || yp || ym || zp;
-
-  float lo = 3.4e38f, hi = -3.4e38f;
-  if (any) {
+    float lo = s_lo[0], hi = s_hi[0];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) { lo = fminf(lo, s[q]); hi = fmaxf(hi, s[q]); }
+    for (int q = 1; q < kMcWaves; ++q) { lo = fminf(lo, s_lo[q]); hi = fmaxf(hi, s_hi[q]); }
+    const int2 r = iso_range(a.isos, a.k, lo, hi);
+    j0 = r.x;
+    j1 = r.y;
   }
-  // an isovalue can touch this lane only if lane_lo < iso <= lane_hi (an edge
-  // crosses iff min(a,b) < iso <= max(a,b); outside, the cell case is 0 or 255)
-  const float lane_lo = lo, lane_hi = hi;
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    lo = fminf(lo, __shfl_xor(lo, o, 64));
-    hi = fmaxf(hi, __shfl_xor(hi, o, 64));
+  if (j0 >= j1) {
+    if (!EMIT && tid == 0) a.block_total[blockIdx.x] = 0u;
+    return;
   }
-  if ((tid & 63) == 0) { s_lo[tid >> 6] = lo; s_hi[tid >> 6] = hi; }
-  __syncthreads();
-  if (tid == 0) {
-    float L = s_lo[0], Hh = s_hi[0];
-    for (int w = 1; w < kMcBlock / 64; ++w) { L = fminf(L, s_lo[w]); Hh = fmaxf(Hh, s_hi[w]); }
-    // isovalues with L < iso <= Hh: [upper_bound(L), upper_bound(Hh))
-    int b0 = 0, e0 = a.k;
-    while (b0 < e0) { int m = (b0 + e0) >> 1; if (a.isos[m] > L) e0 = m; else b0 = m + 1; }
-    int b1 = b0, e1 = a.k;
-    while (b1 < e1) { int m = (b1 + e1) >> 1; if (a.isos[m] > Hh) e1 = m; else b1 = m + 1; }
-    s_range[0] = b0;
-    s_range[1] = L <= Hh ? b1 : b0;
-  }
-  __syncthreads();
-  const int j0 = s_range[0], j1 = s_range[1];
-  const float fx = (float)px, fy = (float)py, fz = (float)pz;
-  const int lane = tid & 63;
-  const uint32_t pid = (uint32_t)(((int64_t)pz * a.npy + py) * a.npx + px);  // candidate ids
-  const int priv = (int)(blockIdx.x % kMcPriv);
 
-  const int64_t cap = a.cap;
-  float *o = a.out;
-  uint32_t *os = a.out_slot;
+  // this lane's grid point, and the steps to its neighbours in s_v
+  const int lf = lane & 15, l1 = lane >> 4;
+  const int x = px + (a.zfast ? w : lf), y = py + l1, z = pz + (a.zfast ? lf : w);
+  const int dx = a.zfast ? kMcF * kMcM : 1, dz = a.zfast ? 1 : kMcF * kMcM;
+  const int at = lf + kMcF * l1 + kMcF * kMcM * w;
+  const float v0 = s_v[at], vx = s_v[at + dx], vy = s_v[at + kMcF], vz = s_v[at + dz];
+  // which cells around P exist and are classified (isovalue independent):
+  // all of them, inside
+  bool xp = true, xm = true, yp = true, ym = true, zp = true, cell = true;
+  if (px == 0 || py == 0 || pz == 0 || px + ex > a.ncx || py + 4 > a.ncy || pz + ez > a.ncz ||
+      px + ex - 1 + (int64_t)a.gx * (py + 3 + (int64_t)a.gy * (pz + ez - 1)) >= a.ncls) {
+    const bool live = x < a.npx && y < a.npy && z < a.npz;
+    const bool c000 = live && cell_ok(a, x, y, z);
+    const bool c001 = live && cell_ok(a, x, y, z - 1);
+    const bool c010 = live && cell_ok(a, x, y - 1, z);
+    const bool c011 = live && cell_ok(a, x, y - 1, z - 1);
+    const bool c100 = live && cell_ok(a, x - 1, y, z);
+    const bool c101 = live && cell_ok(a, x - 1, y, z - 1);
+    const bool c110 = live && cell_ok(a, x - 1, y - 1, z);
+    xp = c000 || c001;  // x edge: + / - orientation present
+    xm = c010 || c011;
+    yp = c100 || c101;  // y edge
+    ym = c000 || c001;
+    zp = c000 || c100 || c010 || c110;  // z edge (always +)
+    cell = c000;
+  }
+  const uint64_t has_x = __ballot(xp || xm), has_y = __ballot(yp || ym), has_z = __ballot(zp);
+  // a crossing: lane | edge << 6 | + present << 8 | - present << 9 | isovalue << 10
+  const uint32_t item_x = lane | (uint32_t)xp << 8 | (uint32_t)xm << 9;
+  const uint32_t item_y = lane | 1u << 6 | (uint32_t)yp << 8 | (uint32_t)ym << 9;
+  const uint32_t item_z = lane | 2u << 6 | 1u << 8;
+  // the isovalues this wave's edges can cross
+  int2 own = make_int2(j0, j1);
+  if (!EMIT && !STATS) {
+    float lo = fminf(fminf(v0, vx), fminf(vy, vz)), hi = fmaxf(fmaxf(v0, vx), fmaxf(vy, vz));
+    wave_minmax(lo, hi);
+    own = iso_range(a.isos, a.k, lo, hi);
+  }
   const int64_t bbase = EMIT ? (int64_t)a.block_base[blockIdx.x] : 0;
-  for (int jc = j0; jc < j1; jc += kMcRound) {
+  float *const out = a.out + 3 * bbase;
+  uint32_t *const out_slot = a.out_slot ? a.out_slot + bbase : nullptr;
+  const uint32_t room = EMIT ? (uint32_t)min(max(a.cap - bbase, (int64_t)0), (int64_t)INT32_MAX) : 0u;
+  uint32_t run = 0;  // emit pass: vertices of the block in the rounds before
+  for (int jc = j0, round = 0; jc < j1; jc += kMcRound, ++round) {
     const int jn = min(kMcRound, j1 - jc);
-    uint16_t *wc = a.wave_counts + ((int64_t)blockIdx.x * a.max_rounds + (jc - j0) / kMcRound) *
+    uint16_t *wc = a.wave_counts + ((int64_t)blockIdx.x * a.max_rounds + round) *
                                        (kMcRound * kMcWaves);
+    // lane u holds isovalue u of the round
+    const float iso_u = lane < jn ? a.isos[jc + lane] : 0.0f;
+    const int slot_u = lane < jn ? a.slot[jc + lane] : 0;
+    uint32_t count_u = 0, rel_u = 0;
+    uint64_t todo;  // the isovalues to look at
     if (EMIT) {
-      // this round's vertices per (isovalue, wave) from the count pass, then
-      // the offsets of (isovalue, wave) within the block
-      if (tid < jn * kMcWaves) s_wt[tid / kMcWaves][tid % kMcWaves] = wc[tid];
-      __syncthreads();
-      if (tid == 0) {
-        uint32_t run = s_run;
-        for (int u = 0; u < jn; ++u)
-          for (int q = 0; q < kMcWaves; ++q) {
-            s_off[u][q] = run;
-            run += s_wt[u][q];
-          }
-        s_run = run;
-      }
-      __syncthreads();
+      // the vertices of the round's isovalues in each wave from the count pass
+      ushort4 c = make_ushort4(0, 0, 0, 0);
+      if (lane < jn) c = ((const ushort4 *)wc)[lane];
+      const uint32_t mine = w == 0 ? c.x : w == 1 ? c.y : w == 2 ? c.z : c.w;
+      const uint32_t before = (w > 0 ? c.x : 0) + (w > 1 ? c.y : 0) + (w > 2 ? c.z : 0);
+      uint32_t all, ours;
+      rel_u = run + before + prefix32(c.x + c.y + c.z + c.w, all) - prefix32(mine, ours);
+      run += all;
+      todo = __ballot(mine != 0u);
+    } else {
+      const int u0 = max(own.x - jc, 0), u1 = min(own.y - jc, jn);
+      todo = u1 > u0 ? (~0ull >> (64 - u1)) & (~0ull << u0) : 0ull;
     }
-    for (int u = 0; u < jn; ++u) {
-      const float iso = a.isos[jc + u];
-      if (__ballot(lane_lo < iso && iso <= lane_hi) == 0) {  // nothing for this wave
-        if (!EMIT && lane == 0) { s_wt[u][w] = 0u; s_wa[u][w] = 0u; s_wv[u][w] = 0u; }
-        continue;
-      }
-      const int slot = a.slot[jc + u];
-      const bool in0 = s[0] < iso;
-      // candidate vertices: x+, x-, y+, y-, z+ (value along the edge axis)
-      float vxp = 0, vxm = 0, vyp = 0, vym = 0, vzp = 0;
-      bool exp_ = false, exm = false, eyp = false, eym = false, ezp = false;
-      if ((xp || xm) && in0 != (s[1] < iso)) {
-        if (xp) { vxp = fx + (iso - s[0]) / (s[1] - s[0]); exp_ = true; }
-        if (xm) { vxm = (fx + 1.0f) - (iso - s[1]) / (s[0] - s[1]); exm = true; }
-        if (exp_ && exm && vxp == vxm) exm = false;
-      }
-      if ((yp || ym) && in0 != (s[3] < iso)) {
-        if (yp) { vyp = fy + (iso - s[0]) / (s[3] - s[0]); eyp = true; }
-        if (ym) { vym = (fy + 1.0f) - (iso - s[3]) / (s[0] - s[3]); eym = true; }
-        if (eyp && eym && vyp == vym) eym = false;
-      }
-      if (zp && in0 != (s[4] < iso)) { vzp = fz + (iso - s[0]) / (s[4] - s[0]); ezp = true; }
+    uint32_t head = 0, tail = 0, seq = 0;
+    // works out the n crossings at the queue's head, one per lane
+    auto work_out = [&](uint32_t n) {
+      const uint32_t item = s_queue[w][(head + lane) & (kMcQueue - 1)];
+      const bool valid = (uint32_t)lane < n;
+      const int l = item & 63, edge = (item >> 6) & 3, u = (item >> 10) & 31;
+      const bool plus = item & (1u << 8), minus = item & (1u << 9);
+      const int qf = l & 15, q1 = (l >> 4) & 3;
+      const int qx = px + (a.zfast ? w : qf), qy = py + q1, qz = pz + (a.zfast ? qf : w);
+      const int p0 = qf + kMcF * q1 + kMcF * kMcM * w;
+      const float f0 = s_v[p0], f1 = s_v[p0 + (edge == 0 ? dx : edge == 1 ? kMcF : dz)];
+      const float iso = __int_as_float(__builtin_amdgcn_ds_bpermute(u << 2, __float_as_int(iso_u)));
+      const float fx = (float)qx, fy = (float)qy, fz = (float)qz;
+      const float base = edge == 0 ? fx : edge == 1 ? fy : fz;
+      const float vp = base + (iso - f0) / (f1 - f0);
+      const float vm = (base + 1.0f) - (iso - f1) / (f0 - f1);
+      bool has_p = valid && plus, has_m = valid && minus && !(plus && vp == vm);
       // grid-point vertices: the first claim wins (count pass), its owner emits
-      const uint64_t kslot = (uint64_t)slot << 40;
-      auto gp = [&](int gxp, int gyp, int gzp) {
-        return kslot | (uint64_t)((int64_t)gxp + (int64_t)a.npx * ((int64_t)gyp + (int64_t)a.npy * gzp));
-      };
-      auto take = [&](uint64_t key, uint32_t kind) {
-        const uint32_t id = pid * 5u + kind;
-        return EMIT ? corner_owned(a, key, id) : corner_claim(a, key, id);
-      };
-      if (exp_ && (vxp == fx || vxp == fx + 1.0f)) exp_ = take(gp((int)vxp, py, pz), 0);
-      if (exm && (vxm == fx || vxm == fx + 1.0f)) exm = take(gp((int)vxm, py, pz), 1);
-      if (eyp && (vyp == fy || vyp == fy + 1.0f)) eyp = take(gp(px, (int)vyp, pz), 2);
-      if (eym && (vym == fy || vym == fy + 1.0f)) eym = take(gp(px, (int)vym, pz), 3);
-      if (ezp && (vzp == fz || vzp == fz + 1.0f)) ezp = take(gp(px, py, (int)vzp), 4);
-      const uint32_t cnt = (uint32_t)exp_ + exm + eyp + eym + ezp;
-      // cnt <= 5 (3 bits) over bit-sliced ballots: the wave's sum (count
-      // pass) or this lane's place in the wave's run (emit pass)
-      const uint64_t b0 = __ballot(cnt & 1u), b1 = __ballot(cnt & 2u), b2 = __ballot(cnt & 4u);
-      if (EMIT) {
-        if (cnt) {
-          int64_t pos = bbase + s_off[u][w] + lane_prefix(b0) + 2 * lane_prefix(b1) +
-                        4 * lane_prefix(b2);
-          auto put = [&](float x, float y, float z) {
-            if (pos < cap) {
-              o[3 * pos] = x;
-              o[3 * pos + 1] = y;
-              o[3 * pos + 2] = z;
-              if (os) os[pos] = (uint32_t)slot;
-            }
-            ++pos;
-          };
-          if (exp_) put(vxp, fy, fz);
-          if (exm) put(vxm, fy, fz);
-          if (eyp) put(fx, vyp, fz);
-          if (eym) put(fx, vym, fz);
-          if (ezp) put(fx, fy, vzp);
-        }
-        continue;
+      const bool grid_p = has_p && (vp == base || vp == base + 1.0f);
+      const bool grid_m = has_m && (vm == base || vm == base + 1.0f);
+      int slot = 0;
+      if (EMIT || __ballot(grid_p || grid_m)) slot = __builtin_amdgcn_ds_bpermute(u << 2, slot_u);
+      if (grid_p || grid_m) {
+        const uint32_t id =
+            (uint32_t)(((int64_t)qz * a.npy + qy) * a.npx + qx) * 5u + 2u * (uint32_t)edge;
+        auto take = [&](float v, uint32_t kind) {
+          const int gx = edge == 0 ? (int)v : qx, gy = edge == 1 ? (int)v : qy;
+          const int gz = edge == 2 ? (int)v : qz;
+          const uint64_t key =
+              (uint64_t)slot << 40 |
+              (uint64_t)((int64_t)gx + (int64_t)a.npx * ((int64_t)gy + (int64_t)a.npy * gz));
+          return EMIT ? corner_owned(a, key, id + kind) : corner_claim(a, key, id + kind);
+        };
+        if (grid_p) has_p = take(vp, 0u);
+        if (grid_m) has_m = take(vm, 1u);
       }
-      const uint32_t cnt_w = __popcll(b0) + 2 * __popcll(b1) + 4 * __popcll(b2);
-      if (lane == 0) s_wt[u][w] = cnt_w;
-      if (!EMIT && STATS) {
-        // cell statistics of the cell at P
-        uint32_t act = 0, tot = 0;
-        if (c000) {
-          uint32_t ci = 0;
+      if (EMIT) {
+        const uint64_t bp = __ballot(has_p), bm = __ballot(has_m);
+        const uint32_t rel = (uint32_t)__builtin_amdgcn_ds_bpermute(u << 2, (int)rel_u);
+        uint32_t pos = rel + seq + lane_prefix(bp) + lane_prefix(bm);
+        seq += (uint32_t)__popcll(bp) + (uint32_t)__popcll(bm);
+        auto put = [&](float v) {
+          if (pos < room) {
+            float3 p;
+            p.x = edge == 0 ? v : fx;
+            p.y = edge == 1 ? v : fy;
+            p.z = edge == 2 ? v : fz;
+            *(float3 *)(out + 3u * pos) = p;
+            if (out_slot) out_slot[pos] = (uint32_t)slot;
+          }
+          ++pos;
+        };
+        if (has_p) put(vp);
+        if (has_m) put(vm);
+      } else {  // one vertex has been counted for it
+        const int fix = (int)has_p + (int)has_m - 1;
+        if (valid && fix) atomicAdd(&s_fix[w][u], fix);
+      }
+      head += n;
+    };
+    while (todo) {
+      const int u = __ffsll((unsigned long long)todo) - 1;
+      todo &= todo - 1;
+      const float iso = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(iso_u), u));
+      const uint64_t m0 = __ballot(v0 < iso);
+      const uint64_t cx = (m0 ^ __ballot(vx < iso)) & has_x;
+      const uint64_t cy = (m0 ^ __ballot(vy < iso)) & has_y;
+      const uint64_t cz = (m0 ^ __ballot(vz < iso)) & has_z;
+      const uint32_t n = (uint32_t)__popcll(cx) + (uint32_t)__popcll(cy) + (uint32_t)__popcll(cz);
+      if (n) {
+        // a lane's crossings in a row, lane after lane
+        uint32_t r = tail + lane_prefix(cx) + lane_prefix(cy) + lane_prefix(cz);
+        const uint32_t tag = (uint32_t)u << 10;
+        if (__builtin_amdgcn_inverse_ballot_w64(cx)) s_queue[w][r++ & (kMcQueue - 1)] = item_x | tag;
+        if (__builtin_amdgcn_inverse_ballot_w64(cy)) s_queue[w][r++ & (kMcQueue - 1)] = item_y | tag;
+        if (__builtin_amdgcn_inverse_ballot_w64(cz)) s_queue[w][r & (kMcQueue - 1)] = item_z | tag;
+        tail += n;
+        if (!EMIT) count_u = lane == u ? n : count_u;
+        while (tail - head >= 64u) work_out(64u);
+      }
+      if (STATS) {
+        // cell statistics of the cell at P, reference corner order
+        const float s[8] = {v0,
+                            vx,
+                            s_v[at + dx + kMcF],
+                            vy,
+                            vz,
+                            s_v[at + dx + dz],
+                            s_v[at + dx + kMcF + dz],
+                            s_v[at + kMcF + dz]};
+        uint32_t ci = 0;
 #pragma unroll
-          for (int q = 0; q < 8; ++q) ci |= (uint32_t)(s[q] < iso) << q;
-          tot = s_nv[ci];
-          act = tot > 0;
-        }
-        const uint32_t act_w = __popcll(__ballot(act != 0));
+        for (int q = 0; q < 8; ++q) ci |= (uint32_t)(s[q] < iso) << q;
+        const uint32_t tot = cell ? s_nv[ci] : 0u;
+        const uint32_t act_w = __popcll(__ballot(tot != 0u));
         const uint32_t tot_w = __popcll(__ballot(tot & 1u)) + 2 * __popcll(__ballot(tot & 2u)) +
                                4 * __popcll(__ballot(tot & 4u)) + 8 * __popcll(__ballot(tot & 8u));
-        if (lane == 0) { s_wa[u][w] = act_w; s_wv[u][w] = tot_w; }
+        if (lane == 0) { s_wa[round & 1][u][w] = act_w; s_wv[round & 1][u][w] = tot_w; }
       }
     }
-    __syncthreads();
+    if (tail != head) work_out(tail - head);
     if (!EMIT) {
-      if (tid < jn * kMcWaves) wc[tid] = (uint16_t)s_wt[tid / kMcWaves][tid % kMcWaves];
-      // one lane per isovalue of the round folds the wave sums into the block's
+      if (lane < jn) {
+        s_wt[round & 1][lane][w] = count_u + (uint32_t)s_fix[w][lane];
+        s_fix[w][lane] = 0;
+      }
+      // the waves' counts of a round are read while the next one's go into the
+      // other half
+      __syncthreads();
       if (tid < jn) {
-        uint32_t vj = 0, aj = 0, tj = 0;
+        const uint32_t *wt = s_wt[round & 1][tid];
+        ((ushort4 *)wc)[tid] = make_ushort4((uint16_t)wt[0], (uint16_t)wt[1], (uint16_t)wt[2],
+                                            (uint16_t)wt[3]);
+        const uint32_t vj = wt[0] + wt[1] + wt[2] + wt[3];
+        uint32_t aj = 0, tj = 0;
+        if (STATS) {
 #pragma unroll
-        for (int q = 0; q < kMcWaves; ++q) {
-          vj += s_wt[tid][q];
-          if (STATS) { aj += s_wa[tid][q]; tj += s_wv[tid][q]; }
-        }
-        const int r = jc + tid - j0;
-        if (r < kMcAcc) {
-          s_accv[r] += vj;
-          if (STATS) { s_acca[r] += aj; s_acct[r] += tj; }
-        } else if (vj || aj) {  // past the LDS accumulators: straight to the counters
-          const int slot = a.slot[jc + tid];
-          atomicAdd(&a.counts_priv[(int64_t)priv * a.k + slot], vj);
-          if (STATS) {
-            atomicAdd(&a.stats_priv[((int64_t)priv * a.k + slot) * 2], (unsigned long long)aj);
-            atomicAdd(&a.stats_priv[((int64_t)priv * a.k + slot) * 2 + 1], (unsigned long long)tj);
+          for (int q = 0; q < kMcWaves; ++q) {
+            aj += s_wa[round & 1][tid][q];
+            tj += s_wv[round & 1][tid][q];
           }
         }
-        if (vj) atomicAdd(&s_run, vj);
-      }
-      __syncthreads();  // s_wt is rewritten by the next round
-    }
-    // (emit pass: the barrier above ends the round's reads of s_off and s_wt)
-  }
-  if (!EMIT) {
-    __syncthreads();
-    if (tid == 0) a.block_total[blockIdx.x] = s_run;
-    const int nacc = min(j1 - j0, kMcAcc);
-    for (int r = tid; r < nacc; r += kMcBlock) {
-      const uint32_t vj = s_accv[r], aj = s_acca[r], tj = s_acct[r];
-      if (vj || aj) {
-        const int slot = a.slot[j0 + r];
-        atomicAdd(&a.counts_priv[(int64_t)priv * a.k + slot], vj);
-        if (STATS) {
-          atomicAdd(&a.stats_priv[((int64_t)priv * a.k + slot) * 2], (unsigned long long)aj);
-          atomicAdd(&a.stats_priv[((int64_t)priv * a.k + slot) * 2 + 1], (unsigned long long)tj);
+        const int64_t priv = (int64_t)(blockIdx.x % kMcPriv) * a.k + slot_u;
+        if (vj) {
+          atomicAdd(&a.counts_priv[priv], vj);
+          atomicAdd(&s_run, vj);
+        }
+        if (STATS && aj) {
+          atomicAdd(&a.stats_priv[priv * 2], (unsigned long long)aj);
+          atomicAdd(&a.stats_priv[priv * 2 + 1], (unsigned long long)tj);
         }
       }
     }
   }
+  // (wave 0 added up the rounds)
+  if (!EMIT && tid == 0) a.block_total[blockIdx.x] = s_run;
 }
 
 // Per-isovalue totals from the privatised counters (counts[s] = the sum of
