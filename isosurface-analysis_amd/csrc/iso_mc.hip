@@ -48,6 +48,7 @@ constexpr int kMcBlock = 256;
 constexpr int kMcWaves = kMcBlock / 64;
 constexpr int kMcRound = 32;  // isovalues per pool reservation (bit masks of 32)
 constexpr unsigned long long kEmpty = ~0ull;
+constexpr int kMcOddVertices = 4;  // word of the counters
 
 // ---- case tables, generated from first principles -------------------------
 // Corners 0..7 of a cell sit at (0,0,0) (1,0,0) (1,1,0) (0,1,0) (0,0,1)
@@ -766,7 +767,8 @@ __global__ __launch_bounds__(kApBlock) void approx_multi_kernel(ApMultiArgs a) {
 
 namespace iso {
 
-int sort_vertices_lex(iso_ctx *ctx, float *d_xyz, int64_t n);
+int sort_vertices_lex(iso_ctx *ctx, float *d_xyz, int64_t n, int gx, int gy, int gz,
+                      uint32_t *d_odd);
 
 // Voxel approximation at k isovalues in one pass, pool output like mc_multi.
 int approx_multi(iso_ctx *ctx, const float *d_img, int X, int Y, int Z, const float *d_isos_sorted,
@@ -896,7 +898,8 @@ int mc_multi(iso_ctx *ctx, const float *d_vol, int gx, int gy, int gz, uint32_t 
     ISO_TRY(ws_get(ctx, WS_MC_CORNER_TABLE, slots * 12, false, &tab));  // keys, then owners
     ISO_TRY(ws_get(ctx, WS_MC_COUNTERS, 64, false, &ctr));
     ISO_TRY(fill_u32(ctx, tab, 0xffffffffu, slots * 2));
-    ISO_TRY(fill_u32(ctx, ctr, 0u, 4));  // [overflow, vertex total, 64-bit vertex total]
+    // [overflow, vertex total, 64-bit vertex total, kMcOddVertices: of a sort to follow]
+    ISO_TRY(fill_u32(ctx, ctr, 0u, 5));
     ISO_TRY(fill_u32(ctx, priv, 0u, (size_t)kMcPriv * k * 5));
     a.corner_tab = (unsigned long long *)tab;
     a.corner_owner = (uint32_t *)(a.corner_tab + slots);
@@ -1017,7 +1020,11 @@ int iso_mc_extract(iso_ctx *ctx, const float *d_vol, int gx, int gy, int gz, flo
   if ((int64_t)hs.count > cap)
     return iso::fail(ctx, ISO_ERR_CAPACITY, "iso_mc_extract: %lld vertices, capacity %lld",
                      (long long)hs.count, (long long)cap);
-  if (flags & ISO_MC_SORTED) ISO_TRY(iso::sort_vertices_lex(ctx, d_xyz, hs.count));
+  if ((flags & ISO_MC_SORTED) && hs.count > 1) {
+    void *ctr = nullptr;
+    ISO_TRY(iso::ws_get(ctx, WS_MC_COUNTERS, 64, false, &ctr));
+    ISO_TRY(iso::sort_vertices_lex(ctx, d_xyz, hs.count, gx, gy, gz, (uint32_t *)ctr + kMcOddVertices));
+  }
   ISO_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
   return ISO_OK;
 }
