@@ -1538,14 +1538,16 @@ int df_pool(iso_ctx *ctx, const void *d_xyz, bool is_int, int64_t ntot, const ui
                        (const int *)la, (const uint32_t *)cnt, (int *)roots);
     // bricks of 4 x 4 x 4*spl samples
     const int bx = (g.nx + 3) / 4, by = (g.ny + 3) / 4, bz = (g.nz + 4 * spl - 1) / (4 * spl);
-    // persistent: up to 8 waves per SIMD (4 SIMDs per CU); with at least 4
-    // bricks per wave they pull chunks of about 1/16 of their share from
-    // cnt[2], rounded up to whole columns of bz bricks (a chunk then starts a
-    // column, and every brick but a column's first starts from the bound of
-    // the brick below it), else each takes a fixed stride
+    // With at least 4 bricks per wave that fits on the chip (8 per SIMD), waves
+    // stay and pull chunks of about 1/16 of their share from cnt[2], rounded up
+    // to whole columns of bz bricks (a chunk then starts a column, and every
+    // brick but a column's first starts from the bound of the brick below it).
+    // With fewer, a wave per brick: the bricks' costs differ by far more than a
+    // wave's start (16,384 bricks of 64^3 samples, 16 isovalues: walk 238 -> 205
+    // us against two bricks a wave; 9,728 of one isovalue: 292 -> 263).
     const uint64_t total = (uint64_t)bx * by * bz * (uint64_t)S;
     const uint64_t max_waves = (uint64_t)ctx->cu_count * 32;
-    const uint64_t waves = std::min<uint64_t>(max_waves, (total + 1) / 2);
+    const uint64_t waves = total < 4 * max_waves ? total : max_waves;
     uint32_t chunk = 0u, nbig = 0u, nhalf = 0u, small = 1u;
     if (total >= 4 * waves) {
       const uint64_t c = std::min<uint64_t>(256, std::max<uint64_t>(1, total / (waves * 16)));
