@@ -49,7 +49,7 @@ struct BatchArgs {
   const float *mins, *maxs;  // per field of the batch (DistanceField::getInterval)
   const BatchTask *tasks;
   int ntasks;
-  uint32_t *next;          // queue head, cleared before each launch
+  uint32_t *next;          // queue heads, cleared before each launch
   float *const *maps;      // per job: map (row-major n x n)
   uint32_t *ghist;         // per workgroup drain area (16-bit path), zero at rest
   int H;
@@ -59,6 +59,15 @@ struct BatchArgs {
 };
 
 constexpr int kBBlock = iso::kHistBlock;
+
+// The tasks come in tiles of 4 x 8 pairs of fields, and kTile tasks in a row go
+// to one queue.  Workgroup b (XCD b % kQueues) takes from queue b % kQueues, so
+// the pairs that run on an XCD at a time share 12 fields in its L2; when its
+// queue is empty it goes on with the next one's.  31,054 pairs of 8 volumes, 128
+// bins: 10.05 -> 9.5 ms, 36 GB past the L2s, against one queue in row order.
+constexpr int kTileI = 4, kTileJ = 8, kTile = kTileI * kTileJ;
+constexpr int kQueues = 8;
+constexpr int kHeadStride = 8;  // words between two queue heads
 
 // Everything a workgroup keeps in LDS, after the histogram.
 template <bool PACK16>
@@ -77,9 +86,17 @@ __global__ __launch_bounds__(kBBlock) __attribute__((amdgpu_waves_per_eu(PACK16 
   const int tid = threadIdx.x, H = a.H;
   const int words = H * iso::kRowWords;
   uint32_t *gh = a.ghist + (int64_t)blockIdx.x * H * H;
+  int queue = blockIdx.x % kQueues, empty = 0;  // (lane 0's)
   while (true) {
     if (tid == 0) {
-      s.task = (int)atomicAdd(a.next, 1u);
+      int task;
+      while (true) {
+        const uint32_t i = atomicAdd(a.next + queue * kHeadStride, 1u);
+        task = (int)min((i / kTile * kQueues + queue) * kTile + i % kTile, (uint32_t)a.ntasks);
+        if (task < a.ntasks || ++empty == kQueues) break;
+        queue = (queue + 1) % kQueues;
+      }
+      s.task = task;
       s.prog[0] = s.prog[1] = 0u;
       s.flushed = 0;
     }
@@ -106,7 +123,7 @@ __global__ __launch_bounds__(kBBlock) __attribute__((amdgpu_waves_per_eu(PACK16 
             s.flushed = 1;
           });
         else
-          iso::accumulate32<SUB, 8>(bin, f1 + b, f2 + b, len, s_hist);
+          iso::accumulate32<SUB, 4>(bin, f1 + b, f2 + b, len, s_hist);
       };
       if (__builtin_amdgcn_readfirstlane(bin.subtract)) accumulate(std::true_type());
       else accumulate(std::false_type());
@@ -267,22 +284,24 @@ int iso_ism_batch(iso_ctx *ctx, iso_ism_job *jobs, int njobs, int extractor, int
     ISO_TRY(iso::field_interval(ctx, fb, m, F[b], d_mins + mmbase, d_maxs + mmbase));
     int64_t processed = F[b];
     if ((flags & ISO_COMPAT_HIST_CHUNKS) && F[b] > 0 && F[b] % 1000000 == 0) processed -= 1000000;
-    for (int i = 0; i < m; ++i)
-      for (int j = i; j < m; ++j) {
-        BatchTask t;
-        t.fi = fbase[b] + (int64_t)i * F[b];
-        t.fj = fbase[b] + (int64_t)j * F[b];
-        t.F = F[b];
-        t.processed = processed;
-        t.mm_i = mmbase + i;
-        t.mm_j = mmbase + j;
-        t.pad0 = t.pad1 = 0;
-        t.map_i = i;
-        t.map_j = j;
-        t.job = b;
-        t.n = m;
-        tasks.push_back(t);
-      }
+    for (int i0 = 0; i0 < m; i0 += kTileI)
+      for (int j0 = i0 / kTileJ * kTileJ; j0 < m; j0 += kTileJ)
+        for (int i = i0; i < std::min(m, i0 + kTileI); ++i)
+          for (int j = std::max(i, j0); j < std::min(m, j0 + kTileJ); ++j) {
+            BatchTask t;
+            t.fi = fbase[b] + (int64_t)i * F[b];
+            t.fj = fbase[b] + (int64_t)j * F[b];
+            t.F = F[b];
+            t.processed = processed;
+            t.mm_i = mmbase + i;
+            t.mm_j = mmbase + j;
+            t.pad0 = t.pad1 = 0;
+            t.map_i = i;
+            t.map_j = j;
+            t.job = b;
+            t.n = m;
+            tasks.push_back(t);
+          }
     mmbase += m;
   }
   ISO_HIP_CHECK(ctx, hipEventRecord(ev[1], ctx->stream));
@@ -320,7 +339,7 @@ int iso_ism_batch(iso_ctx *ctx, iso_ism_job *jobs, int njobs, int extractor, int
       for (int i0 = 0; i0 < nt; i0 += most) {
         ba.tasks = d_tasks + i0;
         ba.ntasks = std::min(most, nt - i0);
-        ISO_TRY(iso::fill_u32(ctx, ba.next, 0u, 1));
+        ISO_TRY(iso::fill_u32(ctx, ba.next, 0u, kQueues * kHeadStride));
         if (pack16)
           hipLaunchKernelGGL(hist_batch_kernel<true>, dim3(groups), dim3(kBBlock), lds, ctx->stream, ba);
         else
@@ -338,7 +357,7 @@ int iso_ism_batch(iso_ctx *ctx, iso_ism_job *jobs, int njobs, int extractor, int
     const size_t cbytes = nmi32 ? per * (size_t)most + 512 : 0;
     if (nmi32) ISO_TRY(iso::nmi_logs(ctx, &ba.chains.logs));
     if (graph) {
-      // the graph owns one buffer: tasks | maps | queue head | drain area |
+      // the graph owns one buffer: tasks | maps | queue heads | drain area |
       // chains' inputs; its key is the layout: the tasks, the launch shape and
       // the inputs' addresses
       uint64_t key = 1469598103934665603ull;

@@ -99,7 +99,7 @@ struct iso_ctx {
   struct graph_entry {
     uint64_t key = 0;
     hipGraphExec_t exec = nullptr;
-    void *buf = nullptr;  // tasks | maps | queue head | drain area
+    void *buf = nullptr;  // tasks | maps | queue heads | drain area | chains
     size_t bytes = 0;
     uint64_t replays = 0;
   };
