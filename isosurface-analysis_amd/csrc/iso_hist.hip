@@ -15,9 +15,10 @@
 //     128 KB of the 160 KB LDS), 128 words to a row whatever H is;
 //   - bins are computed exactly in fixed point, and 16-bit counters hand on
 //     32,768 of their count before they can wrap (iso_bins.hpp);
-//   - slices of one pair (and what 16-bit counters handed on) merge in a global
-//     32-bit histogram; the last slice to arrive (acq/rel counter) takes the sum
-//     back into its LDS and restores the zeros, so the buffer is zero at rest;
+//   - slices of one pair leave their LDS histograms in memory, and a kernel adds
+//     them up into a global 32-bit histogram, which also takes what 16-bit
+//     counters handed on; a pair's counts go back from there into LDS and the
+//     zeros are restored, so the buffer is zero at rest;
 //   - with ISO_COMPAT_NMI32 the NMI is the reference's float evaluation in the
 //     reference's order: the workgroup writes the pair's nonzero counts out in
 //     both chain orders and a second kernel folds the chains of all pairs
@@ -57,6 +58,7 @@ constexpr int kWaves = kBlock / 64;
 // 16-bit counters that an XCD runs at once (one per CU, 32 CUs).
 constexpr int kTileRows = 4, kTileCols = 8, kTilePairs = kTileRows * kTileCols;
 constexpr int kMaxTasksPerLaunch = 16384;  // one launch per 128-isovalue ISM (no tail wave)
+constexpr size_t kMaxPartBytes = (size_t)128 << 20;  // slices' histograms of a launch
 constexpr size_t kMaxChainBytes = (size_t)4 << 30;  // chains' inputs of a launch
 
 struct HistArgs {
@@ -71,6 +73,7 @@ struct HistArgs {
   const float *maxs;
   uint32_t *ghist;    // ntasks * H*H, zero at rest
   uint32_t *arrive;   // ntasks, zero at rest
+  uint32_t *parts;    // ntasks * slices LDS histograms, or null
   float *map;
   int n;
   int multi;
@@ -101,6 +104,86 @@ struct HistLds {
   uint32_t prog[2];
   int flushed, last;
 };
+
+// The pair's merged counts back into LDS, unless one needs more than its
+// counter; returns where they are then (null: in LDS, and gh is zero again).
+template <bool PACK16>
+__device__ __forceinline__ uint32_t *take_back(uint32_t *s_hist, uint32_t *gh, int H) {
+  const int tid = threadIdx.x, words = H * iso::kRowWords;
+  bool fits = true;
+  // several words per lane under way at a time: they come from beyond the L2
+  constexpr int kAhead = 8;
+  for (int w0 = tid; w0 < words; w0 += kAhead * kBlock) {
+    uint32_t lo[kAhead], hi[kAhead];
+#pragma unroll
+    for (int q = 0; q < kAhead; ++q) {
+      const int w = w0 + q * kBlock;
+      const int r = w / iso::kRowWords, c = (PACK16 ? 2 : 1) * (w % iso::kRowWords);
+      lo[q] = w < words && c < H ? gh[r * H + c] : 0u;
+      hi[q] = PACK16 && w < words && c + 1 < H ? gh[r * H + c + 1] : 0u;
+    }
+#pragma unroll
+    for (int q = 0; q < kAhead; ++q) {
+      if (PACK16) fits &= (lo[q] | hi[q]) <= 0xffffu;
+      if (w0 + q * kBlock < words) s_hist[w0 + q * kBlock] = lo[q] | hi[q] << 16;
+    }
+  }
+  if (PACK16) fits = __syncthreads_and(fits);
+  else __syncthreads();
+  if (!fits) return gh;
+  for (int e = tid; e < H * H; e += kBlock) gh[e] = 0u;  // zero at rest
+  return nullptr;
+}
+
+// What comes of a pair's counts (in LDS, or in src): the joint histogram, the
+// marginals, the NMI or the inputs of its chains.
+template <bool PACK16>
+__device__ __forceinline__ void finish_pair(const HistArgs &a, HistLds<PACK16> &s, uint32_t *s_hist,
+                                            uint32_t *src, int task, int fi, int fj) {
+  const int tid = threadIdx.x, H = a.H, HH = H * H;
+  const bool mirror = !a.multi && fi != fj;
+  const int mj = a.multi ? fj - a.n : fj;
+  if (a.joint) {
+    // the joint histogram out (and its transpose for the mirrored entry),
+    // before the NMI reuses the LDS
+    uint32_t *jout = a.joint + ((int64_t)fi * a.n + mj) * HH;
+    uint32_t *jtr = mirror ? a.joint + ((int64_t)fj * a.n + fi) * HH : nullptr;
+    for (int e = tid; e < HH; e += kBlock) {
+      const uint32_t c = iso::pair_count<PACK16>(s_hist, src, H, e / H, e % H);
+      jout[e] = c;
+      if (jtr) jtr[(e % H) * H + e / H] = c;
+    }
+  }
+  if (a.nmi32) {
+    // ---- the chains of the reference's float order, folded by fold_kernel
+    if (PACK16 && src)
+      iso::emit_chains<PACK16, PACK16>(s_hist, a.hist_bytes, src, H, mirror, s.pair, a.chains, task);
+    else
+      iso::emit_chains<PACK16, false>(s_hist, a.hist_bytes, nullptr, H, mirror, s.pair, a.chains,
+                                      task);
+  } else {
+    // ---- fused NMI from exact counts ----
+    iso::list_bins<PACK16>(s_hist, src, H, s.pair);
+    __syncthreads();
+    const double v = iso::nmi64_pair<PACK16>(s_hist, src, H, a.F, s.pair, s.red);
+    if (tid == 0) {
+      const float out = (v != v) ? 0.0f : (float)v;
+      a.map[(int64_t)fi * a.n + mj] = out;
+      if (mirror) a.map[(int64_t)fj * a.n + fi] = out;
+    }
+  }
+  if (tid < H && a.rows) {  // (every form of the NMI ends its sums with a barrier)
+    const uint32_t r = s.pair.rows[tid], c = s.pair.cols[tid];
+    const int64_t o = ((int64_t)fi * a.n + mj) * H + tid;
+    a.rows[o] = r;
+    a.cols[o] = c;
+    if (mirror) {
+      const int64_t o2 = ((int64_t)fj * a.n + fi) * H + tid;
+      a.rows[o2] = c;
+      a.cols[o2] = r;
+    }
+  }
+}
 
 // STEP (picked by the autotuner): rounds of 8 values per lane and field on their
 // way (16-bit counters), values per step (32-bit ones).
@@ -156,8 +239,21 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(PACK16 ?
   else accumulate(std::false_type());
   __syncthreads();
 
-  const bool use_global = a.slices > 1 || s.flushed;
-  if (use_global) {
+  if (a.parts && a.slices > 1) {
+    // Slices of a pair meet in kernels of their own (merge_kernel,
+    // finish_kernel), at whose start what was stored here is visible.  Added to
+    // the pair's 32-bit histogram instead, with fences and a last workgroup that
+    // takes the sum back, which is left for callers without room for the parts,
+    // 136 pairs of 64^3 fields (128 bins, 3 slices) took 204 us with their
+    // chains, now 108; 256 pairs of 2^20 voxels 307, now 182; 3 pairs of 4M
+    // (256 bins, 85 slices) 165, now 141.  Stored here and added up by the last
+    // workgroup, the release fences wrote the L2 back each time: 254 and 376 us.
+    uint4 *const part = (uint4 *)(a.parts + ((int64_t)task * a.slices + slice) * words);
+    for (int q = tid; q < words / 4; q += kBlock) part[q] = ((const uint4 *)s_hist)[q];
+    return;
+  }
+  uint32_t *src = nullptr;  // where the pair's counts are, if not in LDS
+  if (a.slices > 1 || s.flushed) {
     // LDS -> global 32-bit histogram of this task
     for (int w = tid; w < words; w += kBlock) {
       const uint32_t v = s_hist[w];
@@ -184,73 +280,51 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(PACK16 ?
       if (!s.last) return;
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     }
+    src = take_back<PACK16>(s_hist, gh, H);
   }
-  // the merged counts back into LDS, unless one needs more than its counter
-  uint32_t *src = nullptr;  // where the pair's counts are, if not in LDS
-  if (use_global) {
-    bool fits = true;
-    for (int w = tid; w < words; w += kBlock) {
-      const int r = w / iso::kRowWords, c = (PACK16 ? 2 : 1) * (w % iso::kRowWords);
-      uint32_t v = c < H ? iso::pair_count<PACK16>(nullptr, gh, H, r, c) : 0u;
-      if (PACK16) {
-        const uint32_t hi = c + 1 < H ? iso::pair_count<PACK16>(nullptr, gh, H, r, c + 1) : 0u;
-        fits &= (v | hi) <= 0xffffu;
-        v |= hi << 16;
-      }
-      s_hist[w] = v;
-    }
-    if (PACK16) fits = __syncthreads_and(fits);
-    else __syncthreads();
-    if (fits) {
-      for (int e = tid; e < HH; e += kBlock) gh[e] = 0u;  // zero at rest
-    } else {
-      src = gh;
-    }
-  }
+  finish_pair<PACK16>(a, s, s_hist, src, task, fi, fj);
+  if (tid == 0 && a.slices > 1) a.arrive[task] = 0u;
+}
 
-  const bool mirror = !a.multi && fi != fj;
-  const int mj = a.multi ? fj - a.n : fj;
-  if (a.joint) {
-    // the joint histogram out (and its transpose for the mirrored entry),
-    // before the NMI reuses the LDS
-    uint32_t *jout = a.joint + ((int64_t)fi * a.n + mj) * HH;
-    uint32_t *jtr = mirror ? a.joint + ((int64_t)fj * a.n + fi) * HH : nullptr;
-    for (int e = tid; e < HH; e += kBlock) {
-      const uint32_t c = iso::pair_count<PACK16>(s_hist, src, H, e / H, e % H);
-      jout[e] = c;
-      if (jtr) jtr[(e % H) * H + e / H] = c;
+// The slices' histograms of a pair, added up into its 32-bit one (which holds
+// what 16-bit counters handed on).  A lane per 16 bytes of a histogram.
+template <bool PACK16>
+__global__ __launch_bounds__(256) void merge_kernel(HistArgs a) {
+  const int quads = a.H * iso::kRowWords / 4, q = blockIdx.x * 256 + threadIdx.x;
+  if (q >= quads) return;
+  const uint4 *part = (const uint4 *)a.parts + (int64_t)blockIdx.y * a.slices * quads + q;
+  uint32_t lo[4] = {}, hi[4] = {};
+#pragma unroll 8
+  for (int k = 0; k < a.slices; ++k) {
+    const uint4 v = part[(int64_t)k * quads];
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      lo[e] += PACK16 ? w[e] & 0xffffu : w[e];
+      if (PACK16) hi[e] += w[e] >> 16;
     }
   }
-  if (a.nmi32) {
-    // ---- the chains of the reference's float order, folded by fold_kernel
-    if (PACK16 && src)
-      iso::emit_chains<PACK16, PACK16>(s_hist, a.hist_bytes, src, H, mirror, s.pair, a.chains, task);
-    else
-      iso::emit_chains<PACK16, false>(s_hist, a.hist_bytes, nullptr, H, mirror, s.pair, a.chains,
-                                      task);
-  } else {
-    // ---- fused NMI from exact counts ----
-    iso::list_bins<PACK16>(s_hist, src, H, s.pair);
-    __syncthreads();
-    const double v = iso::nmi64_pair<PACK16>(s_hist, src, H, a.F, s.pair, s.red);
-    if (tid == 0) {
-      const float out = (v != v) ? 0.0f : (float)v;
-      a.map[(int64_t)fi * a.n + mj] = out;
-      if (mirror) a.map[(int64_t)fj * a.n + fi] = out;
-    }
+  const int H = a.H, row = 4 * q / iso::kRowWords, w = 4 * q % iso::kRowWords;
+  uint32_t *gh = a.ghist + (int64_t)blockIdx.y * H * H + row * H;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int c = (PACK16 ? 2 : 1) * (w + e);
+    if (lo[e]) gh[c] += lo[e];
+    if (PACK16 && hi[e]) gh[c + 1] += hi[e];
   }
-  if (tid < H && a.rows) {  // (every form of the NMI ends its sums with a barrier)
-    const uint32_t r = s.pair.rows[tid], c = s.pair.cols[tid];
-    const int64_t o = ((int64_t)fi * a.n + mj) * H + tid;
-    a.rows[o] = r;
-    a.cols[o] = c;
-    if (mirror) {
-      const int64_t o2 = ((int64_t)fj * a.n + fi) * H + tid;
-      a.rows[o2] = c;
-      a.cols[o2] = r;
-    }
-  }
-  if (tid == 0 && use_global && a.slices > 1) a.arrive[task] = 0u;
+}
+
+// ... and what comes of the merged counts, a workgroup per pair.
+template <bool PACK16>
+__global__ __launch_bounds__(kBlock) void finish_kernel(HistArgs a) {
+  extern __shared__ uint4 s_dyn[];
+  uint32_t *s_hist = reinterpret_cast<uint32_t *>(s_dyn);
+  HistLds<PACK16> &s = *reinterpret_cast<HistLds<PACK16> *>(s_hist + a.H * iso::kRowWords);
+  const int task = blockIdx.x;
+  const int2 tk = a.tasks[task];
+  iso::clear_pair_lds(s.pair);
+  uint32_t *src = take_back<PACK16>(s_hist, a.ghist + (int64_t)task * a.H * a.H, a.H);
+  finish_pair<PACK16>(a, s, s_hist, src, task, tk.x, tk.y);
 }
 
 // The float-order NMI of every task of a hist_nmi_kernel launch: kFoldPairs
@@ -367,6 +441,36 @@ int nmi_logs(iso_ctx *ctx, const float **out) {
   return ISO_OK;
 }
 
+// Slices per pair, where the pairs alone leave CUs idle (one workgroup per CU
+// with 16-bit counters, two with 32-bit ones): as few rounds of voxels as
+// possible, a slice counting another 32K voxels' time for its start and the
+// merge (10 us at 3 voxels per ns), with at least 16K voxels each (16 pairs of
+// 262,144, 128 bins, by another 32K, 16K, 8K: 108, 109, 122 us).
+// With a round or more of pairs, slices would only add merges (2,016 pairs of
+// 128^3 fields, 256 bins: 3.7 ms, cut up to even the last round out 7.0 ms).
+static int64_t slice_count(const iso_ctx *ctx, int64_t processed, int64_t nt, bool pack16) {
+  const int64_t cap = (int64_t)(pack16 ? 1 : 2) * ctx->cu_count;
+  int64_t slices = 1, best = INT64_MAX;
+  for (int64_t k = 1; nt < cap && k <= std::max<int64_t>(1, processed / 16384); ++k) {
+    const int64_t cost = (nt * k + cap - 1) / cap * (processed / k + (k > 1 ? 32768 : 0));
+    if (cost < best) {
+      best = cost;
+      slices = k;
+    }
+  }
+  return std::max(slices, (processed + kMaxSlice - 1) / kMaxSlice);
+}
+
+static int64_t processed_voxels(int64_t F, uint32_t flags) {
+  const int64_t C = 1000000;
+  return (flags & ISO_COMPAT_HIST_CHUNKS) && F > 0 && F % C == 0 ? F - C : F;
+}
+
+size_t hist_parts_bytes(const iso_ctx *ctx, int64_t F, int H, uint32_t flags, int64_t nt) {
+  const int64_t slices = slice_count(ctx, processed_voxels(F, flags), nt, H > 128);
+  return slices > 1 ? sizeof(uint32_t) * (size_t)(nt * slices) * H * kRowWords : 0;
+}
+
 // Launches the histogram+NMI kernel over a device task list.
 int hist_nmi_tasks(iso_ctx *ctx, const float *d_fields, int n, int64_t F, int H, int multi,
                    uint32_t flags, const float *d_mins, const float *d_maxs, float *d_map,
@@ -386,11 +490,7 @@ int hist_nmi_tasks(iso_ctx *ctx, const float *d_fields, int n, int64_t F, int H,
     chain_carve(b.chains, c, std::min(most, ntasks), H, F);
     ISO_TRY(nmi_logs(ctx, &b.chains.logs));
   }
-  int64_t processed = F;
-  if (flags & ISO_COMPAT_HIST_CHUNKS) {
-    const int64_t C = 1000000;
-    if (F > 0 && F % C == 0) processed = F - C;
-  }
+  const int64_t processed = processed_voxels(F, flags);
   auto run = [&](int variant) -> int {
     for (int t0 = 0; t0 < ntasks; t0 += most) {
       const int nt = std::min(ntasks - t0, most);
@@ -399,6 +499,13 @@ int hist_nmi_tasks(iso_ctx *ctx, const float *d_fields, int n, int64_t F, int H,
       ISO_TRY(ws_get(ctx, WS_HIST_ARRIVE, sizeof(uint32_t) * (size_t)nt, true, &arr));
       b.ghist = (uint32_t *)gh;
       b.arrive = (uint32_t *)arr;
+      // the slices' histograms: a few hundred workgroups' (only a slice past
+      // kMaxSlice voxels comes with more pairs than that)
+      const size_t pb = hist_parts_bytes(ctx, F, H, flags, nt);
+      void *parts = nullptr;
+      if (pb > 0 && pb <= kMaxPartBytes)
+        ISO_TRY(ws_get(ctx, WS_HIST_PARTS, pb, false, &parts));
+      b.parts = (uint32_t *)parts;
       ISO_TRY(hist_launch(ctx, d_fields, n, F, H, multi, flags, d_mins, d_maxs, d_map,
                           d_tasks + t0, nt, d_joint, d_rows, d_cols, b, variant));
     }
@@ -423,11 +530,7 @@ int hist_launch(iso_ctx *ctx, const float *d_fields, int n, int64_t F, int H, in
   const bool nmi32 = (flags & ISO_COMPAT_NMI32) != 0;
   const size_t hist_bytes = sizeof(uint32_t) * (size_t)H * kRowWords;
   const size_t lds = hist_bytes + (pack16 ? sizeof(HistLds<true>) : sizeof(HistLds<false>));
-  int64_t processed = F;
-  if (flags & ISO_COMPAT_HIST_CHUNKS) {
-    const int64_t C = 1000000;
-    if (F > 0 && F % C == 0) processed = F - C;
-  }
+  const int64_t processed = processed_voxels(F, flags);
   // variants: 16-bit counters with 1 or 2 rounds of 8 values on their way,
   // 32-bit counters with 4 or 8 values per step (the autotuner picks; 16 would
   // take too many registers for two workgroups per CU).  The LDS limit is
@@ -435,33 +538,19 @@ int hist_launch(iso_ctx *ctx, const float *d_fields, int n, int64_t F, int H, in
   static std::once_flag attr_once;
   static hipError_t attr_err = hipSuccess;
   std::call_once(attr_once, [] {
-    const void *kern[4] = {(const void *)hist_nmi_kernel<false, 4>,
+    const void *kern[6] = {(const void *)hist_nmi_kernel<false, 4>,
                            (const void *)hist_nmi_kernel<false, 8>,
                            (const void *)hist_nmi_kernel<true, 1>,
-                           (const void *)hist_nmi_kernel<true, 2>};
-    for (int v = 0; v < 4 && attr_err == hipSuccess; ++v)
+                           (const void *)hist_nmi_kernel<true, 2>,
+                           (const void *)finish_kernel<false>,
+                           (const void *)finish_kernel<true>};
+    for (int v = 0; v < 6 && attr_err == hipSuccess; ++v)
       attr_err = hipFuncSetAttribute(
           kern[v], hipFuncAttributeMaxDynamicSharedMemorySize,
-          v < 2 ? 65536 + (int)sizeof(HistLds<false>) : 131072 + (int)sizeof(HistLds<true>));
+          v < 2 || v == 4 ? 65536 + (int)sizeof(HistLds<false>) : 131072 + (int)sizeof(HistLds<true>));
   });
   ISO_HIP_CHECK(ctx, attr_err);
-  // Slices per pair, where the pairs alone leave CUs idle (one workgroup per CU
-  // with 16-bit counters, two with 32-bit ones): as few rounds of voxels as
-  // possible, a slice counting another 32K voxels' time for its start and the
-  // merge (10 us at 3 voxels per ns), with at least 16K voxels each.  136 pairs
-  // of 64^3 fields, 128 bins: 3 slices in one round 155 us, 4 in two 190 us.
-  // With a round or more of pairs, slices would only add merges (2,016 pairs of
-  // 128^3 fields, 256 bins: 3.7 ms, cut up to even the last round out 7.0 ms).
-  const int64_t cap = (int64_t)(pack16 ? 1 : 2) * ctx->cu_count;
-  int64_t slices = 1, best = INT64_MAX;
-  for (int64_t k = 1; nt < cap && k <= std::max<int64_t>(1, processed / 16384); ++k) {
-    const int64_t cost = (nt * k + cap - 1) / cap * (processed / k + (k > 1 ? 32768 : 0));
-    if (cost < best) {
-      best = cost;
-      slices = k;
-    }
-  }
-  slices = std::max(slices, (processed + kMaxSlice - 1) / kMaxSlice);
+  const int64_t slices = slice_count(ctx, processed, nt, pack16);
   const int64_t chunk = (processed + slices - 1) / slices;
   HistArgs a;
   a.fields = d_fields;
@@ -475,6 +564,7 @@ int hist_launch(iso_ctx *ctx, const float *d_fields, int n, int64_t F, int H, in
   a.maxs = d_maxs;
   a.ghist = b.ghist;
   a.arrive = b.arrive;
+  a.parts = b.parts;
   a.map = d_map;
   a.n = n;
   a.multi = multi;
@@ -492,6 +582,16 @@ int hist_launch(iso_ctx *ctx, const float *d_fields, int n, int64_t F, int H, in
   };
   if (pack16) variant == 0 ? launch(hist_nmi_kernel<true, 1>) : launch(hist_nmi_kernel<true, 2>);
   else variant == 0 ? launch(hist_nmi_kernel<false, 4>) : launch(hist_nmi_kernel<false, 8>);
+  if (a.parts && slices > 1) {
+    const dim3 mg((unsigned)((H * kRowWords / 4 + 255) / 256), (unsigned)nt);
+    if (pack16) {
+      hipLaunchKernelGGL(merge_kernel<true>, mg, dim3(256), 0, ctx->stream, a);
+      hipLaunchKernelGGL(finish_kernel<true>, dim3((unsigned)nt), dim3(kBlock), lds, ctx->stream, a);
+    } else {
+      hipLaunchKernelGGL(merge_kernel<false>, mg, dim3(256), 0, ctx->stream, a);
+      hipLaunchKernelGGL(finish_kernel<false>, dim3((unsigned)nt), dim3(kBlock), lds, ctx->stream, a);
+    }
+  }
   ISO_HIP_CHECK(ctx, hipGetLastError());
   if (nmi32)
     hipLaunchKernelGGL(fold_kernel, dim3((unsigned)((nt + kFoldPairs - 1) / kFoldPairs)),

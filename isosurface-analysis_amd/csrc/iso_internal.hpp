@@ -19,6 +19,7 @@ enum iso_ws_slot {
   WS_HIST_GLOBAL = 0,  // per-task 32-bit joint histograms, zero at rest
   WS_HIST_ARRIVE,      // per-task slice arrival counters, zero at rest
   WS_HIST_TASKS,       // int2 task list
+  WS_HIST_PARTS,       // LDS histograms of the slices of cut-up pairs
   WS_INTERVAL_PART,    // partial min/max per block
   WS_MC_COUNTERS,      // extraction counters
   WS_MC_CORNER_TABLE,  // hash set of grid-point vertices, EMPTY at rest

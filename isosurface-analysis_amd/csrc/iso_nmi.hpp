@@ -650,13 +650,18 @@ int nmi_logs(iso_ctx *ctx, const float **out);
 int nmi_logs_fill(iso_ctx *ctx, float *d_logs);
 
 // Device buffers one launch of the histogram + NMI kernels works in: merged
-// 32-bit histograms and slice arrival counters per task (zero at rest) and,
-// for the reference-order NMI, the chains' inputs.
+// 32-bit histograms and slice arrival counters per task (zero at rest), the
+// slices' own histograms (hist_parts_bytes; null: they are added to the merged
+// ones) and, for the reference-order NMI, the chains' inputs.
 struct HistBufs {
   uint32_t *ghist = nullptr;
   uint32_t *arrive = nullptr;
+  uint32_t *parts = nullptr;
   ChainBufs chains;
 };
+
+// Bytes of HistBufs::parts for a launch over nt pairs (0: pairs are not cut up).
+size_t hist_parts_bytes(const iso_ctx *ctx, int64_t F, int H, uint32_t flags, int64_t nt);
 
 // One launch over tasks d_tasks[0, nt) with the caller's buffers; variant
 // 0 or 1 is the kernel shape (the autotuner's two candidates).

@@ -107,7 +107,7 @@ int iso_hist_nmi_noalloc(iso_ctx *ctx, const float *d_fields, int n, int64_t F, 
   ISO_TRY(scratch_of(ctx, &base));
   char *p = (char *)base;
   const bool nmi32 = (flags & ISO_COMPAT_NMI32) != 0;
-  // layout: logarithms | tasks | arrive | chains' inputs | histograms
+  // layout: logarithms | tasks | arrive | chains' inputs | histograms | slices'
   iso::HistBufs b;
   size_t off = 0;
   size_t per_task = sizeof(int2) + 4 + 4 * (size_t)H * H;
@@ -121,7 +121,9 @@ int iso_hist_nmi_noalloc(iso_ctx *ctx, const float *d_fields, int n, int64_t F, 
   if (off + kPad + per_task > kScratchBytes)
     return iso::fail(ctx, ISO_ERR_UNSUPPORTED, "iso_hist_nmi_noalloc: %d bins exceed the %zu-byte scratch",
                      H, kScratchBytes);
-  const int T = (int)std::min<size_t>((kScratchBytes - off - kPad) / per_task, 16384);
+  const int64_t ntasks = multi ? (int64_t)n * n : (int64_t)n * (n + 1) / 2;
+  const int T = (int)std::min<int64_t>(
+      ntasks, (int64_t)std::min<size_t>((kScratchBytes - off - kPad) / per_task, 16384));
   int2 *tasks = (int2 *)(p + off);
   off += align256(sizeof(int2) * (size_t)T);
   b.arrive = (uint32_t *)(p + off);
@@ -131,16 +133,20 @@ int iso_hist_nmi_noalloc(iso_ctx *ctx, const float *d_fields, int n, int64_t F, 
     off += align256(iso::chain_task_bytes(H, F) * (size_t)T + 512);
   }
   b.ghist = (uint32_t *)(p + off);
+  off += align256(4 * (size_t)T * H * H);
+  // the slices' histograms, where few pairs leave room for them
+  uint32_t *const parts = (uint32_t *)(p + off);
   // what the kernels expect zero at rest (a previous call may have ended
   // early)
   ISO_TRY(iso::fill_u32(ctx, b.arrive, 0u, (size_t)T));
   ISO_TRY(iso::fill_u32(ctx, b.ghist, 0u, (size_t)T * H * H));
-  const int64_t ntasks = multi ? (int64_t)n * n : (int64_t)n * (n + 1) / 2;
   for (int64_t t0 = 0; t0 < ntasks; t0 += T) {
     const int nt = (int)std::min<int64_t>(T, ntasks - t0);
     hipLaunchKernelGGL(pair_tasks_kernel, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0,
                        ctx->stream, n, multi, t0, nt, tasks);
     ISO_HIP_CHECK(ctx, hipGetLastError());
+    const size_t pb = iso::hist_parts_bytes(ctx, F, H, flags, nt);
+    b.parts = pb > 0 && off + pb <= kScratchBytes ? parts : nullptr;
     // the autotuner's default shape (no timing events here)
     ISO_TRY(iso::hist_launch(ctx, d_fields, n, F, H, multi, flags, d_mins, d_maxs, d_map, tasks, nt,
                              d_joint, d_rows, d_cols, b, 1));
