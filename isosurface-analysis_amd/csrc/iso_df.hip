@@ -1487,9 +1487,7 @@ int df_pool(iso_ctx *ctx, const void *d_xyz, bool is_int, int64_t ntot, const ui
     uint32_t *gseg = (uint32_t *)(gbox + 2 * G);
     int *gdelta = (int *)(gseg + G);
     int *la = (int *)lists;  // splits queued by phase 1
-    ISO_TRY(fill_u32(ctx, arr, 0u, (size_t)G));
-    ISO_TRY(fill_u32(ctx, roots, (uint32_t)kNoRoot, (size_t)nseg));
-    ISO_TRY(fill_u32(ctx, cnt, 0u, 16));
+    ISO_TRY(fill3_u32(ctx, arr, 0u, (size_t)G, roots, (uint32_t)kNoRoot, (size_t)nseg, cnt, 0u, 16));
     if (pool_leaves) {
       // keys in pool order, sort of the leaves, their new first points (a
       // scan of their sizes in sorted order), then the copy and the boxes

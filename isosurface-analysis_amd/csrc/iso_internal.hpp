@@ -124,6 +124,8 @@ int enter(iso_ctx *ctx);  // hipSetDevice(ctx->device) + clears last_error
 
 // Fills count 32-bit words with v using a kernel on the context's stream.
 int fill_u32(iso_ctx *ctx, void *p, uint32_t v, size_t count);
+int fill3_u32(iso_ctx *ctx, void *p0, uint32_t v0, size_t n0, void *p1, uint32_t v1, size_t n1,
+              void *p2, uint32_t v2, size_t n2);
 
 // Looks up this context's device address of the no-alloc entry point's
 // scratch array (once per device; see iso_noalloc.hip).

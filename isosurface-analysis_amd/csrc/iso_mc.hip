@@ -897,10 +897,8 @@ int mc_multi(iso_ctx *ctx, const float *d_vol, int gx, int gy, int gz, uint32_t 
     void *tab = nullptr, *ctr = nullptr, *pin = nullptr;
     ISO_TRY(ws_get(ctx, WS_MC_CORNER_TABLE, slots * 12, false, &tab));  // keys, then owners
     ISO_TRY(ws_get(ctx, WS_MC_COUNTERS, 64, false, &ctr));
-    ISO_TRY(fill_u32(ctx, tab, 0xffffffffu, slots * 2));
     // [overflow, vertex total, 64-bit vertex total, kMcOddVertices: of a sort to follow]
-    ISO_TRY(fill_u32(ctx, ctr, 0u, 5));
-    ISO_TRY(fill_u32(ctx, priv, 0u, (size_t)kMcPriv * k * 5));
+    ISO_TRY(fill3_u32(ctx, tab, 0xffffffffu, slots * 2, ctr, 0u, 5, priv, 0u, (size_t)kMcPriv * k * 5));
     a.corner_tab = (unsigned long long *)tab;
     a.corner_owner = (uint32_t *)(a.corner_tab + slots);
     a.corner_mask = (uint32_t)(slots - 1);
