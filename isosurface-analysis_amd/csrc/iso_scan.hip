@@ -220,17 +220,24 @@ __global__ __launch_bounds__(kSortBlock) void radix_scatter_kernel(
     const uint32_t *keys, const uint32_t *vals, int64_t n, int shift, const uint32_t *hist,
     int ntiles, uint32_t *keys_out, uint32_t *vals_out) {
   __shared__ uint32_t s_wcnt[kSortWaves][256];  // per wave: digit counts, then bases
-  __shared__ uint32_t s_all[4][256], s_before[4][256], s_sum[4];
+  // Whole tiles of several keys per digit are put in order in LDS and written
+  // out from there: a store of 64 keys then covers a few runs instead of 64
+  // lines, which the address unit takes one a cycle.
+  constexpr bool kStaged = ITEMS >= 4;
+  __shared__ uint32_t s_all[FEW ? 4 : 1][256], s_before[FEW ? 4 : 1][256], s_sum[4];
+  __shared__ uint32_t s_first[256], s_to[256], s_tile[4];
+  __shared__ uint32_t s_stage[kStaged ? kSortBlock * ITEMS : 1];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int64_t base = (int64_t)blockIdx.x * (kSortBlock * ITEMS) + w * (64 * ITEMS);
-  // the whole tile's keys and values are requested up front, so one memory
-  // latency is exposed per tile instead of one per round
+  // the whole tile's keys are requested up front (and its values before the
+  // keys go out), so one memory latency is exposed per tile instead of one per
+  // round
   uint32_t keyv[ITEMS], valv[ITEMS], rank[ITEMS];
 #pragma unroll
   for (int k = 0; k < ITEMS; ++k) {
     const int64_t i = base + k * 64 + lane;
     keyv[k] = i < n ? keys[i] : 0u;
-    valv[k] = i < n ? vals[i] : 0u;
+    if (!kStaged) valv[k] = i < n ? vals[i] : 0u;
   }
   if (FEW) {  // all counts of each digit, and those in the tiles before this one
     const int d = tid & 255, g = tid >> 8;
@@ -260,13 +267,13 @@ __global__ __launch_bounds__(kSortBlock) void radix_scatter_kernel(
     __builtin_amdgcn_wave_barrier();
   }
   __syncthreads();
+  uint32_t run = 0, mine = 0, all_inc = 0, tile_inc = 0;  // of digit tid
   if (tid < 256) {
-    uint32_t run;
     if (FEW) {
       const uint32_t all = s_all[0][tid] + s_all[1][tid] + s_all[2][tid] + s_all[3][tid];
-      const uint32_t inc = wave_incl_scan(all);
-      if (lane == 63) s_sum[w] = inc;
-      run = inc - all + s_before[0][tid] + s_before[1][tid] + s_before[2][tid] + s_before[3][tid];
+      all_inc = wave_incl_scan(all);
+      if (lane == 63) s_sum[w] = all_inc;
+      run = all_inc - all + s_before[0][tid] + s_before[1][tid] + s_before[2][tid] + s_before[3][tid];
     } else {
       run = hist[(int64_t)tid * ntiles + blockIdx.x];
     }
@@ -275,20 +282,68 @@ __global__ __launch_bounds__(kSortBlock) void radix_scatter_kernel(
     for (int q = 0; q < kSortWaves; ++q) c[q] = s_wcnt[q][tid];
 #pragma unroll
     for (int q = 0; q < kSortWaves; ++q) {
-      s_wcnt[q][tid] = run;
-      run += c[q];
+      s_wcnt[q][tid] = mine;
+      mine += c[q];
+    }
+    if (kStaged) {
+      tile_inc = wave_incl_scan(mine);
+      if (lane == 63) s_tile[w] = tile_inc;
     }
   }
   __syncthreads();
+  if (tid < 256) {
+    if (FEW)  // the digits of the waves before the digit's
+      for (int q = 0; q < w; ++q) run += s_sum[q];
+    uint32_t first = tile_inc - mine;  // the tile's keys of smaller digits
+    if (kStaged)
+      for (int q = 0; q < w; ++q) first += s_tile[q];
+    s_first[tid] = first;
+    s_to[tid] = run - first;
+  }
+  __syncthreads();
+  if (!kStaged) {
+#pragma unroll
+    for (int k = 0; k < ITEMS; ++k) {
+      if (base + k * 64 + lane >= n) break;
+      const uint32_t d = (keyv[k] >> shift) & 255u;
+      const uint32_t pos = s_first[d] + s_to[d] + s_wcnt[w][d] + rank[k];
+      keys_out[pos] = keyv[k];
+      vals_out[pos] = valv[k];
+    }
+    return;
+  }
+  // the tile in sorted order through LDS, keys then values
+  const int64_t tile0 = (int64_t)blockIdx.x * (kSortBlock * ITEMS);
+  const int count = (int)min(n - tile0, (int64_t)(kSortBlock * ITEMS));
 #pragma unroll
   for (int k = 0; k < ITEMS; ++k) {
-    if (base + k * 64 + lane >= n) break;
     const uint32_t d = (keyv[k] >> shift) & 255u;
-    uint32_t pos = s_wcnt[w][d] + rank[k];
-    if (FEW)  // the digits of the waves before the digit's
-      pos += (d >= 64 ? s_sum[0] : 0u) + (d >= 128 ? s_sum[1] : 0u) + (d >= 192 ? s_sum[2] : 0u);
-    keys_out[pos] = keyv[k];
-    vals_out[pos] = valv[k];
+    rank[k] += s_first[d] + s_wcnt[w][d];
+    if (base + k * 64 + lane < n) s_stage[rank[k]] = keyv[k];
+  }
+#pragma unroll
+  for (int k = 0; k < ITEMS; ++k)
+    valv[k] = base + k * 64 + lane < n ? vals[base + k * 64 + lane] : 0u;
+  __syncthreads();
+  uint32_t to[ITEMS];
+#pragma unroll
+  for (int k = 0; k < ITEMS; ++k) {
+    const int i = k * kSortBlock + tid;
+    if (i >= count) break;
+    const uint32_t key = s_stage[i];
+    to[k] = s_to[(key >> shift) & 255u] + i;
+    keys_out[to[k]] = key;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < ITEMS; ++k)
+    if (base + k * 64 + lane < n) s_stage[rank[k]] = valv[k];
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < ITEMS; ++k) {
+    const int i = k * kSortBlock + tid;
+    if (i >= count) break;
+    vals_out[to[k]] = s_stage[i];
   }
 }
 
