@@ -24,21 +24,23 @@
 //     both chain orders and a second kernel folds the chains of all pairs
 //     (iso_nmi.hpp); without it, the same quantity from the exact integer
 //     counts in double (sum c ln c), in the same kernel;
-//   - pairs come in tiles of 4 x 8 fields (12 fields for 32 pairs), and
-//     workgroup ids are remapped so that a tile's pairs run on one XCD at a time
-//     and share their fields in its L2 (row by row, 33 fields for 32 pairs, the
-//     launch read 13.6 GB past the L2s on the 600x248x248 front at 100
-//     isovalues, tiled 10.3 GB; those reads reach 7 TB/s, also where the
-//     256 MB cache holds them).
+//   - pairs come in tiles of 8 x 8 fields, each as two of 4 x 8, and workgroup
+//     ids are remapped so that an XCD runs the pairs of a tile (two workgroups
+//     per CU: 64 at a time, 16 fields) or half a tile (32, 12 fields) at a time,
+//     which share their fields in its L2 (row by row, 33 fields for 32 pairs,
+//     the launch read 13.6 GB past the L2s on the 600x248x248 front at 100
+//     isovalues, tiled 10 GB; those reads reach 7 TB/s, also where the 256 MB
+//     cache holds them).
 //
 // 600x248x248 front, 100 isovalues, 256 bins (5,050 pairs of 576,600 voxels):
 // 3.04 -> 2.0 ms + 0.09 ms for the chains.  The counting's floor is its vector
 // instructions, 11 per pair of values at 4 cycles per wave: 0.9 ms; on top come
 // the rare exact divisions, LDS conflicts between lanes that meet in a counter
 // (2.4e8 cycles over the CUs), the pairs' starts and the lists (0.3 ms), which
-// one workgroup per CU cannot hide.  128 bins (2,016 pairs of 2^20 voxels, two
-// workgroups per CU): 1.55 -> 1.3 ms, at 9.4 GB past the L2s bound by those
-// reads; 256 isovalues of 60,000 voxels (32,896 pairs): 4.9 -> 2.1 ms.
+// one workgroup per CU cannot hide.  128 bins (2,080 pairs of 2^20 voxels, two
+// workgroups per CU): 1.55 -> 1.12 ms (in 4 x 8 tiles alone 1.35); 256 bins,
+// 2,016 pairs of 128^3 fields: 5.6 -> 3.4 ms; 256 isovalues of 60,000 voxels
+// (32,896 pairs): 4.9 -> 2.1 ms.
 #include "iso_internal.hpp"
 #include "iso_bins.hpp"
 #include "iso_nmi.hpp"
@@ -54,8 +56,8 @@ namespace {
 
 constexpr int kBlock = iso::kHistBlock;
 constexpr int kWaves = kBlock / 64;
-// Pairs of a tile of the pair matrix (4 x 8), which is also the workgroups of
-// 16-bit counters that an XCD runs at once (one per CU, 32 CUs).
+// Pairs of half a tile of the pair matrix (4 x 8), which is also the workgroups
+// of 16-bit counters that an XCD runs at once (one per CU, 32 CUs).
 constexpr int kTileRows = 4, kTileCols = 8, kTilePairs = kTileRows * kTileCols;
 constexpr int kMaxTasksPerLaunch = 16384;  // one launch per 128-isovalue ISM (no tail wave)
 constexpr size_t kMaxPartBytes = (size_t)128 << 20;  // slices' histograms of a launch
@@ -600,14 +602,16 @@ int hist_launch(iso_ctx *ctx, const float *d_fields, int n, int64_t F, int H, in
   return ISO_OK;
 }
 
-// Unordered pairs (i <= j), or all n*n pairs (i, n + j) for multi, in tiles.
+// Unordered pairs (i <= j), or all n*n pairs (i, n + j) for multi, in tiles of 8
+// x 8, the upper four rows first.
 void build_tasks(int n, int multi, std::vector<int2> &t) {
   t.clear();
-  for (int i0 = 0; i0 < n; i0 += kTileRows)
+  for (int i0 = 0; i0 < n; i0 += 2 * kTileRows)
     for (int j0 = multi ? 0 : i0; j0 < n; j0 += kTileCols)
-      for (int i = i0; i < std::min(i0 + kTileRows, n); ++i)
-        for (int j = multi ? j0 : std::max(i, j0); j < std::min(j0 + kTileCols, n); ++j)
-          t.push_back(make_int2(i, multi ? n + j : j));
+      for (int h = i0; h < std::min(i0 + 2 * kTileRows, n); h += kTileRows)
+        for (int i = h; i < std::min(h + kTileRows, n); ++i)
+          for (int j = multi ? j0 : std::max(i, j0); j < std::min(j0 + kTileCols, n); ++j)
+            t.push_back(make_int2(i, multi ? n + j : j));
 }
 
 }  // namespace iso
