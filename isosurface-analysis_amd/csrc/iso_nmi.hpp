@@ -378,8 +378,8 @@ __device__ __attribute__((always_inline)) void emit_chains(uint32_t *s_hist, int
 // ---- the chains -------------------------------------------------------------
 constexpr int kFoldPairs = 2;                // pairs of a workgroup
 constexpr int kFoldChains = 4 * kFoldPairs;  // (i, j), (j, i), columns, rows of each
-constexpr int kFoldBlock = 256;              // terms of a chain per step
-constexpr int kFoldWaves = 3;                // the first folds, the others lay terms out
+constexpr int kFoldBlock = 128;              // terms of a chain per step
+constexpr int kFoldWaves = 5;                // the first folds, the others lay terms out
 // terms of a chain's row in LDS, padded so that the chains' 16-byte reads meet
 // different banks
 constexpr int kFoldRow = kFoldBlock + 2;
@@ -395,20 +395,23 @@ struct FoldOut {
   float *ij, *ji;
 };
 
-// The NMI of pair tasks t0 and t0 + 1 (below ntasks), by a workgroup of 3 waves.
+// The NMI of pair tasks t0 and t0 + 1 (below ntasks), by a workgroup of 5 waves.
 // out(t) gives task t's outputs.
 //
 // Chain c of the 8 is pair c / 4's (i, j), (j, i), column or row chain.  Lane c
-// of the first wave folds it, acc = fmaf(-c, logf(c), acc), in order, 256 terms
-// a step from one of two LDS buffers, while the other waves lay the next 256 of
-// every chain out in the other; their counts are read three steps ahead and
+// of the first wave folds it, acc = fmaf(-c, logf(c), acc), in order, 128 terms
+// a step from one of two LDS buffers, while each of the other waves lays the
+// next 128 of a list out in the other; their counts are read three steps ahead and
 // their logarithms looked up two steps ahead.  Past a chain's end the terms are
 // (0, 0), and fmaf(-0, 0, acc) is acc exactly.
 //
-// The fold is a chain of dependent multiply-adds (about 1.2 us a step); by one
+// The fold is a chain of dependent multiply-adds (about 0.6 us a step); by one
 // wave alone, the counts, look-ups and stores between its folds took twice as
-// long again (600x248x248 front, up to 9,400 terms: 140 us for 5,050 pairs, 3.3
-// us a step).
+// long again.  Six such workgroups fit a CU; 256 terms a step and two waves for
+// the four lists fit four, and two waves keep up with neither: 5,050 pairs of
+// the 600x248x248 front (up to 9,400 terms) 90 -> 71 us, 32,896 pairs of 60,000
+// voxels 741 -> 594, 2,016 of 128^3 fields 258 -> 247 (128 terms and two waves
+// 98, 590, 410).
 template <class Out>
 __device__ __attribute__((always_inline)) void fold_chains(const ChainBufs &b, int H, int64_t t0,
                                                            int64_t ntasks, Out out, FoldLds &s) {
@@ -430,10 +433,9 @@ __device__ __attribute__((always_inline)) void fold_chains(const ChainBufs &b, i
     for (int q = 0; q < steps; ++q) {
       __syncthreads();
       if (lane < kFoldChains) {
-        // 16 terms at a time, the next 16 on their way: a read's latency is
-        // about that of 16 dependent multiply-adds
+        // 8 terms at a time, the next 8 on their way
         const float4 *row = reinterpret_cast<const float4 *>(s.terms[q & 1][lane]);
-        constexpr int kQ = 8;
+        constexpr int kQ = kFoldBlock / 32;
         float4 r0[kQ], r1[kQ];
         auto get = [&](float4(&r)[kQ], int k) {
 #pragma unroll
@@ -494,40 +496,49 @@ __device__ __attribute__((always_inline)) void fold_chains(const ChainBufs &b, i
     wide[u] = __builtin_amdgcn_readfirstlane((int)b.head[t].y) != 0;
     src[u] = b.lists + (2 * (size_t)t + (lc & 1)) * b.list_bytes;
   }
+  constexpr int kPer = kFoldBlock / 64;  // terms of a chain a lane lays out per step
+  static_assert(kPer == 2 || kPer == 4, "a load takes 2 or 4 counts");
   struct Counts {
-    uint32_t v[kOwn][4];
+    uint32_t v[kOwn][kPer];
   };
-  // this lane's counts of step q: entries k .. k + 3 of each chain, k = 256 q +
-  // 4 lane, 0 past the chain's end (a list's room is whole 16-byte pieces, so
-  // the four of its last entry can be read)
+  // this lane's counts of step q: entries k .. k + kPer - 1 of each chain, k =
+  // kFoldBlock q + kPer lane, 0 past the chain's end (a list's room is whole 16-byte
+  // pieces, so those of its last entry can be read)
   auto load = [&](Counts &n, int q) {
 #pragma unroll
     for (int u = 0; u < kOwn; ++u) {
 #pragma unroll
-      for (int c = 0; c < 4; ++c) n.v[u][c] = 0u;
+      for (int c = 0; c < kPer; ++c) n.v[u][c] = 0u;
       if (q * kFoldBlock < len[u]) {
-        const int k = q * kFoldBlock + 4 * lane, i = k < len[u] ? k : 0;
-        uint32_t x[4];
+        const int k = q * kFoldBlock + kPer * lane, i = k < len[u] ? k : 0;
+        uint32_t x[kPer];
+        struct alignas(4 * kPer) Wide { uint32_t v[kPer]; };
+        struct alignas(2 * kPer) Narrow { uint32_t v[kPer / 2]; };
         if (wide[u]) {
-          const uint4 y = reinterpret_cast<const uint4 *>(src[u])[i >> 2];
-          x[0] = y.x; x[1] = y.y; x[2] = y.z; x[3] = y.w;
+          const Wide y = reinterpret_cast<const Wide *>(src[u])[i / kPer];
+#pragma unroll
+          for (int c = 0; c < kPer; ++c) x[c] = y.v[c];
         } else {
-          const uint2 y = reinterpret_cast<const uint2 *>(src[u])[i >> 2];
-          x[0] = y.x & 0xffffu; x[1] = y.x >> 16; x[2] = y.y & 0xffffu; x[3] = y.y >> 16;
+          const Narrow y = reinterpret_cast<const Narrow *>(src[u])[i / kPer];
+#pragma unroll
+          for (int c = 0; c < kPer; c += 2) {
+            x[c] = y.v[c / 2] & 0xffffu;
+            x[c + 1] = y.v[c / 2] >> 16;
+          }
         }
 #pragma unroll
-        for (int c = 0; c < 4; ++c) n.v[u][c] = k + c < len[u] ? x[c] : 0u;
+        for (int c = 0; c < kPer; ++c) n.v[u][c] = k + c < len[u] ? x[c] : 0u;
       }
     }
   };
   struct Logs {
-    float t[kOwn][4];
+    float t[kOwn][kPer];
   };
   auto look_up = [&](const Counts &n, Logs &g, int q) {
 #pragma unroll
     for (int u = 0; u < kOwn; ++u)
 #pragma unroll
-      for (int c = 0; c < 4; ++c)
+      for (int c = 0; c < kPer; ++c)
         g.t[u][c] = q * kFoldBlock < len[u] ? b.logs[min(n.v[u][c], (uint32_t)kLogs - 1u)] : 0.0f;
   };
   // rows past their chain's end are zeroed in both buffers and left
@@ -538,12 +549,13 @@ __device__ __attribute__((always_inline)) void fold_chains(const ChainBufs &b, i
       if (lc >= kLists || (q - 2) * kFoldBlock >= len[u]) continue;
       if (wide[u]) {  // counts past the table
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
+        for (int c = 0; c < kPer; ++c)
           if (n.v[u][c] >= (uint32_t)kLogs) g.t[u][c] = logf_cr((float)n.v[u][c]);
       }
-      float4 *row = reinterpret_cast<float4 *>(&s.terms[q & 1][4 * (lc >> 1) + (lc & 1)][4 * lane]);
-      row[0] = make_float4((float)n.v[u][0], g.t[u][0], (float)n.v[u][1], g.t[u][1]);
-      row[1] = make_float4((float)n.v[u][2], g.t[u][2], (float)n.v[u][3], g.t[u][3]);
+      float4 *row = reinterpret_cast<float4 *>(&s.terms[q & 1][4 * (lc >> 1) + (lc & 1)][kPer * lane]);
+#pragma unroll
+      for (int c = 0; c < kPer; c += 2)
+        row[c / 2] = make_float4((float)n.v[u][c], g.t[u][c], (float)n.v[u][c + 1], g.t[u][c + 1]);
     }
   };
   auto log_of = [&](uint32_t v) -> float {
@@ -551,19 +563,20 @@ __device__ __attribute__((always_inline)) void fold_chains(const ChainBufs &b, i
     if (v >= (uint32_t)kLogs) t = logf_cr((float)v);
     return t;
   };
-  // the marginals: one step (H <= 256), then zeros in both buffers
+  // the marginals: kMarg steps (H <= 256), then zeros in both buffers
+  constexpr int kMarg = 256 / kFoldBlock;
   auto put_marginals = [&](int q) {
 #pragma unroll
     for (int u = 0; u < kOwn; ++u) {
       const int lc = w - 1 + u * (kFoldWaves - 1);
       if (lc >= kLists) continue;
-      const int n = q == 0 ? length(lc >> 1, 2 + (lc & 1)) : 0;
+      const int n = q < kMarg ? length(lc >> 1, 2 + (lc & 1)) : 0;
       const uint32_t *m = b.marg + (2 * (t0 + (n ? lc >> 1 : 0)) + (lc & 1)) * H;
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const int k = 64 * c + lane;
+      for (int c = 0; c < kPer; ++c) {
+        const int i = 64 * c + lane, k = q * kFoldBlock + i;
         const uint32_t v = k < n ? m[k] : 0u;
-        s.terms[q & 1][4 * (lc >> 1) + 2 + (lc & 1)][k] = make_float2((float)v, k < n ? log_of(v) : 0.0f);
+        s.terms[q & 1][4 * (lc >> 1) + 2 + (lc & 1)][i] = make_float2((float)v, k < n ? log_of(v) : 0.0f);
       }
     }
   };
@@ -583,7 +596,7 @@ __device__ __attribute__((always_inline)) void fold_chains(const ChainBufs &b, i
       load(n3, q + 3);
       look_up(n2, g2, q + 2);
       put(n1, g1, q + 1);
-      if (q < 2) put_marginals(q + 1);
+      if (q < kMarg + 1) put_marginals(q + 1);
       n1 = n2;
       g1 = g2;
       n2 = n3;
