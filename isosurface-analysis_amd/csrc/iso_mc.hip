@@ -655,9 +655,13 @@ __global__ __launch_bounds__(kApBlock) void approx_emit_kernel(ApArgs a) {
 }
 
 // Many isovalues per pass (unordered pool output, for the pipeline): lane =
-// cell of a 4 x 4 x 16 brick (z fastest), block-culled loop over the
-// isovalues strictly inside the block's [min, max] in rounds of 32: pass 1
-// counts per wave, one pool reservation per block and round, pass 2 writes.
+// cell of a 4 x 4 x 16 brick (z fastest), whose samples are staged in LDS once
+// (425 for 256 cells), block-culled loop over the isovalues strictly inside the
+// block's [min, max] in rounds of 32: pass 1 counts per wave, one pool
+// reservation per block and round, pass 2 writes.  Bound by its vector
+// instructions and the volume's one reading: 256 isovalues of a
+// 200x160x120 volume 640 -> 121 us (eight loads per cell, and one lane that laid
+// out a round's 128 places and counted each isovalue, before).
 struct ApMultiArgs {
   const float *img;
   int X, Y, Z;
@@ -675,91 +679,103 @@ constexpr int kApWaves = kApBlock / 64;
 constexpr int kApRound = 32;
 
 __global__ __launch_bounds__(kApBlock) void approx_multi_kernel(ApMultiArgs a) {
+  __shared__ float s_v[kMcF * kMcM * kMcM];  // the block's samples, one more per axis
   __shared__ float s_lo[kApWaves], s_hi[kApWaves];
-  __shared__ int s_range[2];
   __shared__ uint32_t s_wt[kApRound][kApWaves], s_off[kApRound][kApWaves];
   __shared__ unsigned long long s_base;
-  __shared__ int s_any;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  __shared__ uint32_t s_run;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int Xc = a.X - 1, Yc = a.Y - 1, Zc = a.Z - 1;
-  int x, y, z;
-  {
-    const int nbz = (Zc + 15) >> 4, nby = (Yc + 3) >> 2;
-    const int64_t b = blockIdx.x;
-    z = (int)(b % nbz) * 16 + (tid & 15);
-    y = (int)((b / nbz) % nby) * 4 + ((tid >> 4) & 3);
-    x = (int)(b / ((int64_t)nbz * nby)) * 4 + (tid >> 6);
-  }
-  const bool live = x < Xc && y < Yc && z < Zc;
-  if (!live) { x = 0; y = 0; z = 0; }
+  const uint32_t nbz = (uint32_t)(Zc + 15) >> 4, nby = (uint32_t)(Yc + 3) >> 2, b = blockIdx.x;
+  const int z0 = (int)(b % nbz) * 16, y0 = (int)(b / nbz % nby) * 4, x0 = (int)(b / nbz / nby) * 4;
   const int64_t YZ = (int64_t)a.Y * a.Z;
-  const float *p = a.img + (x * YZ + (int64_t)y * a.Z + z);
+  for (uint32_t i = tid; i < kMcF * kMcM * kMcM; i += kApBlock) {
+    const uint32_t row = (i * 241u) >> 12, f = i - row * kMcF;     // i / 17 below 425
+    const uint32_t m2 = (row * 205u) >> 10, m1 = row - m2 * kMcM;  // row / 5 below 25
+    const int x = min(x0 + (int)m2, a.X - 1), y = min(y0 + (int)m1, a.Y - 1);
+    s_v[i] = a.img[x * YZ + (int64_t)y * a.Z + min(z0 + (int)f, a.Z - 1)];
+  }
+  __syncthreads();
+  const int lf = lane & 15, l1 = lane >> 4;
+  const int x = x0 + w, y = y0 + l1, z = z0 + lf;
   float lo = 3.4e38f, hi = -3.4e38f;
-  if (live) {
-    const float c[8] = {p[0], p[1], p[a.Z], p[a.Z + 1], p[YZ], p[YZ + 1], p[YZ + a.Z], p[YZ + a.Z + 1]};
+  if (x < Xc && y < Yc && z < Zc) {
+    const float *p = s_v + lf + kMcF * l1 + kMcF * kMcM * w;
+    constexpr int dy = kMcF, dx = kMcF * kMcM;
+    const float c[8] = {p[0], p[1], p[dy], p[dy + 1], p[dx], p[dx + 1], p[dx + dy], p[dx + dy + 1]};
 #pragma unroll
     for (int q = 0; q < 8; ++q) { lo = fminf(lo, c[q]); hi = fmaxf(hi, c[q]); }
   }
-  float blo = lo, bhi = hi;
-#pragma unroll
-  for (int s = 32; s > 0; s >>= 1) {
-    blo = fminf(blo, __shfl_xor(blo, s, 64));
-    bhi = fmaxf(bhi, __shfl_xor(bhi, s, 64));
+  {
+    float wlo = lo, whi = hi;
+    wave_minmax(wlo, whi);
+    if (lane == 0) { s_lo[w] = wlo; s_hi[w] = whi; }
   }
-  if (lane == 0) { s_lo[w] = blo; s_hi[w] = bhi; }
   __syncthreads();
-  if (tid == 0) {
+  int j0 = 0, j1 = 0;  // the isovalues strictly inside the block's range
+  {
     float L = s_lo[0], Hh = s_hi[0];
+#pragma unroll
     for (int q = 1; q < kApWaves; ++q) { L = fminf(L, s_lo[q]); Hh = fmaxf(Hh, s_hi[q]); }
-    int b0 = 0, e0 = a.k;  // first iso > L
-    while (b0 < e0) { int m = (b0 + e0) >> 1; if (a.isos[m] > L) e0 = m; else b0 = m + 1; }
-    int b1 = b0, e1 = a.k;  // first iso >= Hh
-    while (b1 < e1) { int m = (b1 + e1) >> 1; if (a.isos[m] >= Hh) e1 = m; else b1 = m + 1; }
-    s_range[0] = b0;
-    s_range[1] = L < Hh ? b1 : b0;
+    for (int i = lane; __ballot(i < a.k); i += 64) {
+      const float v = i < a.k ? a.isos[i] : 0.0f;
+      j0 += __popcll(__ballot(i < a.k && !(v > L)));
+      j1 += __popcll(__ballot(i < a.k && !(v >= Hh)));
+    }
+    if (!(L < Hh)) j1 = j0;
   }
-  __syncthreads();
-  const int j0 = s_range[0], j1 = s_range[1];
-  const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
   for (int jc = j0; jc < j1; jc += kApRound) {
     const int jn = min(kApRound, j1 - jc);
+    // lane u holds isovalue u of the round and the wave's cells it passes through
+    const float iso_u = lane < jn ? a.isos[jc + lane] : 0.0f;
+    const int slot_u = lane < jn ? a.slot[jc + lane] : 0;
+    uint32_t count_u = 0;
     for (int u = 0; u < jn; ++u) {
-      const float iso = a.isos[jc + u];
-      const uint64_t m = __ballot(lo < iso && iso < hi);  // a corner below and one above
-      if (lane == 0) s_wt[u][w] = (uint32_t)__popcll(m);
+      const float iso = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(iso_u), u));
+      const uint64_t m = __ballot(lo < iso) & __ballot(iso < hi);  // a corner below, one above
+      if (m) count_u = lane == u ? (uint32_t)__popcll(m) : count_u;
     }
+    if (lane < jn) s_wt[lane][w] = count_u;
     __syncthreads();
-    if (tid == 0) {
-      uint32_t run = 0;
-      for (int u = 0; u < jn; ++u) {
-        uint32_t vj = 0;
+    if (w == 0) {
+      uint32_t c[kApWaves] = {}, all = 0, sum;
+      if (lane < jn)
+#pragma unroll
+        for (int q = 0; q < kApWaves; ++q) all += c[q] = s_wt[lane][q];
+      uint32_t off = prefix32(all, sum);
+      if (lane < jn) {
+#pragma unroll
         for (int q = 0; q < kApWaves; ++q) {
-          s_off[u][q] = run + vj;
-          vj += s_wt[u][q];
+          s_off[lane][q] = off;
+          off += c[q];
         }
-        run += vj;
-        if (vj) atomicAdd(&a.counts[a.slot[jc + u]], vj);
+        if (all) atomicAdd(&a.counts[slot_u], all);
       }
-      s_base = run ? atomicAdd(a.pool_count, (unsigned long long)run) : 0ull;
-      s_any = run != 0;
+      if (lane == 0) {
+        s_base = sum ? atomicAdd(a.pool_count, (unsigned long long)sum) : 0ull;
+        s_run = sum;
+      }
     }
     __syncthreads();
-    if (!s_any) continue;  // block-uniform
-    for (int u = 0; u < jn; ++u) {
-      const float iso = a.isos[jc + u];
-      const bool f = lo < iso && iso < hi;
-      const uint64_t m = __ballot(f);
-      if (f) {
-        const int64_t pos = (int64_t)s_base + s_off[u][w] + __popcll(m & lt);
-        if (pos < a.cap) {
-          int32_t *q = a.out + 3 * pos;
-          q[0] = x;
-          q[1] = y;
-          q[2] = z;
-          if (a.out_slot) a.out_slot[pos] = (uint32_t)a.slot[jc + u];
+    const int64_t base = (int64_t)s_base;
+    if (s_run != 0) {  // block-uniform
+      const uint32_t room = (uint32_t)min(max(a.cap - base, (int64_t)0), (int64_t)INT32_MAX);
+      int32_t *const out = a.out + 3 * base;
+      const uint32_t off_u = lane < jn ? s_off[lane][w] : 0u;
+      for (uint64_t todo = __ballot(count_u != 0u); todo; todo &= todo - 1) {
+        const int u = __ffsll((unsigned long long)todo) - 1;
+        const float iso = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(iso_u), u));
+        const uint64_t m = __ballot(lo < iso) & __ballot(iso < hi);
+        const uint32_t pos = (uint32_t)__builtin_amdgcn_readlane((int)off_u, u) + lane_prefix(m);
+        if (__builtin_amdgcn_inverse_ballot_w64(m) && pos < room) {
+          *(int3 *)(out + 3u * pos) = make_int3(x, y, z);
+          if (a.out_slot)
+            a.out_slot[base + pos] = (uint32_t)__builtin_amdgcn_readlane(slot_u, u);
         }
       }
     }
+    __syncthreads();  // s_base and s_run are written again by the next round
   }
 }
 

@@ -62,3 +62,23 @@ def test_many_isovalues(ctx, dims, kind, k):
         want = oracle.df_brute(oracle.normalize(pts, dims), dims, 1)
         assert np.array_equal(got[list(ids).index(i)].ravel(), want.ravel()), i
     assert st.total_points == total
+
+
+@pytest.mark.parametrize("dims", [(2, 2, 2), (17, 5, 33), (9, 18, 6)])
+@pytest.mark.parametrize("kind", ["noise", "levels"])
+@pytest.mark.parametrize("k", [3, 33, 70])
+def test_many_isovalues_of_the_approximation(ctx, dims, kind, k):
+    v = _volume(kind, dims)
+    isos = np.linspace(0.02, 0.98, k).astype(np.float32)
+    isos[k // 2] = 0.5
+    _, ids, st, fields = ctx.ism_volume(ctx.to_device(v), dims, isos, isoamd.EXTRACT_APPROX, 1, 32,
+                                        isoamd.DF_LBVH, want_fields=True)
+    got, total = fields.numpy(), 0
+    for i, iso in enumerate(isos):
+        cells = oracle.approx(v, iso)
+        total += cells.shape[0]
+        assert (i in list(ids)) == (cells.shape[0] > 0)
+        if cells.shape[0]:
+            want = oracle.df_brute(oracle.normalize(cells, dims), dims, 1)
+            assert np.array_equal(got[list(ids).index(i)].ravel(), want.ravel()), i
+    assert st.total_points == total
