@@ -29,7 +29,7 @@
 //     per CU: 64 at a time, 16 fields) or half a tile (32, 12 fields) at a time,
 //     which share their fields in its L2 (row by row, 33 fields for 32 pairs,
 //     the launch read 13.6 GB past the L2s on the 600x248x248 front at 100
-//     isovalues, tiled 10 GB; those reads reach 7 TB/s, also where the 256 MB
+//     isovalues, tiled 7.4 GB; those reads reach 7 TB/s, also where the 256 MB
 //     cache holds them).
 //
 // 600x248x248 front, 100 isovalues, 256 bins (5,050 pairs of 576,600 voxels):
