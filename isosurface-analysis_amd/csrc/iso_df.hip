@@ -958,7 +958,8 @@ constexpr int kTrWaves = kTrBlock / 64;
 // half and quarter columns then come from one shared counter.  With chunk == 0
 // (few bricks) wave i takes bricks i, i + waves, ... and touches no counter.
 // A brick is 4 x 4 x 4*SPL samples: lane (x, y, z) holds samples
-// (x, y, z + 4s), s < SPL.  A wave walks the tree once per brick.  A child is
+// (x, y, z + 4s), s < SPL (or 4 x 4 x zext, zext < 4, for SPL 1 over few bricks:
+// the lanes past zext hold none).  A wave walks the tree once per brick.  A child is
 // entered if any sample's box bound beats that sample's best.  A leaf child
 // (at most BUCKET points) is scanned on the spot, before the internal sibling
 // is tested, so its points tighten that test.
@@ -985,7 +986,8 @@ __global__ __launch_bounds__(kTrBlock) __attribute__((amdgpu_waves_per_eu(SPL >=
                                                             const int *__restrict__ root_of,
                                                             const int *__restrict__ ne_set,
                                                             const int *__restrict__ order, int S,
-                                                            int bx, int by, int bz, int64_t F,
+                                                            int bx, int by, int bz, int zext,
+                                                            int64_t F,
                                                             uint32_t chunk, uint32_t nbig,
                                                             uint32_t nhalf, uint32_t small,
                                                             uint32_t slots, uint32_t group,
@@ -1041,8 +1043,8 @@ __global__ __launch_bounds__(kTrBlock) __attribute__((amdgpu_waves_per_eu(SPL >=
     float sx, sy, sz[SPL], best[SPL];
 #pragma unroll
     for (int q = 0; q < SPL; ++q) {
-      zs[q] = bzi * 4 * SPL + 4 * q + (lane & 3);
-      valid[q] = xs < g.nx && ys < g.ny && zs[q] < g.nz;
+      zs[q] = bzi * zext + 4 * q + (lane & 3);
+      valid[q] = xs < g.nx && ys < g.ny && zs[q] < g.nz && (lane & 3) < zext;
       sample_coords(g, xs, ys, zs[q], sx, sy, sz[q]);
       best[q] = valid[q] ? INFINITY : -1.0f;  // invalid samples never ask for a node
     }
@@ -1054,7 +1056,7 @@ __global__ __launch_bounds__(kTrBlock) __attribute__((amdgpu_waves_per_eu(SPL >=
     // the float d2 of P) it is an upper bound of the float minimum the walk
     // computes, so the walk still finds that minimum (a box or point is
     // skipped only when it cannot go below the bound) and only prunes sooner.
-    if (t == prev_t + 1u && bzi != 0) {
+    if (t == prev_t + 1u && bzi != 0 && zext == 4 * SPL) {
       const float p = __shfl(prev_best[SPL - 1], (lane & ~3) | 3, 64);
       const int zp = bzi * 4 * SPL - 1;
       const float szp = (float)(zp * g.ds + g.ds / 2) / (float)g.Z;
@@ -1535,7 +1537,16 @@ int df_pool(iso_ctx *ctx, const void *d_xyz, bool is_int, int64_t ntot, const ui
                        (const int *)gfirst, (Node *)nodes, (int4 *)pend, (uint32_t *)arr,
                        (const int *)la, (const uint32_t *)cnt, (int *)roots);
     // bricks of 4 x 4 x 4*spl samples
-    const int bx = (g.nx + 3) / 4, by = (g.ny + 3) / 4, bz = (g.nz + 4 * spl - 1) / (4 * spl);
+    // Fewer samples along z where a wave per brick of 64 leaves the chip room: the
+    // brick that most leaves are near to decides the time, and its wave's turns
+    // go down with its samples.  Two layers up to 16,384 bricks, one up to 4,096,
+    // 32,768 or 16,384 waves (one isovalue of the 600x248x248 front: walk over
+    // 9,728 bricks 264 us, by two layers 208, by one 314; the call over 1,216
+    // bricks 432, 388, 341; 128^3 blobs, 512 bricks: 210, 193, 181).
+    const int bx = (g.nx + 3) / 4, by = (g.ny + 3) / 4;
+    const uint64_t full = (uint64_t)bx * by * ((g.nz + 3) / 4) * (uint64_t)S;
+    const int zext = spl > 1 || full > 16384 ? 4 * spl : full > 4096 ? 2 : 1;
+    const int bz = (g.nz + zext - 1) / zext;
     // With at least 4 bricks per wave that fits on the chip (8 per SIMD), waves
     // stay and pull chunks of about 1/16 of their share from cnt[2], rounded up
     // to whole columns of bz bricks (a chunk then starts a column, and every
@@ -1575,7 +1586,7 @@ int df_pool(iso_ctx *ctx, const void *d_xyz, bool is_int, int64_t ntot, const ui
       hipLaunchKernelGGL(kernel, tg, dim3(kTrBlock), 0, ctx->stream, g, (const Node *)nodes,
                          (const Pt *)sorted, d_off_ne, (const int *)roots, d_ne_set,
                          d_walk_order, S, bx,
-                         by, bz, F, chunk, nbig, nhalf, small, slots, group, cnt + 2, d_df);
+                         by, bz, zext, F, chunk, nbig, nhalf, small, slots, group, cnt + 2, d_df);
     };
     // the walk alone, timed on the context's stream when a caller asks
     if (ctx->walk_ev[0]) ISO_HIP_CHECK(ctx, hipEventRecord(ctx->walk_ev[0], ctx->stream));

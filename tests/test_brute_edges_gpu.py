@@ -18,3 +18,18 @@ def test_brute_block_edges(ctx, dims):
         got = ctx.df_points(ctx.to_device(pts), n, dims, 1, isoamd.DF_BRUTE).numpy()
         want = oracle.df_brute(oracle.normalize(pts, dims), dims, 1)
         assert np.array_equal(got.ravel(), want.ravel()), (dims, n)
+
+
+@pytest.mark.parametrize("dims", [(5, 3, 2), (9, 9, 9), (70, 66, 71), (130, 70, 129)])
+def test_tree_walk_over_few_bricks_equals_brute(ctx, dims):
+    # one, two and four layers of samples to a wave (at most 4,096 and 16,384
+    # bricks of 4 x 4 x 4, and more), ragged at the grid's ends
+    rng = np.random.default_rng(sum(dims))
+    n = 3000
+    pts = (rng.random((n, 3)) * np.array(dims)).astype(np.float32)
+    d = ctx.to_device(pts)
+    brute = ctx.df_points(d, n, dims, 1, isoamd.DF_BRUTE).numpy()
+    for _ in range(2):  # the variants' first call, then the kept one
+        tree = ctx.df_points(d, n, dims, 1, isoamd.DF_LBVH).numpy()
+        assert np.array_equal(tree, brute)
+    d.free()
