@@ -1547,16 +1547,19 @@ int df_pool(iso_ctx *ctx, const void *d_xyz, bool is_int, int64_t ntot, const ui
     const uint64_t full = (uint64_t)bx * by * ((g.nz + 3) / 4) * (uint64_t)S;
     const int zext = spl > 1 || full > 16384 ? 4 * spl : full > 4096 ? 2 : 1;
     const int bz = (g.nz + zext - 1) / zext;
-    // With at least 4 bricks per wave that fits on the chip (8 per SIMD), waves
+    // With at least 32 bricks per wave that fits on the chip (8 per SIMD), waves
     // stay and pull chunks of about 1/16 of their share from cnt[2], rounded up
     // to whole columns of bz bricks (a chunk then starts a column, and every
     // brick but a column's first starts from the bound of the brick below it).
-    // With fewer, a wave per brick: the bricks' costs differ by far more than a
-    // wave's start (16,384 bricks of 64^3 samples, 16 isovalues: walk 238 -> 205
-    // us against two bricks a wave; 9,728 of one isovalue: 292 -> 263).
+    // With fewer, a wave per brick, which the chip deals out as waves end: a
+    // column's bricks one after the other take longer than the bound saves (maps
+    // of 64^3 blobs, 16,384 bricks, two a wave against one: walk 238, 205 us;
+    // from 4 bricks a wave in columns against one each: 96^3, 16 isovalues 1,204,
+    // 776 us; 100^3, 24: 1,350, 958; 200^3 at ds 2, 48: 2,400, 1,768; and 262,144
+    // bricks of 256^3 at ds 2, 64 isovalues, walk 2,522 in columns, 2,568).
     const uint64_t total = (uint64_t)bx * by * bz * (uint64_t)S;
     const uint64_t max_waves = (uint64_t)ctx->cu_count * 32;
-    const uint64_t waves = total < 4 * max_waves ? total : max_waves;
+    const uint64_t waves = total < 32 * max_waves ? total : max_waves;
     uint32_t chunk = 0u, nbig = 0u, nhalf = 0u, small = 1u;
     if (total >= 4 * waves) {
       const uint64_t c = std::min<uint64_t>(256, std::max<uint64_t>(1, total / (waves * 16)));
