@@ -1461,7 +1461,8 @@ int df_pool(iso_ctx *ctx, const void *d_xyz, bool is_int, int64_t ntot, const ui
     pfirst = (int *)pf;
   }
 
-  auto run_variant = [&](int B, int spl, bool pool_leaves) -> int {
+  const uint64_t max_waves = (uint64_t)ctx->cu_count * 32;  // on the chip, 8 per SIMD
+  auto run_variant = [&](int B, int spl, bool pool_leaves, uint64_t stay) -> int {
     if (!pool_leaves && can_pool) ISO_TRY(prep_sorted());  // both paths tuned: part of the cost
     if (pool_leaves)
       hipLaunchKernelGGL(flat_bound_kernel, dim3((unsigned)((nbb + kBndSub - 1) / kBndSub)),
@@ -1547,21 +1548,17 @@ int df_pool(iso_ctx *ctx, const void *d_xyz, bool is_int, int64_t ntot, const ui
     const uint64_t full = (uint64_t)bx * by * ((g.nz + 3) / 4) * (uint64_t)S;
     const int zext = spl > 1 || full > 16384 ? 4 * spl : full > 4096 ? 2 : 1;
     const int bz = (g.nz + zext - 1) / zext;
-    // With at least 32 bricks per wave that fits on the chip (8 per SIMD), waves
-    // stay and pull chunks of about 1/16 of their share from cnt[2], rounded up
-    // to whole columns of bz bricks (a chunk then starts a column, and every
-    // brick but a column's first starts from the bound of the brick below it).
+    // With at least `stay` bricks per wave that fits on the chip, waves stay and
+    // pull chunks of about 1/16 of their share from cnt[2], rounded up to whole
+    // columns of bz bricks (a chunk then starts a column, and every brick but a
+    // column's first starts from the bound of the brick below it).
     // With fewer, a wave per brick, which the chip deals out as waves end: a
-    // column's bricks one after the other take longer than the bound saves (maps
-    // of 64^3 blobs, 16,384 bricks, two a wave against one: walk 238, 205 us;
-    // from 4 bricks a wave in columns against one each: 96^3, 16 isovalues 1,204,
-    // 776 us; 100^3, 24: 1,350, 958; 200^3 at ds 2, 48: 2,400, 1,768; and 262,144
-    // bricks of 256^3 at ds 2, 64 isovalues, walk 2,522 in columns, 2,568).
+    // column's bricks one after the other take longer than the bound saves (a map
+    // of 64^3 blobs, 16,384 bricks, two a wave against one: walk 238, 205 us).
     const uint64_t total = (uint64_t)bx * by * bz * (uint64_t)S;
-    const uint64_t max_waves = (uint64_t)ctx->cu_count * 32;
-    const uint64_t waves = total < 32 * max_waves ? total : max_waves;
+    const uint64_t waves = total < stay * max_waves ? total : max_waves;
     uint32_t chunk = 0u, nbig = 0u, nhalf = 0u, small = 1u;
-    if (total >= 4 * waves) {
+    if (total >= stay * max_waves) {
       const uint64_t c = std::min<uint64_t>(256, std::max<uint64_t>(1, total / (waves * 16)));
       chunk = (uint32_t)(((c + bz - 1) / bz) * bz);
       // the last waves x chunk / 2 bricks go out `small` (a quarter column)
@@ -1606,30 +1603,44 @@ int df_pool(iso_ctx *ctx, const void *d_xyz, bool is_int, int64_t ntot, const ui
     if (ctx->walk_ev[1]) ISO_HIP_CHECK(ctx, hipEventRecord(ctx->walk_ev[1], ctx->stream));
     return ISO_OK;
   };
+  // Waves stay from 4 bricks for each.  From there up to 32, one variant has a
+  // wave per brick all the same, with 4 samples per lane if that leaves enough
+  // bricks: which is faster hangs on the sets, not on their sizes (maps in
+  // columns, by brick, us: 96^3 blobs, 16 isovalues 1,204, 776; 100^3, 24: 1,350,
+  // 958; 200^3 at ds 2, 48: 2,400, 1,768; a 600x248x248 front at ds 4, 12: 2,055,
+  // 2,212; 50: 8,358, 10,250).  It takes the place of the leaves of 48 points.
+  const auto bricks = [&](int spl) {
+    return (uint64_t)((g.nx + 3) / 4) * ((g.ny + 3) / 4) * ((g.nz + 4 * spl - 1) / (4 * spl)) * S;
+  };
+  const int by_brick = bricks(2) < 4 * max_waves || bricks(4) >= 32 * max_waves ? 0
+                       : bricks(4) >= 4 * max_waves                              ? 4
+                                                                                : 2;
   // (B, samples per lane) per variant, picked by the autotuner; ISO_DF_LEAF=B
   // (8..64) forces B, with ISO_DF_SPL=1, 2 or 4 (default 1)
-  static const int kLeaf[4] = {64, 48, 64, 64};
-  static const int kSpl[4] = {4, 2, 2, 1};
+  const int leaf[4] = {64, by_brick ? 64 : 48, 64, 64};
+  const int lane[4] = {4, by_brick ? by_brick : 2, 2, 1};
   if (const char *e = std::getenv("ISO_DF_LEAF")) {  // read per call
     const int v = std::atoi(e);
     const char *q = std::getenv("ISO_DF_SPL");
     const int spl = q && (q[0] == '2' || q[0] == '4') ? q[0] - '0' : 1;
-    if (v >= 8 && v <= kMaxLeaf) return run_variant(v, spl, can_pool);
+    if (v >= 8 && v <= kMaxLeaf) return run_variant(v, spl, can_pool, 4);
   }
   // variants 0-3: leaves from the pool's runs; 4-7 (or 0-3 when the pool path
   // is out): leaves from the sorted points
   const bool both = can_pool && can_sort;
   const uint64_t key = ((uint64_t)(can_pool ? 1 + both : 0) << 32) |
                        ((uint64_t)ceil_log2((uint64_t)(ntot / S + 1)) << 16) |
-                       (uint64_t)ceil_log2((uint64_t)F);
-  const char *what = both ? "lbvh (leaves, leaf points, samples per lane) {runs 64,4|runs 48,2|"
-                            "runs 64,2|runs 64,1|sorted 64,4|sorted 48,2|sorted 64,2|sorted 64,1}"
+                       ((uint64_t)ceil_log2((uint64_t)F) << 3) | (uint64_t)by_brick;
+  const char *what = both ? "lbvh (leaves, leaf points, samples per lane) {runs 64,4|runs 48,2 or by "
+                            "brick|runs 64,2|runs 64,1|sorted 64,4|sorted 48,2 or by brick|"
+                            "sorted 64,2|sorted 64,1}"
                      : can_pool ? "lbvh (leaves from runs: leaf points, samples per lane) "
-                                  "{64,4|48,2|64,2|64,1}"
+                                  "{64,4|48,2 or by brick|64,2|64,1}"
                                 : "lbvh (leaves from sorted points: leaf points, samples per lane) "
-                                  "{64,4|48,2|64,2|64,1}";
+                                  "{64,4|48,2 or by brick|64,2|64,1}";
   return tune_pick(ctx, kTuneTraverse, key, both ? 8 : 4, 2, what, [&](int v) {
-    return run_variant(kLeaf[v & 3], kSpl[v & 3], can_pool && v < 4);
+    const bool brick = by_brick && (v & 3) == 1;
+    return run_variant(leaf[v & 3], lane[v & 3], can_pool && v < 4, brick ? 32 : 4);
   });
 }
 

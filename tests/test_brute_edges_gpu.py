@@ -33,3 +33,17 @@ def test_tree_walk_over_few_bricks_equals_brute(ctx, dims):
         tree = ctx.df_points(d, n, dims, 1, isoamd.DF_LBVH).numpy()
         assert np.array_equal(tree, brute)
     d.free()
+
+
+@pytest.mark.parametrize("dims", [(161, 160, 157), (162, 161, 165), (255, 258, 130)])
+def test_tree_walk_between_bricks_and_columns_equals_brute(ctx, dims):
+    # from 4 to 32 bricks per wave the tuner also times a wave per brick, with two
+    # and with four samples per lane; every variant runs in the first call
+    rng = np.random.default_rng(sum(dims))
+    n = 2000
+    pts = (rng.random((n, 3)) * np.array(dims)).astype(np.float32)
+    d = ctx.to_device(pts)
+    brute = ctx.df_points(d, n, dims, 1, isoamd.DF_BRUTE).numpy()
+    for _ in range(2):
+        assert np.array_equal(ctx.df_points(d, n, dims, 1, isoamd.DF_LBVH).numpy(), brute)
+    d.free()
