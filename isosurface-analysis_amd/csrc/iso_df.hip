@@ -1626,7 +1626,8 @@ int df_pool(iso_ctx *ctx, const void *d_xyz, bool is_int, int64_t ntot, const ui
     if (v >= 8 && v <= kMaxLeaf) return run_variant(v, spl, can_pool, 4);
   }
   // variants 0-3: leaves from the pool's runs; 4-7 (or 0-3 when the pool path
-  // is out): leaves from the sorted points
+  // is out): leaves from the sorted points.  The second variant's form is the
+  // key's least part, so that sizes decide which tuned key is the nearest.
   const bool both = can_pool && can_sort;
   const uint64_t key = ((uint64_t)(can_pool ? 1 + both : 0) << 32) |
                        ((uint64_t)ceil_log2((uint64_t)(ntot / S + 1)) << 16) |
