@@ -272,6 +272,7 @@ __global__ __launch_bounds__(kMcBlock) __attribute__((amdgpu_waves_per_eu(8, 8))
   __shared__ uint32_t s_queue[kMcWaves][kMcQueue];
   __shared__ uint8_t s_nv[256];
   __shared__ float s_lo[kMcWaves], s_hi[kMcWaves];
+  __shared__ uint32_t s_nan[kMcWaves];  // count pass: NaN samples
   // count pass, per (isovalue of the round, wave), of two rounds in turn:
   // vertices, active cells, case vertices; corrections to the vertices
   __shared__ uint32_t s_wt[2][kMcRound][kMcWaves], s_wa[2][kMcRound][kMcWaves];
@@ -302,6 +303,7 @@ __global__ __launch_bounds__(kMcBlock) __attribute__((amdgpu_waves_per_eu(8, 8))
   const int ex = a.zfast ? 4 : 16, ez = a.zfast ? 16 : 4;  // the brick's extent
   {
     float lo = 3.4e38f, hi = -3.4e38f;
+    bool nan = false;
     const uint32_t sm = (uint32_t)(a.zfast ? a.sx : a.sz), sy = (uint32_t)a.sy;
     const bool inside = px + (a.zfast ? kMcM : kMcF) <= a.gx && py + kMcM <= a.gy &&
                         pz + (a.zfast ? kMcF : kMcM) <= a.gz;
@@ -321,9 +323,15 @@ __global__ __launch_bounds__(kMcBlock) __attribute__((amdgpu_waves_per_eu(8, 8))
       s_v[i] = v;
       lo = fminf(lo, v);
       hi = fmaxf(hi, v);
+      if (!EMIT) nan |= v != v;
     }
     wave_minmax(lo, hi);
-    if (lane == 0) { s_lo[w] = lo; s_hi[w] = hi; }
+    const uint64_t nans = __ballot(nan);
+    if (lane == 0) {
+      s_lo[w] = lo;
+      s_hi[w] = hi;
+      if (!EMIT) s_nan[w] = nans != 0ull;
+    }
   }
   __syncthreads();
   int j0, j1;
@@ -373,7 +381,14 @@ __global__ __launch_bounds__(kMcBlock) __attribute__((amdgpu_waves_per_eu(8, 8))
   const uint32_t item_z = lane | 2u << 6 | 1u << 8;
   // the isovalues this wave's edges can cross
   int2 own = make_int2(j0, j1);
-  if (!EMIT && !STATS) {
+  // With NaN samples in the block, a wave looks at an isovalue if one of its
+  // cells has a corner below it and one at or above it, NaN corners aside, and
+  // then takes every edge whose ends compare differently, an edge to a NaN
+  // among them.  (Without NaN samples this is what the crossings give: an edge
+  // that crosses an isovalue is an edge of such a cell.)
+  const bool nans = !EMIT && (s_nan[0] | s_nan[1] | s_nan[2] | s_nan[3]) != 0u;
+  static_assert(kMcWaves == 4, "four flags");
+  if (!EMIT && !STATS && !nans) {
     float lo = fminf(fminf(v0, vx), fminf(vy, vz)), hi = fmaxf(fmaxf(v0, vx), fmaxf(vy, vz));
     wave_minmax(lo, hi);
     own = iso_range(a.isos, a.k, lo, hi);
@@ -405,6 +420,26 @@ __global__ __launch_bounds__(kMcBlock) __attribute__((amdgpu_waves_per_eu(8, 8))
     } else {
       const int u0 = max(own.x - jc, 0), u1 = min(own.y - jc, jn);
       todo = u1 > u0 ? (~0ull >> (64 - u1)) & (~0ull << u0) : 0ull;
+      if (nans) {
+        float lo = 3.4e38f, hi = -3.4e38f;
+        if (__builtin_amdgcn_inverse_ballot_w64(has_x | has_y | has_z)) {
+#pragma unroll
+          for (int q = 0; q < 8; ++q) {
+            const float v = s_v[at + (q & 1 ? dx : 0) + (q & 2 ? kMcF : 0) + (q & 4 ? dz : 0)];
+            lo = fminf(lo, v);
+            hi = fmaxf(hi, v);
+          }
+        }
+        uint64_t reached = 0ull;
+        for (uint64_t t = todo; t; t &= t - 1) {
+          const int u = __ffsll((unsigned long long)t) - 1;
+          const float iso = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(iso_u), u));
+          if (__ballot(lo < iso && iso <= hi)) reached |= 1ull << u;
+        }
+        if (STATS && lane < jn)
+          s_wa[round & 1][lane][w] = s_wv[round & 1][lane][w] = 0u;  // of those left out
+        todo = reached;
+      }
     }
     uint32_t head = 0, tail = 0, seq = 0;
     // works out the n crossings at the queue's head, one per lane
