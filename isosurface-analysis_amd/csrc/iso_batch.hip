@@ -232,7 +232,7 @@ int iso_ism_batch(iso_ctx *ctx, iso_ism_job *jobs, int njobs, int extractor, int
     std::vector<int> order(k);
     std::iota(order.begin(), order.end(), 0);
     std::stable_sort(order.begin(), order.end(),
-                     [&](int x, int y) { return jb.h_isos[x] < jb.h_isos[y]; });
+                     [&](int x, int y) { return iso::iso_before(jb.h_isos[x], jb.h_isos[y]); });
     const size_t blk = 4 * (size_t)k * 2 + 4 * (size_t)k + 16 * (size_t)k;
     void *dblk = nullptr, *hblk = nullptr;
     ISO_TRY(iso::ws_get(ctx, WS_PIPE_A, blk + 1024, false, &dblk));

@@ -137,6 +137,9 @@ inline int ceil_log2(uint64_t v) {
   return b;
 }
 
+// Order of isovalues: ascending, NaN (whose surface is empty) past all others.
+inline bool iso_before(float a, float b) { return a < b || (b != b && a == a); }
+
 enum iso_tune_kind { kTuneHist = 1, kTuneTraverse = 2 };
 
 // Autotuner.  run(v) enqueues variant v (0 <= v < ncand) of one launch on the

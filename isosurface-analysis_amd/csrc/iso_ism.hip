@@ -108,7 +108,9 @@ int iso_ism_volume(iso_ctx *ctx, const float *d_vol, int X, int Y, int Z, const 
   // ---- isovalues, ascending, with their caller slots
   std::vector<int> order(k);
   std::iota(order.begin(), order.end(), 0);
-  std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return h_isos[a] < h_isos[b]; });
+  std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
+    return iso::iso_before(h_isos[a], h_isos[b]);
+  });
   const size_t bb = IsmBlock::bytes(k);
   void *dblk = nullptr, *hblk = nullptr;
   ISO_TRY(iso::ws_get(ctx, WS_PIPE_A, bb, false, &dblk));

@@ -218,12 +218,13 @@ __device__ __forceinline__ void wave_minmax(float &lo, float &hi) {
 }
 
 // isovalues that values in [lo, hi] can cross, lo < iso <= hi: [first, second)
+// (a NaN, which nothing crosses, stands past all others and counts in neither)
 __device__ __forceinline__ int2 iso_range(const float *isos, int k, float lo, float hi) {
   int b0 = 0, b1 = 0;
   for (int i = threadIdx.x & 63; __ballot(i < k); i += 64) {
     const float v = i < k ? isos[i] : 0.0f;
-    b0 += __popcll(__ballot(i < k && !(v > lo)));
-    b1 += __popcll(__ballot(i < k && !(v > hi)));
+    b0 += __popcll(__ballot(i < k && v <= lo));
+    b1 += __popcll(__ballot(i < k && v <= hi));
   }
   return make_int2(b0, lo <= hi ? b1 : b0);
 }
@@ -755,8 +756,8 @@ __global__ __launch_bounds__(kApBlock) void approx_multi_kernel(ApMultiArgs a) {
     for (int q = 1; q < kApWaves; ++q) { L = fminf(L, s_lo[q]); Hh = fmaxf(Hh, s_hi[q]); }
     for (int i = lane; __ballot(i < a.k); i += 64) {
       const float v = i < a.k ? a.isos[i] : 0.0f;
-      j0 += __popcll(__ballot(i < a.k && !(v > L)));
-      j1 += __popcll(__ballot(i < a.k && !(v >= Hh)));
+      j0 += __popcll(__ballot(i < a.k && v <= L));
+      j1 += __popcll(__ballot(i < a.k && v < Hh));
     }
     if (!(L < Hh)) j1 = j0;
   }
