@@ -156,8 +156,6 @@ __global__ __launch_bounds__(kBBlock) __attribute__((amdgpu_waves_per_eu(PACK16 
         iso::emit_chains<PACK16, false>(s_hist, a.hist_bytes, nullptr, Hv, mirror, s.pair, a.chains,
                                         ti);
     } else {
-      iso::list_bins<PACK16>(s_hist, src, Hv, s.pair);
-      __syncthreads();
       const double v = iso::nmi64_pair<PACK16>(s_hist, src, Hv, t.F, s.pair, s.red);
       if (tid == 0) {
         float *map = a.maps[t.job];

@@ -165,8 +165,6 @@ __device__ __forceinline__ void finish_pair(const HistArgs &a, HistLds<PACK16> &
                                       task);
   } else {
     // ---- fused NMI from exact counts ----
-    iso::list_bins<PACK16>(s_hist, src, H, s.pair);
-    __syncthreads();
     const double v = iso::nmi64_pair<PACK16>(s_hist, src, H, a.F, s.pair, s.red);
     if (tid == 0) {
       const float out = (v != v) ? 0.0f : (float)v;

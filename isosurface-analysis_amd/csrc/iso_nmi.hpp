@@ -89,28 +89,29 @@ __device__ __forceinline__ uint32_t lanes_below(uint64_t m) {
 
 // LDS the NMI uses beside the histogram: nonzero bins per wave and column (then
 // those in the waves before), nonzero bins in the rows (columns) before, the
-// marginals and, for the double form, a list of nonzero bins (row << 8 | column).
+// marginals and, for the double form, a list of nonzero bins (row << 8 | column):
+// as many as fit one workgroup per CU (16-bit counters) or two.
 template <bool PACK16>
 struct PairLds {
   static constexpr int kH = PACK16 ? 256 : 128;    // most bins per axis
   static constexpr int kRows = kH / kHistWaves;    // rows of a wave
   static constexpr int kCols = kH / 64;            // columns of a lane
-  static constexpr int kBins = 3072;  // most listed bins, 3 per lane
+  static constexpr int kBins = PACK16 ? 10240 : 6144;  // most listed bins
   union {
     uint8_t colpre[kHistWaves][kH];
     uint16_t bins[kBins];
   };
   uint32_t rowbase[kH], colbase[kH];
   uint32_t rows[kH], cols[kH];
-  uint32_t nbins, big;
-  uint32_t wtot[8];
+  uint32_t big;
+  uint32_t wtot[kHistWaves];
 };
 
 // Clears the marginals and counters; a barrier comes before their use.
 template <bool PACK16>
 __device__ __forceinline__ void clear_pair_lds(PairLds<PACK16> &s) {
   if (threadIdx.x < PairLds<PACK16>::kH) s.rows[threadIdx.x] = s.cols[threadIdx.x] = 0u;
-  if (threadIdx.x == 0) s.nbins = s.big = 0u;
+  if (threadIdx.x == 0) s.big = 0u;
 }
 
 // The count of bin (i, j): from the LDS histogram or, when gh is not null, from
@@ -137,15 +138,16 @@ __device__ __forceinline__ uint32_t slot_count(uint2 v, int c) {
   return c == 0 ? v.x : v.y;
 }
 
-// Counts the nonzero bins of the LDS histogram (or of gh) and lists the first
-// kBins of them, in any order.  The caller's barrier comes after; the number is
-// then s.nbins.
+// Lists the nonzero bins of the LDS histogram (or of gh) if they are kBins at
+// most, and returns their number (uniform).  Their order hangs on the counts
+// alone: lane after lane, each its slots in turn.
 template <bool PACK16>
-__device__ __attribute__((always_inline)) void list_bins(const uint32_t *s_hist, const uint32_t *gh,
-                                                         int H, PairLds<PACK16> &s) {
+__device__ __attribute__((always_inline)) uint32_t list_bins(const uint32_t *s_hist,
+                                                             const uint32_t *gh, int H,
+                                                             PairLds<PACK16> &s) {
   using L = PairLds<PACK16>;
   constexpr int kPer = kSlotBins<PACK16>;
-  const int l = threadIdx.x & 63;
+  const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
   // kPer bits per slot of the lane: which of its bins are not zero
   uint64_t nz = 0ull;
 #pragma unroll
@@ -162,40 +164,49 @@ __device__ __attribute__((always_inline)) void list_bins(const uint32_t *s_hist,
       nz |= (uint64_t)(n != 0u) << (kPer * q + c);
     }
   }
+  // the lane's place in the wave's run, then the wave's in the list
   const uint32_t n = (uint32_t)__popcll(nz);
-  // the lane's place in the wave's run, the wave's in the list
   uint32_t incl = n;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
     const uint32_t t = __shfl_up(incl, o, 64);
     if (l >= o) incl += t;
   }
-  const uint32_t tot = __shfl(incl, 63, 64);
-  uint32_t base = 0u;
-  if (tot && l == 0) base = atomicAdd(&s.nbins, tot);
-  uint32_t at = __builtin_amdgcn_readfirstlane(base) + incl - n;
-  // a list that is full already serves nobody
-  if (__builtin_amdgcn_readfirstlane(base) + tot > (uint32_t)L::kBins) return;
+  if (l == 63) s.wtot[w] = incl;
+  __syncthreads();
+  uint32_t at = incl - n, all = 0u;
+#pragma unroll
+  for (int q = 0; q < kHistWaves; ++q) {
+    const uint32_t t = s.wtot[q];
+    at += q < w ? t : 0u;
+    all += t;
+  }
+  all = __builtin_amdgcn_readfirstlane(all);
+  if (all > (uint32_t)L::kBins) return all;
   while (nz) {
     const int b = __ffsll((unsigned long long)nz) - 1;
     nz &= nz - 1ull;
     const int k = (b / kPer) * kHistBlock + (int)threadIdx.x;
     s.bins[at++] = (uint16_t)((k >> 6) << 8 | ((k & 63) * kPer + b % kPer));
   }
+  __syncthreads();
+  return all;
 }
 
-// f(i, j, count) for every nonzero bin of a pair whose bins are not listed.
+// f(i, j, count) for every nonzero bin of a pair whose bins are not listed: bin i
+// H + j is lane (i H + j) % 1024's.
 template <bool PACK16, class F>
 __device__ __forceinline__ void each_bin(const uint32_t *s_hist, const uint32_t *gh, int H, F f) {
-  constexpr int kPer = kSlotBins<PACK16>;
-  for (int k = threadIdx.x; k < H * 64; k += kHistBlock) {
-#pragma unroll
-    for (int c = 0; c < kPer; ++c) {
-      const int j = (k & 63) * kPer + c;
-      if (j < H) {
-        const uint32_t v = pair_count<PACK16>(s_hist, gh, H, k >> 6, j);
-        if (v) f(k >> 6, j, v);
-      }
+  const int di = kHistBlock / H, dj = kHistBlock - di * H;
+  int i = (int)threadIdx.x / H, j = (int)threadIdx.x - i * H;
+  while (i < H) {
+    const uint32_t v = pair_count<PACK16>(s_hist, gh, H, i, j);
+    if (v) f(i, j, v);
+    i += di;
+    j += dj;
+    if (j >= H) {
+      j -= H;
+      ++i;
     }
   }
 }
@@ -612,6 +623,14 @@ __device__ __forceinline__ double wave_sum(double v) {
 
 // NMI of a pair in double from the exact counts (arguments as for emit_chains;
 // the histogram's LDS is left as it is); the value is lane 0's, NaN included.
+//
+// Every lane sums the same bins in the same order whenever the counts are the
+// same: bins that a counter drawn by the waves dealt out gave sums, and now and
+// then a float, that changed from run to run.  With a bin per lane at most there
+// is nothing to list (5,050 pairs of 5,000 voxels, 16 bins: 124 us listed, 115
+// not; 64 bins, smooth fields: 151 listed, 175 not).  The list holds what the LDS
+// has room for, and past it every bin is looked at (200 bins, noise of 4,700 bins:
+// 1,064 us with room for 3,072, 431 with room for 10,240).
 template <bool PACK16>
 __device__ __attribute__((always_inline)) double nmi64_pair(const uint32_t *s_hist, uint32_t *gh,
                                                             int H, int64_t N, PairLds<PACK16> &s,
@@ -626,8 +645,11 @@ __device__ __attribute__((always_inline)) double nmi64_pair(const uint32_t *s_hi
     atomicAdd(&s.cols[j], c);
     if (gh) gh[i * H + j] = 0u;  // zero at rest
   };
-  if (s.nbins <= (uint32_t)L::kBins) {
-    for (uint32_t k = tid; k < s.nbins; k += kHistBlock) {
+  const uint32_t nbins = __builtin_amdgcn_readfirstlane(H * H) > kHistBlock
+                             ? list_bins<PACK16>(s_hist, gh, H, s)
+                             : ~0u;
+  if (nbins <= (uint32_t)L::kBins) {
+    for (uint32_t k = tid; k < nbins; k += kHistBlock) {
       const int i = s.bins[k] >> 8, j = s.bins[k] & 255;
       fold(i, j, pair_count<PACK16>(s_hist, gh, H, i, j));
     }
