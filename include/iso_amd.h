@@ -201,7 +201,9 @@ int iso_field_interval(iso_ctx *ctx, const float *d_fields, int nfields, int64_t
  * Plain: d_map[i*n+j] = NMI of the H-bin joint histogram of fields (i, j),
  * all n*n entries.  multi != 0: d_fields holds 2n fields and
  * d_map[i*n+j] pairs field i with field n+j (TSM/VSM).  Bins follow
- * findBucket_d with the pair range [min(min_i,min_j), max(max_i,max_j)];
+ * findBucket_d with the pair range [min(min_i,min_j), max(max_i,max_j)], which
+ * d_mins and d_maxs must make cover both fields, as iso_field_interval's do (of a
+ * pair with values past its range the results are unspecified);
  * counts are exact; NMI follows the reference's float order with
  * ISO_COMPAT_NMI32 in flags, else it is evaluated from the exact counts in
  * double and rounded to float.  Optional outputs (NULL to skip), reference layout:

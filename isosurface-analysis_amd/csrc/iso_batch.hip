@@ -119,6 +119,7 @@ __global__ __launch_bounds__(kBBlock) __attribute__((amdgpu_waves_per_eu(PACK16 
         constexpr bool SUB = decltype(sub)::value;
         if constexpr (PACK16)
           iso::accumulate16<SUB, 2>(bin, f1 + b, f2 + b, len, s_hist, s.prog, [&](int i, int j) {
+            if (i >= H || j >= H) return;
             atomicAdd(&gh[i * H + j], 32768u);
             s.flushed = 1;
           });
@@ -137,8 +138,8 @@ __global__ __launch_bounds__(kBBlock) __attribute__((amdgpu_waves_per_eu(PACK16 
       for (int w = tid; w < words; w += kBBlock) {
         const uint32_t v = s_hist[w];
         const int r = w / iso::kRowWords, c = 2 * (w % iso::kRowWords);
-        if (v & 0xffffu) atomicAdd(&gh[r * H + c], v & 0xffffu);
-        if (v >> 16) atomicAdd(&gh[r * H + c + 1], v >> 16);
+        if ((v & 0xffffu) && c < H) atomicAdd(&gh[r * H + c], v & 0xffffu);
+        if ((v >> 16) && c + 1 < H) atomicAdd(&gh[r * H + c + 1], v >> 16);
       }
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
       __syncthreads();

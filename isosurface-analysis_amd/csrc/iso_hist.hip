@@ -229,6 +229,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(PACK16 ?
     constexpr bool SUB = decltype(sub)::value;
     if constexpr (PACK16)
       iso::accumulate16<SUB, STEP>(bin, f1, f2, len, s_hist, s.prog, [&](int i, int j) {
+        if (i >= H || j >= H) return;  // a value past the interval given
         atomicAdd(&gh[i * H + j], 32768u);
         s.flushed = 1;
       });
@@ -254,16 +255,17 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(PACK16 ?
   }
   uint32_t *src = nullptr;  // where the pair's counts are, if not in LDS
   if (a.slices > 1 || s.flushed) {
-    // LDS -> global 32-bit histogram of this task
+    // LDS -> global 32-bit histogram of this task (columns past H hold counts
+    // only for values past the interval given)
     for (int w = tid; w < words; w += kBlock) {
       const uint32_t v = s_hist[w];
       if (v) {
         const int r = w / iso::kRowWords, c = w % iso::kRowWords;
         if (PACK16) {
           const uint32_t lo = v & 0xffffu, hi = v >> 16;
-          if (lo) atomicAdd(&gh[r * H + 2 * c], lo);
-          if (hi) atomicAdd(&gh[r * H + 2 * c + 1], hi);
-        } else {
+          if (lo && 2 * c < H) atomicAdd(&gh[r * H + 2 * c], lo);
+          if (hi && 2 * c + 1 < H) atomicAdd(&gh[r * H + 2 * c + 1], hi);
+        } else if (c < H) {
           atomicAdd(&gh[r * H + c], v);
         }
       }
@@ -309,8 +311,8 @@ __global__ __launch_bounds__(256) void merge_kernel(HistArgs a) {
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const int c = (PACK16 ? 2 : 1) * (w + e);
-    if (lo[e]) gh[c] += lo[e];
-    if (PACK16 && hi[e]) gh[c + 1] += hi[e];
+    if (lo[e] && c < H) gh[c] += lo[e];
+    if (PACK16 && hi[e] && c + 1 < H) gh[c + 1] += hi[e];
   }
 }
 

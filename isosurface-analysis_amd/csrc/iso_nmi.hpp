@@ -323,7 +323,9 @@ __device__ __attribute__((always_inline)) void emit_chains(uint32_t *s_hist, int
     if (q < H) b.marg[(2 * t + (tid < 768 ? 0 : 1)) * H + q] = tid < 768 ? s.cols[q] : s.rows[q];
   }
   __syncthreads();
-  const uint32_t nz = s.wtot[4] + s.wtot[5] + s.wtot[6] + s.wtot[7];
+  // (columns past H hold counts only for values past the interval given)
+  const uint32_t nz = min(s.wtot[4] + s.wtot[5] + s.wtot[6] + s.wtot[7],
+                          (uint32_t)(b.list_bytes / sizeof(uint32_t)));
   const bool wide = s.big != 0u;
   if (tid < 512) {
     uint32_t off = 0u;
