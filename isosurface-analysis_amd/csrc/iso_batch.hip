@@ -315,12 +315,17 @@ int iso_ism_batch(iso_ctx *ctx, iso_ism_job *jobs, int njobs, int extractor, int
     const bool nmi32 = (flags & ISO_COMPAT_NMI32) != 0;
     const size_t hist_bytes = sizeof(uint32_t) * (size_t)H * iso::kRowWords;
     const size_t lds = hist_bytes + (pack16 ? sizeof(BatchLds<true>) : sizeof(BatchLds<false>));
+    // the LDS limit of the device's kernel, at the most bins' need: set to each
+    // call's own, one thread could lower it between another's call and launch
+    constexpr size_t row = sizeof(uint32_t) * iso::kRowWords;
     if (pack16)
       ISO_HIP_CHECK(ctx, hipFuncSetAttribute((const void *)hist_batch_kernel<true>,
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+                                             hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             (int)(256 * row + sizeof(BatchLds<true>))));
     else
       ISO_HIP_CHECK(ctx, hipFuncSetAttribute((const void *)hist_batch_kernel<false>,
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+                                             hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             (int)(128 * row + sizeof(BatchLds<false>))));
     BatchArgs ba;
     ba.fields = (const float *)fields;
     ba.mins = d_mins;

@@ -15,7 +15,6 @@
 // loop bound is a float (dataSize), so voxel i counts iff float(i) < float(n).
 #include <algorithm>
 #include <cstring>
-#include <mutex>
 
 #include "iso_internal.hpp"
 
@@ -273,13 +272,9 @@ int iso_equalized_isovalues(iso_ctx *ctx, const float *d_img, int64_t n, float r
   ISO_TRY(iso::enter(ctx));
   if (!d_img || n <= 0 || k <= 0 || !h_isos)
     return iso::fail(ctx, ISO_ERR_INVALID_ARG, "iso_equalized_isovalues: bad arguments");
-  static std::once_flag attr_once;
-  static hipError_t attr_err = hipSuccess;
-  std::call_once(attr_once, [] {
-    attr_err = hipFuncSetAttribute((const void *)uniform_hist_kernel,
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, kBins * 2);
-  });
-  ISO_HIP_CHECK(ctx, attr_err);
+  // (of the context's device: a process may hold contexts on several)
+  ISO_HIP_CHECK(ctx, hipFuncSetAttribute((const void *)uniform_hist_kernel,
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, kBins * 2));
   // voxel i counts iff float(i) < float(n): those below the first that does not
   const float fn = (float)n;
   int64_t counted = 0;
