@@ -280,8 +280,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(PACK16 ?
       }
       __syncthreads();
       if (!s.last) return;
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     }
+    // take_back reads with plain loads: no line of this CU's cache may be older
+    // than the atomics (an odd H's histogram shares lines with the pair before)
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     src = take_back<PACK16>(s_hist, gh, H);
   }
   finish_pair<PACK16>(a, s, s_hist, src, task, fi, fj);
