@@ -220,7 +220,7 @@ int iso_hist_nmi(iso_ctx *ctx, const float *d_fields, int n, int64_t F, int H, i
  * Same arguments, same results as iso_hist_nmi (the same kernel; the
  * default launch shape, no autotuning).  Its working memory is a
  * 64 MiB array per device, held until the process ends; pairs go through
- * in launches of as many as it holds (84 pairs at 256 bins).  Rejects
+ * in launches of as many as it holds (126 pairs at 256 bins).  Rejects
  * H > 256 and more than 65535 fields (ISO_ERR_UNSUPPORTED).  Calls that
  * overlap on one device share that array and race: serialise them. */
 int iso_hist_nmi_noalloc(iso_ctx *ctx, const float *d_fields, int n, int64_t F, int H, int multi,

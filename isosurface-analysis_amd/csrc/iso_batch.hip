@@ -333,12 +333,11 @@ int iso_ism_batch(iso_ctx *ctx, iso_ism_job *jobs, int njobs, int extractor, int
     ba.H = H;
     ba.nmi32 = nmi32 ? 1 : 0;
     ba.hist_bytes = (int)hist_bytes;
-    // tasks of a launch: what the memory for the chains' inputs holds (a graph
-    // keeps its own; the tasks' largest field comes first)
+    // tasks of a launch: what the memory for the chains' inputs holds (the tasks'
+    // largest field comes first)
     const bool graph = (flags & ISO_BATCH_GRAPH) != 0;
-    const size_t per = nmi32 ? iso::chain_task_bytes(H, tasks[0].F) : 1;
-    const int most = (int)std::min<size_t>(
-        nt, std::max<size_t>(1, nmi32 ? ((size_t)(graph ? 1 : 4) << 30) / per : (size_t)nt));
+    const int most = nmi32 ? iso::chain_tasks(ctx, H, tasks[0].F, nt) : nt;
+    if (nmi32) ISO_TRY(iso::chain_get(ctx, most, H, tasks[0].F, ba.chains));
     auto launch = [&](const BatchTask *d_tasks) -> int {
       for (int i0 = 0; i0 < nt; i0 += most) {
         ba.tasks = d_tasks + i0;
@@ -358,12 +357,13 @@ int iso_ism_batch(iso_ctx *ctx, iso_ism_job *jobs, int njobs, int extractor, int
     };
     const size_t tbytes = sizeof(BatchTask) * (size_t)nt, mbytes = sizeof(float *) * (size_t)njobs;
     const size_t hbytes = sizeof(uint32_t) * (size_t)groups * H * H;
-    const size_t cbytes = nmi32 ? per * (size_t)most + 512 : 0;
-    if (nmi32) ISO_TRY(iso::nmi_logs(ctx, &ba.chains.logs));
     if (graph) {
-      // the graph owns one buffer: tasks | maps | queue heads | drain area |
-      // chains' inputs; its key is the layout: the tasks, the launch shape and
-      // the inputs' addresses
+      // the graph owns one buffer: tasks | maps | queue heads | drain area; its
+      // key is the layout: the tasks, the launch shape and the addresses of the
+      // inputs and of the chains' inputs.  Those are the context's own, which
+      // every launch fills anew: a workspace that has grown gets another address,
+      // or at the same one holds what the graph needs, which has just been asked
+      // for.
       uint64_t key = 1469598103934665603ull;
       auto mix = [&](const void *p, size_t n) {
         const unsigned char *c = (const unsigned char *)p;
@@ -372,17 +372,18 @@ int iso_ism_batch(iso_ctx *ctx, iso_ism_job *jobs, int njobs, int extractor, int
       mix(tasks.data(), tbytes);
       // every kernel argument the capture bakes in: d_maxs = d_mins + ktotal
       // moves with ktotal even where d_mins and the tasks stay the same
-      const uint64_t shape[9] = {(uint64_t)H, (uint64_t)groups, (uint64_t)njobs,
+      const uint64_t shape[12] = {(uint64_t)H, (uint64_t)groups, (uint64_t)njobs,
                                  (uint64_t)(uintptr_t)fields, (uint64_t)(uintptr_t)d_mins,
                                  (uint64_t)(uintptr_t)d_maxs, (uint64_t)nt,
-                                 (uint64_t)ba.nmi32, (uint64_t)lds};
+                                 (uint64_t)ba.nmi32, (uint64_t)lds, (uint64_t)most,
+                                 (uint64_t)(uintptr_t)ba.chains.head,
+                                 (uint64_t)(uintptr_t)ba.chains.logs};
       mix(shape, sizeof shape);
       iso_ctx::graph_entry *ge = nullptr;
       for (auto &e : ctx->graphs)
         if (e.key == key) ge = &e;
       const size_t o_maps = (tbytes + 255) & ~(size_t)255, o_head = o_maps + ((mbytes + 255) & ~(size_t)255);
-      const size_t o_hist = o_head + 256, o_chains = o_hist + ((hbytes + 255) & ~(size_t)255);
-      const size_t need = o_chains + cbytes;
+      const size_t o_hist = o_head + 256, need = o_hist + hbytes;
       if (!ge) {
         if (ctx->graphs.size() >= 8) {  // keep a few layouts: drop the oldest
           ISO_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
@@ -401,7 +402,6 @@ int iso_ism_batch(iso_ctx *ctx, iso_ism_job *jobs, int njobs, int extractor, int
         ba.maps = (float *const *)(gb + o_maps);
         ba.next = (uint32_t *)(gb + o_head);
         ba.ghist = (uint32_t *)(gb + o_hist);
-        if (nmi32) iso::chain_carve(ba.chains, gb + o_chains, most, H, tasks[0].F);
         hipGraph_t captured = nullptr;
         ISO_HIP_CHECK(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
         const int rc = launch((const BatchTask *)gb);
@@ -434,11 +434,6 @@ int iso_ism_batch(iso_ctx *ctx, iso_ism_job *jobs, int njobs, int extractor, int
       ISO_TRY(iso::ws_get(ctx, WS_PIPE_G, 256, false, &dq));
       ISO_TRY(iso::ws_get(ctx, WS_PIPE_F, mbytes, false, &dmaps));
       ISO_TRY(iso::ws_get(ctx, WS_HIST_GLOBAL, hbytes, true, &gh));
-      if (nmi32) {
-        void *c = nullptr;
-        ISO_TRY(iso::ws_get(ctx, WS_NMI_CHAINS, cbytes, false, &c));
-        iso::chain_carve(ba.chains, c, most, H, tasks[0].F);
-      }
       ISO_HIP_CHECK(ctx, hipMemcpyAsync(dt, tasks.data(), tbytes, hipMemcpyHostToDevice,
                                         ctx->stream));
       ISO_HIP_CHECK(ctx, hipMemcpyAsync(dmaps, maps.data(), mbytes, hipMemcpyHostToDevice,

@@ -61,7 +61,6 @@ constexpr int kWaves = kBlock / 64;
 constexpr int kTileRows = 4, kTileCols = 8, kTilePairs = kTileRows * kTileCols;
 constexpr int kMaxTasksPerLaunch = 16384;  // one launch per 128-isovalue ISM (no tail wave)
 constexpr size_t kMaxPartBytes = (size_t)128 << 20;  // slices' histograms of a launch
-constexpr size_t kMaxChainBytes = (size_t)4 << 30;  // chains' inputs of a launch
 
 struct HistArgs {
   const float *fields;
@@ -445,6 +444,26 @@ int nmi_logs(iso_ctx *ctx, const float **out) {
   return ISO_OK;
 }
 
+int chain_tasks(const iso_ctx *ctx, int H, int64_t F, int64_t ntasks) {
+  size_t limit = kChainBytes;
+  if (const char *e = std::getenv("ISO_NMI_CHAIN_MIB")) {  // read per call
+    const long v = std::atol(e);
+    if (v > 0) limit = (size_t)std::min<long>(v, 65536) << 20;
+  }
+  // (a workspace that grows takes a quarter more)
+  const int64_t fit = (int64_t)(limit / 5 * 4 / chain_task_bytes(H, F));
+  const int64_t round = (int64_t)(H > 128 ? 1 : 2) * ctx->cu_count;
+  const int64_t most = fit >= round ? fit / round * round : std::max<int64_t>(1, fit);
+  return (int)std::min<int64_t>(most, std::min<int64_t>(ntasks, INT32_MAX));
+}
+
+int chain_get(iso_ctx *ctx, int64_t ntasks, int H, int64_t F, ChainBufs &b) {
+  void *p = nullptr;
+  ISO_TRY(ws_get(ctx, WS_NMI_CHAINS, chain_task_bytes(H, F) * (size_t)ntasks + kChainPad, false, &p));
+  chain_carve(b, p, ntasks, H, F);
+  return nmi_logs(ctx, &b.logs);
+}
+
 // Slices per pair, where the pairs alone leave CUs idle (one workgroup per CU
 // with 16-bit counters, two with 32-bit ones): as few rounds of voxels as
 // possible, a slice counting another 32K voxels' time for its start and the
@@ -486,13 +505,8 @@ int hist_nmi_tasks(iso_ctx *ctx, const float *d_fields, int n, int64_t F, int H,
   HistBufs b;
   int most = kMaxTasksPerLaunch;
   if (nmi32) {
-    // the chains' inputs, at most kMaxChainBytes of them (a launch's tasks)
-    const size_t per = chain_task_bytes(H, F);
-    most = (int)std::max<size_t>(1, std::min<size_t>(most, kMaxChainBytes / per));
-    void *c = nullptr;
-    ISO_TRY(ws_get(ctx, WS_NMI_CHAINS, per * (size_t)std::min(most, ntasks) + 512, false, &c));
-    chain_carve(b.chains, c, std::min(most, ntasks), H, F);
-    ISO_TRY(nmi_logs(ctx, &b.chains.logs));
+    most = std::min(most, chain_tasks(ctx, H, F, ntasks));
+    ISO_TRY(chain_get(ctx, most, H, F, b.chains));
   }
   const int64_t processed = processed_voxels(F, flags);
   auto run = [&](int variant) -> int {

@@ -100,7 +100,7 @@ struct iso_ctx {
   struct graph_entry {
     uint64_t key = 0;
     hipGraphExec_t exec = nullptr;
-    void *buf = nullptr;  // tasks | maps | queue heads | drain area | chains
+    void *buf = nullptr;  // tasks | maps | queue heads | drain area
     size_t bytes = 0;
     uint64_t replays = 0;
   };

@@ -47,25 +47,31 @@ namespace iso {
 __device__ __forceinline__ float logf_cr(float x) { return (float)log((double)x); }
 
 // Where a launch leaves what the chains need, per pair task: a header (number
-// of nonzero bins; 1 if a count needs 32 bits), the counts row by row and,
-// list_bytes after it, column by column (16 bits each, or 32), and the
-// marginals (H column sums, then H row sums).
+// of nonzero bins, number of entries in `large`), the low 16 bits of the counts
+// row by row and, list_bytes after it, column by column, those counts that need
+// more in full (place, past 2^31 in the column list; count), and the marginals (H
+// column sums, then H row sums).
 struct ChainBufs {
   uint2 *head = nullptr;
   unsigned char *lists = nullptr;  // 2 * list_bytes per task
   size_t list_bytes = 0;           // a multiple of 16
+  uint2 *large = nullptr;          // nlarge per task
+  uint32_t nlarge = 0;
   uint32_t *marg = nullptr;        // 2 * H words per task
   const float *logs = nullptr;     // logf of 0 (taken as 0) to kLogs - 1
 };
 constexpr int kLogs = 65536;
 
-// Room for one list: every nonzero bin, at most one per voxel, 32 bits each.
+// Room for one list: every nonzero bin, at most one per voxel, 16 bits each.
 __host__ __device__ inline size_t chain_list_bytes(int H, int64_t F) {
   const int64_t n = (int64_t)H * H < F ? (int64_t)H * H : F;
-  return ((size_t)n * 4 + 15) & ~(size_t)15;
+  return ((size_t)n * 2 + 15) & ~(size_t)15;
 }
 
-// Takes a launch's ChainBufs out of p (chain_task_bytes per task + 512).
+// Counts of 2^16 and more, in both lists: at most one per 2^16 voxels and list.
+__host__ __device__ inline size_t chain_large(int64_t F) { return 2 * (size_t)(F >> 16); }
+
+// Takes a launch's ChainBufs out of p (chain_task_bytes per task + kChainPad).
 inline void chain_carve(ChainBufs &b, void *p, int64_t ntasks, int H, int64_t F) {
   auto up = [](size_t n) { return (n + 255) & ~(size_t)255; };
   char *q = (char *)p;
@@ -73,13 +79,19 @@ inline void chain_carve(ChainBufs &b, void *p, int64_t ntasks, int H, int64_t F)
   q += up(sizeof(uint2) * (size_t)ntasks);
   b.marg = (uint32_t *)q;
   q += up(2 * sizeof(uint32_t) * (size_t)H * (size_t)ntasks);
+  b.large = (uint2 *)q;
+  b.nlarge = (uint32_t)chain_large(F);
+  q += up(sizeof(uint2) * b.nlarge * (size_t)ntasks);
   b.lists = (unsigned char *)q;
   b.list_bytes = chain_list_bytes(H, F);
 }
 
-// Device bytes of ChainBufs per task (without the logarithms).
+// Device bytes of ChainBufs per task (without the logarithms), and what rounding
+// its parts up takes.
+constexpr size_t kChainPad = 768;
 __host__ __device__ inline size_t chain_task_bytes(int H, int64_t F) {
-  return sizeof(uint2) + 2 * chain_list_bytes(H, F) + 2 * sizeof(uint32_t) * (size_t)H;
+  return sizeof(uint2) * (1 + chain_large(F)) + 2 * chain_list_bytes(H, F) +
+         2 * sizeof(uint32_t) * (size_t)H;
 }
 
 // number of set bits of m in the lanes below this one
@@ -103,7 +115,7 @@ struct PairLds {
   };
   uint32_t rowbase[kH], colbase[kH];
   uint32_t rows[kH], cols[kH];
-  uint32_t big;
+  uint32_t big, large;
   uint32_t wtot[kHistWaves];
 };
 
@@ -111,7 +123,7 @@ struct PairLds {
 template <bool PACK16>
 __device__ __forceinline__ void clear_pair_lds(PairLds<PACK16> &s) {
   if (threadIdx.x < PairLds<PACK16>::kH) s.rows[threadIdx.x] = s.cols[threadIdx.x] = 0u;
-  if (threadIdx.x == 0) s.big = 0u;
+  if (threadIdx.x == 0) s.big = s.large = 0u;
 }
 
 // The count of bin (i, j): from the LDS histogram or, when gh is not null, from
@@ -221,7 +233,7 @@ __device__ __forceinline__ void each_bin(const uint32_t *s_hist, const uint32_t 
 // The counts wait in registers while their LDS takes the lists, so the lists
 // leave in coalesced stores (scattered 2-byte stores of some 4,000 bins to both
 // lists would cost the L2 8,000 transactions per pair).  Counts past 16 bits
-// (rare) go out one by one.
+// (rare) go out one by one as well.
 template <bool PACK16, bool GH>
 __device__ __attribute__((always_inline)) void emit_chains(uint32_t *s_hist, int hist_bytes,
                                                            uint32_t *gh, int H, bool mirror,
@@ -325,7 +337,7 @@ __device__ __attribute__((always_inline)) void emit_chains(uint32_t *s_hist, int
   __syncthreads();
   // (columns past H hold counts only for values past the interval given)
   const uint32_t nz = min(s.wtot[4] + s.wtot[5] + s.wtot[6] + s.wtot[7],
-                          (uint32_t)(b.list_bytes / sizeof(uint32_t)));
+                          (uint32_t)(b.list_bytes / sizeof(uint16_t)));
   const bool wide = s.big != 0u;
   if (tid < 512) {
     uint32_t off = 0u;
@@ -333,12 +345,11 @@ __device__ __attribute__((always_inline)) void emit_chains(uint32_t *s_hist, int
     const int q = tid & 255;
     if (q < kH) (tid < 256 ? s.colbase : s.rowbase)[q] = incl - mine + off;
   }
-  if (tid == 0) b.head[t] = make_uint2(nz, wide ? 1u : 0u);
   __syncthreads();
   unsigned char *la = b.lists + 2 * (size_t)t * b.list_bytes, *lb = la + b.list_bytes;
   // each list's room in LDS, whole 16-byte pieces
   const uint32_t room = (2u * nz + 15u) & ~15u;
-  const bool staged = !GH && !wide && 2u * room <= (uint32_t)hist_bytes;
+  const bool staged = !GH && 2u * room <= (uint32_t)hist_bytes;
   uint16_t *wa = reinterpret_cast<uint16_t *>(s_hist), *wb = wa + room / 2;
   uint32_t col[C];  // the lane's columns' next places
 #pragma unroll
@@ -367,12 +378,15 @@ __device__ __attribute__((always_inline)) void emit_chains(uint32_t *s_hist, int
         if (staged) {
           if (row < nz) wa[row] = (uint16_t)v[c];
           if (mirror && col[c] < nz) wb[col[c]] = (uint16_t)v[c];
-        } else if (wide) {
-          if (row < nz) reinterpret_cast<uint32_t *>(la)[row] = v[c];
-          if (mirror && col[c] < nz) reinterpret_cast<uint32_t *>(lb)[col[c]] = v[c];
         } else {
           if (row < nz) reinterpret_cast<uint16_t *>(la)[row] = (uint16_t)v[c];
           if (mirror && col[c] < nz) reinterpret_cast<uint16_t *>(lb)[col[c]] = (uint16_t)v[c];
+        }
+        if (wide && v[c] > 0xffffu) {
+          const uint32_t k = atomicAdd(&s.large, mirror ? 2u : 1u);
+          uint2 *at = b.large + (size_t)t * b.nlarge + k;
+          if (k < b.nlarge) at[0] = make_uint2(row, v[c]);
+          if (mirror && k + 1u < b.nlarge) at[1] = make_uint2(col[c] | 1u << 31, v[c]);
         }
         if (GH) gh[(i0 + r) * H + j0 + c] = 0u;  // zero at rest (zero bins already are)
         ++row;
@@ -380,8 +394,9 @@ __device__ __attribute__((always_inline)) void emit_chains(uint32_t *s_hist, int
       }
     }
   }
-  if (!staged) return;
   __syncthreads();
+  if (tid == 0) b.head[t] = make_uint2(nz, min(s.large, b.nlarge));
+  if (!staged) return;
   const uint4 *src = reinterpret_cast<const uint4 *>(s_hist);
   const int n16 = (int)(room / 16u);
   for (int k = tid; k < (mirror ? 2 : 1) * n16; k += kHistBlock)
@@ -499,14 +514,16 @@ __device__ __attribute__((always_inline)) void fold_chains(const ChainBufs &b, i
   // chains of the same numbers
   constexpr int kLists = 2 * kFoldPairs, kOwn = (kLists + kFoldWaves - 2) / (kFoldWaves - 1);
   int len[kOwn];
-  bool wide[kOwn];
+  uint32_t nlarge[kOwn];
+  const uint2 *large[kOwn];
   const unsigned char *src[kOwn];
 #pragma unroll
   for (int u = 0; u < kOwn; ++u) {
     const int lc = w - 1 + u * (kFoldWaves - 1);
     len[u] = lc < kLists ? length(lc >> 1, lc & 1) : 0;
     const int64_t t = t0 + (len[u] ? lc >> 1 : 0);
-    wide[u] = __builtin_amdgcn_readfirstlane((int)b.head[t].y) != 0;
+    nlarge[u] = (uint32_t)__builtin_amdgcn_readfirstlane((int)b.head[t].y);
+    large[u] = b.large + (size_t)t * b.nlarge;
     src[u] = b.lists + (2 * (size_t)t + (lc & 1)) * b.list_bytes;
   }
   constexpr int kPer = kFoldBlock / 64;  // terms of a chain a lane lays out per step
@@ -525,19 +542,19 @@ __device__ __attribute__((always_inline)) void fold_chains(const ChainBufs &b, i
       if (q * kFoldBlock < len[u]) {
         const int k = q * kFoldBlock + kPer * lane, i = k < len[u] ? k : 0;
         uint32_t x[kPer];
-        struct alignas(4 * kPer) Wide { uint32_t v[kPer]; };
         struct alignas(2 * kPer) Narrow { uint32_t v[kPer / 2]; };
-        if (wide[u]) {
-          const Wide y = reinterpret_cast<const Wide *>(src[u])[i / kPer];
+        const Narrow y = reinterpret_cast<const Narrow *>(src[u])[i / kPer];
 #pragma unroll
-          for (int c = 0; c < kPer; ++c) x[c] = y.v[c];
-        } else {
-          const Narrow y = reinterpret_cast<const Narrow *>(src[u])[i / kPer];
+        for (int c = 0; c < kPer; c += 2) {
+          x[c] = y.v[c / 2] & 0xffffu;
+          x[c + 1] = y.v[c / 2] >> 16;
+        }
+        for (uint32_t e = 0; e < nlarge[u]; ++e) {
+          const uint2 full = large[u][e];
+          const uint32_t list = (uint32_t)(w - 1 + u * (kFoldWaves - 1)) & 1u;
 #pragma unroll
-          for (int c = 0; c < kPer; c += 2) {
-            x[c] = y.v[c / 2] & 0xffffu;
-            x[c + 1] = y.v[c / 2] >> 16;
-          }
+          for (int c = 0; c < kPer; ++c)
+            if (full.x == ((uint32_t)(k + c) | list << 31)) x[c] = full.y;
         }
 #pragma unroll
         for (int c = 0; c < kPer; ++c) n.v[u][c] = k + c < len[u] ? x[c] : 0u;
@@ -560,7 +577,7 @@ __device__ __attribute__((always_inline)) void fold_chains(const ChainBufs &b, i
     for (int u = 0; u < kOwn; ++u) {
       const int lc = w - 1 + u * (kFoldWaves - 1);
       if (lc >= kLists || (q - 2) * kFoldBlock >= len[u]) continue;
-      if (wide[u]) {  // counts past the table
+      if (nlarge[u]) {  // counts past the table
 #pragma unroll
         for (int c = 0; c < kPer; ++c)
           if (n.v[u][c] >= (uint32_t)kLogs) g.t[u][c] = logf_cr((float)n.v[u][c]);
@@ -685,6 +702,16 @@ __device__ __attribute__((always_inline)) double nmi64_pair(const uint32_t *s_hi
 // first use, or into the caller's memory.
 int nmi_logs(iso_ctx *ctx, const float **out);
 int nmi_logs_fill(iso_ctx *ctx, float *d_logs);
+
+// Tasks of a launch in the reference's float order, ntasks at most: as many whole
+// rounds of workgroups as kChainBytes of the chains' inputs hold (F: the tasks'
+// largest), one task in any case.  ISO_NMI_CHAIN_MIB in the environment sets
+// another limit.
+constexpr size_t kChainBytes = (size_t)2 << 30;
+int chain_tasks(const iso_ctx *ctx, int H, int64_t F, int64_t ntasks);
+
+// The context's ChainBufs for a launch of ntasks tasks.
+int chain_get(iso_ctx *ctx, int64_t ntasks, int H, int64_t F, ChainBufs &b);
 
 // Device buffers one launch of the histogram + NMI kernels works in: merged
 // 32-bit histograms and slice arrival counters per task (zero at rest), the

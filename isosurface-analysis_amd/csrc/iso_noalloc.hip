@@ -6,7 +6,7 @@
 // and the reference-order NMI's logarithms and chain inputs -- lives in one
 // file-scope device array, `scratch`, of 64 MiB per device, held until the
 // process ends.  Pairs go through in launches of as many tasks as the array
-// holds at once (84 at 256 bins), so any number of fields fits.
+// holds at once (126 at 256 bins), so any number of fields fits.
 //
 // Host code never uses the array's name as an address: at set-up (the
 // context's creation, else this entry point's first call on a device) the
@@ -117,7 +117,7 @@ int iso_hist_nmi_noalloc(iso_ctx *ctx, const float *d_fields, int n, int64_t F, 
     off += align256(sizeof(float) * iso::kLogs);
     per_task += iso::chain_task_bytes(H, F);
   }
-  constexpr size_t kPad = 5 * 256;  // what rounding the parts up takes
+  constexpr size_t kPad = 8 * 256;  // what rounding the parts up takes
   if (off + kPad + per_task > kScratchBytes)
     return iso::fail(ctx, ISO_ERR_UNSUPPORTED, "iso_hist_nmi_noalloc: %d bins exceed the %zu-byte scratch",
                      H, kScratchBytes);
@@ -130,7 +130,7 @@ int iso_hist_nmi_noalloc(iso_ctx *ctx, const float *d_fields, int n, int64_t F, 
   off += align256(4 * (size_t)T);
   if (nmi32) {
     iso::chain_carve(b.chains, p + off, T, H, F);
-    off += align256(iso::chain_task_bytes(H, F) * (size_t)T + 512);
+    off += align256(iso::chain_task_bytes(H, F) * (size_t)T + iso::kChainPad);
   }
   b.ghist = (uint32_t *)(p + off);
   off += align256(4 * (size_t)T * H * H);
