@@ -1616,14 +1616,15 @@ int df_pool(iso_ctx *ctx, const void *d_xyz, bool is_int, int64_t ntot, const ui
                        : bricks(4) >= 4 * max_waves                              ? 4
                                                                                 : 2;
   // (B, samples per lane) per variant, picked by the autotuner; ISO_DF_LEAF=B
-  // (8..64) forces B, with ISO_DF_SPL=1, 2 or 4 (default 1)
+  // (8..64) forces B, with ISO_DF_SPL=1, 2 or 4 (default 1) and ISO_DF_STAY=32 a
+  // wave per brick up to 32 for each that fits the chip (default 4)
   const int leaf[4] = {64, by_brick ? 64 : 48, 64, 64};
   const int lane[4] = {4, by_brick ? by_brick : 2, 2, 1};
   if (const char *e = std::getenv("ISO_DF_LEAF")) {  // read per call
     const int v = std::atoi(e);
-    const char *q = std::getenv("ISO_DF_SPL");
+    const char *q = std::getenv("ISO_DF_SPL"), *r = std::getenv("ISO_DF_STAY");
     const int spl = q && (q[0] == '2' || q[0] == '4') ? q[0] - '0' : 1;
-    if (v >= 8 && v <= kMaxLeaf) return run_variant(v, spl, can_pool, 4);
+    if (v >= 8 && v <= kMaxLeaf) return run_variant(v, spl, can_pool, r && std::atoi(r) == 32 ? 32 : 4);
   }
   // variants 0-3: leaves from the pool's runs; 4-7 (or 0-3 when the pool path
   // is out): leaves from the sorted points.  The second variant's form is the
