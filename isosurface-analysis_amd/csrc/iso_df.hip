@@ -1608,42 +1608,48 @@ int df_pool(iso_ctx *ctx, const void *d_xyz, bool is_int, int64_t ntot, const ui
   // bricks: which is faster hangs on the sets, not on their sizes (maps in
   // columns, by brick, us: 96^3 blobs, 16 isovalues 1,204, 776; 100^3, 24: 1,350,
   // 958; 200^3 at ds 2, 48: 2,400, 1,768; a 600x248x248 front at ds 4, 12: 2,055,
-  // 2,212; 50: 8,358, 10,250).  It takes the place of the leaves of 48 points.
+  // 2,212; 50: 8,358, 10,250).
   const auto bricks = [&](int spl) {
     return (uint64_t)((g.nx + 3) / 4) * ((g.ny + 3) / 4) * ((g.nz + 4 * spl - 1) / (4 * spl)) * S;
   };
   const int by_brick = bricks(2) < 4 * max_waves || bricks(4) >= 32 * max_waves ? 0
                        : bricks(4) >= 4 * max_waves                              ? 4
                                                                                 : 2;
-  // (B, samples per lane) per variant, picked by the autotuner; ISO_DF_LEAF=B
-  // (8..64) forces B, with ISO_DF_SPL=1, 2 or 4 (default 1) and ISO_DF_STAY=32 a
-  // wave per brick up to 32 for each that fits the chip (default 4)
-  const int leaf[4] = {64, by_brick ? 64 : 48, 64, 64};
-  const int lane[4] = {4, by_brick ? by_brick : 2, 2, 1};
+  // ISO_DF_LEAF=B (8..64) forces B, with ISO_DF_SPL=1, 2 or 4 samples per lane
+  // (default 1) and ISO_DF_STAY=32 a wave per brick up to 32 for each that fits the
+  // chip (default 4)
   if (const char *e = std::getenv("ISO_DF_LEAF")) {  // read per call
     const int v = std::atoi(e);
     const char *q = std::getenv("ISO_DF_SPL"), *r = std::getenv("ISO_DF_STAY");
     const int spl = q && (q[0] == '2' || q[0] == '4') ? q[0] - '0' : 1;
     if (v >= 8 && v <= kMaxLeaf) return run_variant(v, spl, can_pool, r && std::atoi(r) == 32 ? 32 : 4);
   }
-  // variants 0-3: leaves from the pool's runs; 4-7 (or 0-3 when the pool path
-  // is out): leaves from the sorted points.  The second variant's form is the
-  // key's least part, so that sizes decide which tuned key is the nearest.
-  const bool both = can_pool && can_sort;
+  // Forms, picked by the autotuner: leaf points and samples per lane 64,4, 48,2,
+  // 64,2, 64,1 and by brick; their numbers, and from 8 on the same over leaves from
+  // the sorted points instead of the pool's runs.  By brick is a candidate where
+  // by_brick is not 0, in place of 48,2.  The choice of other sizes may bring either
+  // anywhere: by brick then stands for 64,2, whose waves take a brick each below
+  // 4 x max_waves and stay from 32 x.
+  // by_brick is the key's least part, so that sizes decide which tuned key is the
+  // nearest.
+  enum { kWide, kSmallLeaves, kTwo, kOne, kByBrick, kSorted = 8 };
+  const bool pool = can_pool, both = can_pool && can_sort;
+  std::vector<int> cand;
+  for (int s = pool ? 0 : kSorted; s <= (both || !pool ? kSorted : 0); s += kSorted)
+    for (int f : {(int)kWide, by_brick ? (int)kByBrick : (int)kSmallLeaves, (int)kTwo, (int)kOne})
+      cand.push_back(s + f);
   const uint64_t key = ((uint64_t)(can_pool ? 1 + both : 0) << 32) |
                        ((uint64_t)ceil_log2((uint64_t)(ntot / S + 1)) << 16) |
                        ((uint64_t)ceil_log2((uint64_t)F) << 3) | (uint64_t)by_brick;
-  const char *what = both ? "lbvh (leaves, leaf points, samples per lane) {runs 64,4|runs 48,2 or by "
-                            "brick|runs 64,2|runs 64,1|sorted 64,4|sorted 48,2 or by brick|"
-                            "sorted 64,2|sorted 64,1}"
-                     : can_pool ? "lbvh (leaves from runs: leaf points, samples per lane) "
-                                  "{64,4|48,2 or by brick|64,2|64,1}"
-                                : "lbvh (leaves from sorted points: leaf points, samples per lane) "
-                                  "{64,4|48,2 or by brick|64,2|64,1}";
-  return tune_pick(ctx, kTuneTraverse, key, both ? 8 : 4, 2, what, [&](int v) {
-    const bool brick = by_brick && (v & 3) == 1;
-    return run_variant(leaf[v & 3], lane[v & 3], can_pool && v < 4, brick ? 32 : 4);
-  });
+  return tune_pick(ctx, kTuneTraverse, key, cand, pool ? kTwo : kSorted + kTwo,
+                   "lbvh leaf points, samples per lane {0: 64,4 | 1: 48,2 | 2: 64,2 | 3: 64,1 | "
+                   "4: 64, by brick; from 8: the same over sorted points}",
+                   [&](int v) {
+                     const int f = v & 7, spl = f == kWide ? 4 : f == kOne ? 1 : 2;
+                     const bool runs = pool && (v < kSorted || !both);
+                     if (f == kByBrick && by_brick) return run_variant(64, by_brick, runs, 32);
+                     return run_variant(f == kSmallLeaves ? 48 : 64, spl, runs, 4);
+                   });
 }
 
 }  // namespace iso

@@ -531,8 +531,8 @@ int hist_nmi_tasks(iso_ctx *ctx, const float *d_fields, int n, int64_t F, int H,
   };
   const uint64_t key = ((uint64_t)H << 32) | ((uint64_t)ceil_log2((uint64_t)processed) << 16) |
                        (uint64_t)ceil_log2((uint64_t)ntasks);
-  return tune_pick(ctx, kTuneHist, key, 2, 1,
-                   pack16 ? "hist16 rounds ahead {1,2}" : "hist32 loads/step {4,8}", run);
+  return tune_pick(ctx, kTuneHist, key, {0, 1}, 1,
+                   pack16 ? "hist16 rounds ahead {0: 1, 1: 2}" : "hist32 loads/step {0: 4, 1: 8}", run);
 }
 
 // One launch of the histogram + NMI kernels over nt tasks with the caller's

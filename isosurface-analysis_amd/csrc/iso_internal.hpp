@@ -142,16 +142,20 @@ inline bool iso_before(float a, float b) { return a < b || (b != b && a == a); }
 
 enum iso_tune_kind { kTuneHist = 1, kTuneTraverse = 2 };
 
-// Autotuner.  run(v) enqueues variant v (0 <= v < ncand) of one launch on the
-// context's stream; every variant computes the same result.  The first time
-// a (kind, key) shape class is seen, each variant runs once on the real data,
-// timed with HIP events, the two fastest run once more, and the one of those
-// two with the smaller total is kept for the context's lifetime;
+// Autotuner.  run(v) enqueues variant v of one launch on the context's stream;
+// every variant computes the same result.  A variant's number (below 16) means
+// one form of a kind whatever the key; cand holds those that a key's shapes are
+// timed with (run takes any: a frozen lookup may bring the number of a form that
+// another key's shapes were timed with).  The first time a (kind, key) shape class
+// is seen, each candidate runs once on the real data, timed with HIP events, the
+// two fastest run once more, and the one of those two with the smaller total is
+// kept for the context's lifetime;
 // later calls run the kept variant only.  ISO_AUTOTUNE=0 in the environment
 // keeps the default variant instead of measuring.
 template <class Run>
-int tune_pick(iso_ctx *ctx, int kind, uint64_t key, int ncand, int dflt, const char *what,
-              Run &&run) {
+int tune_pick(iso_ctx *ctx, int kind, uint64_t key, const std::vector<int> &cand, int dflt,
+              const char *what, Run &&run) {
+  const int ncand = (int)cand.size();
   const uint64_t k = ((uint64_t)kind << 56) ^ key;
   auto it = ctx->tune.find(k);
   if (it != ctx->tune.end()) return run(it->second);
@@ -188,7 +192,7 @@ int tune_pick(iso_ctx *ctx, int kind, uint64_t key, int ncand, int dflt, const c
   }
   int best = dflt, st = ISO_OK;
   ctx->tune_measured++;
-  char buf[512];
+  char buf[768];
   int pos = snprintf(buf, sizeof buf, "%s [key %llx]:", what, (unsigned long long)key);
   auto timed = [&](int v, float &ms) -> bool {
     (void)hipEventRecord(e0, ctx->stream);
@@ -204,8 +208,9 @@ int tune_pick(iso_ctx *ctx, int kind, uint64_t key, int ncand, int dflt, const c
   std::vector<float> t(ncand, 3.0e38f);
   bool ok = true;
   for (int v = 0; v < ncand && ok; ++v) {
-    ok = timed(v, t[v]);
-    if (ok && pos < (int)sizeof buf) pos += snprintf(buf + pos, sizeof buf - pos, " %.3f", t[v]);
+    ok = timed(cand[v], t[v]);
+    if (ok && pos < (int)sizeof buf)
+      pos += snprintf(buf + pos, sizeof buf - pos, " %d: %.3f", cand[v], t[v]);
   }
   if (ok) {
     int a = 0, b = -1;
@@ -214,11 +219,12 @@ int tune_pick(iso_ctx *ctx, int kind, uint64_t key, int ncand, int dflt, const c
       else if (b < 0 || t[v] < t[b]) b = v;
     }
     float ra = 0.0f, rb = 0.0f;
-    ok = timed(a, ra) && timed(b, rb);
+    ok = timed(cand[a], ra) && timed(cand[b], rb);
     if (ok) {
-      best = (t[a] + ra <= t[b] + rb) ? a : b;
+      best = (t[a] + ra <= t[b] + rb) ? cand[a] : cand[b];
       if (pos < (int)sizeof buf)
-        pos += snprintf(buf + pos, sizeof buf - pos, " | again %d: %.3f, %d: %.3f", a, ra, b, rb);
+        pos += snprintf(buf + pos, sizeof buf - pos, " | again %d: %.3f, %d: %.3f", cand[a], ra,
+                        cand[b], rb);
     }
   }
   (void)hipEventDestroy(e0);
