@@ -265,15 +265,18 @@ __global__ __launch_bounds__(kBfBlock) void brute_kernel(iso::SampleGrid g, int6
   }
   __syncthreads();  // the points are read
 #pragma unroll
-  for (int q = 0; q < kBfSamples; ++q) s.best[w][q][lane] = (&best[0][0][0])[q];
+  for (int q = 0; q < kBfSamples; ++q)  // (turned by q: lanes read along q below)
+    s.best[w][q][(lane + q) & 63] = (&best[0][0][0])[q];
   __syncthreads();
   uint32_t *out = best_bits + (int64_t)seg * F;
-  for (int t = threadIdx.x; t < 64 * kBfSamples; t += kBfBlock) {  // z fastest, then blocks
-    const int k = t % TZ, l = t / TZ % 64, ij = t / TZ / 64;
+  // z fastest, then blocks; samples, then blocks where a block is a line
+  constexpr int kRun = TX == kBfSamples || TY == kBfSamples ? kBfSamples : TZ;
+  for (int t = threadIdx.x; t < 64 * kBfSamples; t += kBfBlock) {
+    const int l = t / kRun % 64, q = t % kRun + t / kRun / 64 * kRun, k = q % TZ, ij = q / TZ;
     if ((int64_t)blockIdx.x * 64 + l >= blocks) continue;
     float m = INFINITY;
 #pragma unroll
-    for (int i = 0; i < kBfWaves; ++i) m = fminf(m, s.best[i][ij * TZ + k][l]);
+    for (int i = 0; i < kBfWaves; ++i) m = fminf(m, s.best[i][q][(l + q) & 63]);
     corner(l, x0, y0, z0);
     const int x = x0 + ij / TY, y = y0 + ij % TY, z = z0 + k;
     if (x < g.nx && y < g.ny && z < g.nz)
@@ -296,10 +299,22 @@ void brute_launch_as(iso_ctx *ctx, const iso::SampleGrid &g, int64_t F, const Pt
 // bits[s*F + i] = min(bits[s*F + i], squared distance of sample i to set s)
 void brute_launch(iso_ctx *ctx, const iso::SampleGrid &g, int64_t F, const Pt *pts,
                   const int64_t *d_off, int S, int64_t avg, uint32_t *bits) {
-  if (g.nz == 1)  // a flat grid would leave three quarters of a 2 x 4 x 4 block empty
-    brute_launch_as<8, 4, 1>(ctx, g, F, pts, d_off, S, avg, bits);
-  else
-    brute_launch_as<2, 4, 4>(ctx, g, F, pts, d_off, S, avg, bits);
+  // the shape of a lane's block that costs the least vector instructions, a point's
+  // for a block times the blocks: 2 x 4 x 4 unless a short axis would leave most of
+  // it empty, which shows from 64 workgroups of such blocks on (100,000 samples on a line along x, y, z against 5,000 points: 171, 279,
+  // 218 us by 2 x 4 x 4 or 8 x 4 x 1, 93, 83, 71 by lines; 300 x 1 x 300: 126, 71)
+  const auto cost = [&](int tx, int ty, int tz, int per_block) {
+    return (int64_t)((g.nx + tx - 1) / tx) * ((g.ny + ty - 1) / ty) * ((g.nz + tz - 1) / tz) * per_block;
+  };
+  const int64_t block = cost(2, 4, 4, 68), flat = cost(8, 4, 1, 101), x = cost(32, 1, 1, 146),
+                y = cost(1, 32, 1, 115), z = cost(1, 1, 32, 84);
+  const int64_t least = block < 68 * 64 * 64 ? (g.nz == 1 ? flat : block)
+                                             : std::min({block, flat, x, y, z});
+  if (least == block) brute_launch_as<2, 4, 4>(ctx, g, F, pts, d_off, S, avg, bits);
+  else if (least == flat) brute_launch_as<8, 4, 1>(ctx, g, F, pts, d_off, S, avg, bits);
+  else if (least == z) brute_launch_as<1, 1, 32>(ctx, g, F, pts, d_off, S, avg, bits);
+  else if (least == y) brute_launch_as<1, 32, 1>(ctx, g, F, pts, d_off, S, avg, bits);
+  else brute_launch_as<32, 1, 1>(ctx, g, F, pts, d_off, S, avg, bits);
 }
 
 __global__ void finish_kernel(uint32_t *bits, int64_t F, const int64_t *off, int S, float *df) {
