@@ -82,9 +82,9 @@ template <bool PACK16>
 __global__ __launch_bounds__(kBBlock) __attribute__((amdgpu_waves_per_eu(PACK16 ? 4 : 8))) void hist_batch_kernel(BatchArgs a) {
   extern __shared__ uint4 s_dyn[];
   uint32_t *s_hist = reinterpret_cast<uint32_t *>(s_dyn);
-  BatchLds<PACK16> &s = *reinterpret_cast<BatchLds<PACK16> *>(s_hist + a.H * iso::kRowWords);
+  BatchLds<PACK16> &s = *reinterpret_cast<BatchLds<PACK16> *>(s_hist + a.H * iso::kRowWords<PACK16>);
   const int tid = threadIdx.x, H = a.H;
-  const int words = H * iso::kRowWords;
+  const int words = H * iso::kRowWords<PACK16>;
   uint32_t *gh = a.ghist + (int64_t)blockIdx.x * H * H;
   int queue = blockIdx.x % kQueues, empty = 0;  // (lane 0's)
   while (true) {
@@ -137,7 +137,7 @@ __global__ __launch_bounds__(kBBlock) __attribute__((amdgpu_waves_per_eu(PACK16 
       src = gh;
       for (int w = tid; w < words; w += kBBlock) {
         const uint32_t v = s_hist[w];
-        const int r = w / iso::kRowWords, c = 2 * (w % iso::kRowWords);
+        const int r = w / iso::kRowWords<PACK16>, c = 2 * (w % iso::kRowWords<PACK16>);
         if ((v & 0xffffu) && c < H) atomicAdd(&gh[r * H + c], v & 0xffffu);
         if ((v >> 16) && c + 1 < H) atomicAdd(&gh[r * H + c + 1], v >> 16);
       }
@@ -313,19 +313,19 @@ int iso_ism_batch(iso_ctx *ctx, iso_ism_job *jobs, int njobs, int extractor, int
     const int per_cu = pack16 ? 1 : 2;  // 1024-lane workgroups per CU (LDS)
     const int groups = std::min(nt, per_cu * ctx->cu_count);
     const bool nmi32 = (flags & ISO_COMPAT_NMI32) != 0;
-    const size_t hist_bytes = sizeof(uint32_t) * (size_t)H * iso::kRowWords;
+    const size_t hist_bytes = sizeof(uint32_t) * (size_t)H * iso::row_words(H);
     const size_t lds = hist_bytes + (pack16 ? sizeof(BatchLds<true>) : sizeof(BatchLds<false>));
     // the LDS limit of the device's kernel, at the most bins' need: set to each
     // call's own, one thread could lower it between another's call and launch
-    constexpr size_t row = sizeof(uint32_t) * iso::kRowWords;
+    
     if (pack16)
       ISO_HIP_CHECK(ctx, hipFuncSetAttribute((const void *)hist_batch_kernel<true>,
                                              hipFuncAttributeMaxDynamicSharedMemorySize,
-                                             (int)(256 * row + sizeof(BatchLds<true>))));
+                                             (int)(256 * 4 * iso::kRowWords<true> + sizeof(BatchLds<true>))));
     else
       ISO_HIP_CHECK(ctx, hipFuncSetAttribute((const void *)hist_batch_kernel<false>,
                                              hipFuncAttributeMaxDynamicSharedMemorySize,
-                                             (int)(128 * row + sizeof(BatchLds<false>))));
+                                             (int)(128 * 4 * iso::kRowWords<false> + sizeof(BatchLds<false>))));
     BatchArgs ba;
     ba.fields = (const float *)fields;
     ba.mins = d_mins;

@@ -38,6 +38,17 @@ __device__ __forceinline__ uint32_t max3_u16(uint32_t a, uint32_t b, uint32_t c)
   return r;
 }
 
+// Words of a row of the LDS histogram: 256 16-bit or 128 32-bit counters, and 8
+// more between the 32-bit rows.  Rows of 128 words put a column's counters of all
+// rows into one bank: with 2 bins per axis the lanes met in 2 banks of 64 (820 pairs
+// of 300,000 voxels of noise: 528 us, with the 8 words 427), and those of smooth
+// fields, which lie along the diagonal, in fewer than now (5,050 pairs of 100,000
+// voxels, 128 bins: 757 us, 581).
+template <bool PACK16>
+constexpr int kRowWords = PACK16 ? 128 : 136;
+// ... with H bins per axis (16-bit counters past 128)
+inline int row_words(int H) { return H > 128 ? kRowWords<true> : kRowWords<false>; }
+
 // Joint bins of a pair of fields with range [mn, mx] and H <= 256 bins, as
 // the reference computes them (JointHistogram.cu:63-75, :127-129): step =
 // (mx - mn) / H, bin = (int)((v - mn) / step) clamped to H - 1, step == 0 ->
@@ -99,8 +110,8 @@ struct PairBins {
   }
 
   // Byte offset of (row, col)'s counter in the LDS histogram.  16-bit counters:
-  // rows of 512 bytes, 2 per column; bits 0 and 1 are not part of the word's
-  // address.  32-bit ones: rows of 512 bytes, 4 per column.
+  // 2 per column; bits 0 and 1 are not part of the word's address.  32-bit ones: 4
+  // per column.
   static constexpr uint32_t kColBytes = PACK16 ? 2u : 4u;
 
   // at[u] = offset of (x[u], y[u])'s counter
@@ -114,7 +125,7 @@ struct PairBins {
 #pragma unroll
     for (int u = 0; u < N; ++u) {
       const uint32_t ux = fixed(x[u]), uy = fixed(y[u]);
-      at[u] = mad_hi16(uy, kColBytes, mad_hi16(ux, 512u, 0u));
+      at[u] = mad_hi16(uy, kColBytes, mad_hi16(ux, 4u * kRowWords<PACK16>, 0u));
       most = max3_u16(most, ux, uy);
     }
     if (__builtin_expect(__ballot((most & 0xffffu) > top) != 0ull, 0)) {
@@ -123,7 +134,7 @@ struct PairBins {
         float a = x[u], b = y[u];
         asm volatile("" : "+v"(a), "+v"(b));  // nothing of this ahead of the branch
         const uint32_t low = max3_u16(0u, fixed(a), fixed(b));
-        if (__ballot((low & 0xffffu) > top) != 0ull) at[u] = exact(a) * 512u + exact(b) * kColBytes;
+        if (__ballot((low & 0xffffu) > top) != 0ull) at[u] = exact(a) * (4u * kRowWords<PACK16>) + exact(b) * kColBytes;
       }
     }
   }
@@ -137,14 +148,11 @@ struct PairBins {
   }
 };
 
-// words of a row of the LDS histogram: 256 16-bit or 128 32-bit counters
-constexpr int kRowWords = 128;
-
 // The count of bin (i, j) in the LDS histogram.
 template <bool PACK16>
 __device__ __forceinline__ uint32_t lds_count(const uint32_t *s, int i, int j) {
-  if (PACK16) return (s[i * kRowWords + (j >> 1)] >> ((j & 1) << 4)) & 0xffffu;
-  return s[i * kRowWords + j];
+  if (PACK16) return (s[i * kRowWords<true> + (j >> 1)] >> ((j & 1) << 4)) & 0xffffu;
+  return s[i * kRowWords<false> + j];
 }
 
 // word 3 of a raw 32-bit buffer resource on the gfx9 family

@@ -299,10 +299,11 @@ void brute_launch_as(iso_ctx *ctx, const iso::SampleGrid &g, int64_t F, const Pt
 // bits[s*F + i] = min(bits[s*F + i], squared distance of sample i to set s)
 void brute_launch(iso_ctx *ctx, const iso::SampleGrid &g, int64_t F, const Pt *pts,
                   const int64_t *d_off, int S, int64_t avg, uint32_t *bits) {
-  // the shape of a lane's block that costs the least vector instructions, a point's
+  // The shape of a lane's block that costs the least vector instructions, a point's
   // for a block times the blocks: 2 x 4 x 4 unless a short axis would leave most of
-  // it empty, which shows from 64 workgroups of such blocks on (100,000 samples on a line along x, y, z against 5,000 points: 171, 279,
-  // 218 us by 2 x 4 x 4 or 8 x 4 x 1, 93, 83, 71 by lines; 300 x 1 x 300: 126, 71)
+  // it empty, which shows from 64 workgroups of such blocks on (5,000 points, 100,000
+  // samples on a line along x, y, z: 171, 279, 218 us by 2 x 4 x 4 or 8 x 4 x 1, by
+  // lines 93, 83, 71; 300 x 1 x 300: 126, 71; 40 x 40 x 2, below: 43, 47).
   const auto cost = [&](int tx, int ty, int tz, int per_block) {
     return (int64_t)((g.nx + tx - 1) / tx) * ((g.ny + ty - 1) / ty) * ((g.nz + tz - 1) / tz) * per_block;
   };

@@ -11,8 +11,8 @@
 //   - one workgroup (1024 lanes, 16 waves) owns one unordered pair (or one
 //     voxel slice of it when there are too few pairs to fill 256 CUs); the
 //     pair's joint histogram is privatised in LDS (32-bit counters for
-//     H <= 128: 64 KB; 16-bit counters packed two per dword for H <= 256:
-//     128 KB of the 160 KB LDS), 128 words to a row whatever H is;
+//     H <= 128: 68 KB; 16-bit counters packed two per dword for H <= 256:
+//     128 KB of the 160 KB LDS), a row as long whatever H is;
 //   - bins are computed exactly in fixed point, and 16-bit counters hand on
 //     32,768 of their count before they can wrap (iso_bins.hpp);
 //   - slices of one pair leave their LDS histograms in memory, and a kernel adds
@@ -110,7 +110,7 @@ struct HistLds {
 // counter; returns where they are then (null: in LDS, and gh is zero again).
 template <bool PACK16>
 __device__ __forceinline__ uint32_t *take_back(uint32_t *s_hist, uint32_t *gh, int H) {
-  const int tid = threadIdx.x, words = H * iso::kRowWords;
+  const int tid = threadIdx.x, words = H * iso::kRowWords<PACK16>;
   bool fits = true;
   // several words per lane under way at a time: they come from beyond the L2
   constexpr int kAhead = 8;
@@ -119,7 +119,8 @@ __device__ __forceinline__ uint32_t *take_back(uint32_t *s_hist, uint32_t *gh, i
 #pragma unroll
     for (int q = 0; q < kAhead; ++q) {
       const int w = w0 + q * kBlock;
-      const int r = w / iso::kRowWords, c = (PACK16 ? 2 : 1) * (w % iso::kRowWords);
+      constexpr int kRow = iso::kRowWords<PACK16>;
+      const int r = w / kRow, c = (PACK16 ? 2 : 1) * (w % kRow);
       lo[q] = w < words && c < H ? gh[r * H + c] : 0u;
       hi[q] = PACK16 && w < words && c + 1 < H ? gh[r * H + c + 1] : 0u;
     }
@@ -190,12 +191,12 @@ template <bool PACK16, int STEP>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(PACK16 ? 4 : 8))) void hist_nmi_kernel(HistArgs a) {
   extern __shared__ uint4 s_dyn[];
   uint32_t *s_hist = reinterpret_cast<uint32_t *>(s_dyn);
-  HistLds<PACK16> &s = *reinterpret_cast<HistLds<PACK16> *>(s_hist + a.H * iso::kRowWords);
+  HistLds<PACK16> &s = *reinterpret_cast<HistLds<PACK16> *>(s_hist + a.H * iso::kRowWords<PACK16>);
 
   const int tid = threadIdx.x;
   const int H = a.H;
   const int HH = H * H;
-  const int words = H * iso::kRowWords;
+  const int words = H * iso::kRowWords<PACK16>;
 
   // Workgroups that run on an XCD at the same time take the pairs of one tile
   // of the pair matrix, slice by slice, so each value read serves several of
@@ -259,7 +260,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(PACK16 ?
     for (int w = tid; w < words; w += kBlock) {
       const uint32_t v = s_hist[w];
       if (v) {
-        const int r = w / iso::kRowWords, c = w % iso::kRowWords;
+        const int r = w / iso::kRowWords<PACK16>, c = w % iso::kRowWords<PACK16>;
         if (PACK16) {
           const uint32_t lo = v & 0xffffu, hi = v >> 16;
           if (lo && 2 * c < H) atomicAdd(&gh[r * H + 2 * c], lo);
@@ -293,7 +294,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(PACK16 ?
 // what 16-bit counters handed on).  A lane per 16 bytes of a histogram.
 template <bool PACK16>
 __global__ __launch_bounds__(256) void merge_kernel(HistArgs a) {
-  const int quads = a.H * iso::kRowWords / 4, q = blockIdx.x * 256 + threadIdx.x;
+  const int quads = a.H * iso::kRowWords<PACK16> / 4, q = blockIdx.x * 256 + threadIdx.x;
   if (q >= quads) return;
   const uint4 *part = (const uint4 *)a.parts + (int64_t)blockIdx.y * a.slices * quads + q;
   uint32_t lo[4] = {}, hi[4] = {};
@@ -307,7 +308,8 @@ __global__ __launch_bounds__(256) void merge_kernel(HistArgs a) {
       if (PACK16) hi[e] += w[e] >> 16;
     }
   }
-  const int H = a.H, row = 4 * q / iso::kRowWords, w = 4 * q % iso::kRowWords;
+  constexpr int kRow = iso::kRowWords<PACK16>;
+  const int H = a.H, row = 4 * q / kRow, w = 4 * q % kRow;
   uint32_t *gh = a.ghist + (int64_t)blockIdx.y * H * H + row * H;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
@@ -322,7 +324,7 @@ template <bool PACK16>
 __global__ __launch_bounds__(kBlock) void finish_kernel(HistArgs a) {
   extern __shared__ uint4 s_dyn[];
   uint32_t *s_hist = reinterpret_cast<uint32_t *>(s_dyn);
-  HistLds<PACK16> &s = *reinterpret_cast<HistLds<PACK16> *>(s_hist + a.H * iso::kRowWords);
+  HistLds<PACK16> &s = *reinterpret_cast<HistLds<PACK16> *>(s_hist + a.H * iso::kRowWords<PACK16>);
   const int task = blockIdx.x;
   const int2 tk = a.tasks[task];
   iso::clear_pair_lds(s.pair);
@@ -491,7 +493,7 @@ static int64_t processed_voxels(int64_t F, uint32_t flags) {
 
 size_t hist_parts_bytes(const iso_ctx *ctx, int64_t F, int H, uint32_t flags, int64_t nt) {
   const int64_t slices = slice_count(ctx, processed_voxels(F, flags), nt, H > 128);
-  return slices > 1 ? sizeof(uint32_t) * (size_t)(nt * slices) * H * kRowWords : 0;
+  return slices > 1 ? sizeof(uint32_t) * (size_t)(nt * slices) * H * row_words(H) : 0;
 }
 
 // Launches the histogram+NMI kernel over a device task list.
@@ -546,7 +548,7 @@ int hist_launch(iso_ctx *ctx, const float *d_fields, int n, int64_t F, int H, in
   if (nt <= 0) return ISO_OK;
   const bool pack16 = H > 128;
   const bool nmi32 = (flags & ISO_COMPAT_NMI32) != 0;
-  const size_t hist_bytes = sizeof(uint32_t) * (size_t)H * kRowWords;
+  const size_t hist_bytes = sizeof(uint32_t) * (size_t)H * row_words(H);
   const size_t lds = hist_bytes + (pack16 ? sizeof(HistLds<true>) : sizeof(HistLds<false>));
   const int64_t processed = processed_voxels(F, flags);
   // variants: 16-bit counters with 1 or 2 rounds of 8 values on their way,
@@ -565,7 +567,8 @@ int hist_launch(iso_ctx *ctx, const float *d_fields, int n, int64_t F, int H, in
     for (int v = 0; v < 6 && attr_err == hipSuccess; ++v)
       attr_err = hipFuncSetAttribute(
           kern[v], hipFuncAttributeMaxDynamicSharedMemorySize,
-          v < 2 || v == 4 ? 65536 + (int)sizeof(HistLds<false>) : 131072 + (int)sizeof(HistLds<true>));
+          v < 2 || v == 4 ? 128 * 4 * kRowWords<false> + (int)sizeof(HistLds<false>)
+                          : 256 * 4 * kRowWords<true> + (int)sizeof(HistLds<true>));
   });
   ISO_HIP_CHECK(ctx, attr_err);
   const int64_t slices = slice_count(ctx, processed, nt, pack16);
@@ -601,7 +604,7 @@ int hist_launch(iso_ctx *ctx, const float *d_fields, int n, int64_t F, int H, in
   if (pack16) variant == 0 ? launch(hist_nmi_kernel<true, 1>) : launch(hist_nmi_kernel<true, 2>);
   else variant == 0 ? launch(hist_nmi_kernel<false, 4>) : launch(hist_nmi_kernel<false, 8>);
   if (a.parts && slices > 1) {
-    const dim3 mg((unsigned)((H * kRowWords / 4 + 255) / 256), (unsigned)nt);
+    const dim3 mg((unsigned)((H * row_words(H) / 4 + 255) / 256), (unsigned)nt);
     if (pack16) {
       hipLaunchKernelGGL(merge_kernel<true>, mg, dim3(256), 0, ctx->stream, a);
       hipLaunchKernelGGL(finish_kernel<true>, dim3((unsigned)nt), dim3(kBlock), lds, ctx->stream, a);

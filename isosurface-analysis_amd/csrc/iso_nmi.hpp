@@ -108,7 +108,7 @@ struct PairLds {
   static constexpr int kH = PACK16 ? 256 : 128;    // most bins per axis
   static constexpr int kRows = kH / kHistWaves;    // rows of a wave
   static constexpr int kCols = kH / 64;            // columns of a lane
-  static constexpr int kBins = PACK16 ? 10240 : 6144;  // most listed bins
+  static constexpr int kBins = PACK16 ? 10240 : 4608;  // most listed bins
   union {
     uint8_t colpre[kHistWaves][kH];
     uint16_t bins[kBins];
@@ -145,6 +145,11 @@ template <bool PACK16>
 constexpr int kSlots = PairLds<PACK16>::kH * 64 / kHistBlock;
 
 template <bool PACK16>
+__device__ __forceinline__ uint2 slot_words(const uint32_t *s_hist, int row, int l) {
+  return reinterpret_cast<const uint2 *>(s_hist)[row * (kRowWords<PACK16> / 2) + l];
+}
+
+template <bool PACK16>
 __device__ __forceinline__ uint32_t slot_count(uint2 v, int c) {
   if (PACK16) return ((c < 2 ? v.x : v.y) >> (16 * (c & 1))) & 0xffffu;
   return c == 0 ? v.x : v.y;
@@ -167,7 +172,7 @@ __device__ __attribute__((always_inline)) uint32_t list_bins(const uint32_t *s_h
     const int k = q * kHistBlock + (int)threadIdx.x;
     if (k >= H * 64) break;
     uint2 v = make_uint2(0u, 0u);
-    if (!gh) v = reinterpret_cast<const uint2 *>(s_hist)[k];
+    if (!gh) v = slot_words<PACK16>(s_hist, k >> 6, k & 63);
 #pragma unroll
     for (int c = 0; c < kPer; ++c) {
       const int j = (k & 63) * kPer + c;
@@ -253,7 +258,7 @@ __device__ __attribute__((always_inline)) void emit_chains(uint32_t *s_hist, int
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     slot[r] = make_uint2(0u, 0u);
-    if (!GH && i0 + r < H) slot[r] = reinterpret_cast<const uint2 *>(s_hist)[(i0 + r) * 64 + l];
+    if (!GH && i0 + r < H) slot[r] = slot_words<PACK16>(s_hist, i0 + r, l);
   }
   auto count = [&](int r, int c) -> uint32_t {
     if (GH)
