@@ -477,7 +477,10 @@ static int64_t slice_count(const iso_ctx *ctx, int64_t processed, int64_t nt, bo
   const int64_t cap = (int64_t)(pack16 ? 1 : 2) * ctx->cu_count;
   int64_t slices = 1, best = INT64_MAX;
   for (int64_t k = 1; nt < cap && k <= std::max<int64_t>(1, processed / 16384); ++k) {
-    const int64_t cost = (nt * k + cap - 1) / cap * (processed / k + (k > 1 ? 32768 : 0));
+    const int64_t rounds = (nt * k + cap - 1) / cap;
+    // (no larger k can cost less than its rounds' starts and the voxels' share)
+    if (rounds * 32768 + nt * (processed - k) / cap > best) break;
+    const int64_t cost = rounds * (processed / k + (k > 1 ? 32768 : 0));
     if (cost < best) {
       best = cost;
       slices = k;
