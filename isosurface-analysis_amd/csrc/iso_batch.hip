@@ -336,7 +336,7 @@ int iso_ism_batch(iso_ctx *ctx, iso_ism_job *jobs, int njobs, int extractor, int
     // tasks of a launch: what the memory for the chains' inputs holds (the tasks'
     // largest field comes first)
     const bool graph = (flags & ISO_BATCH_GRAPH) != 0;
-    const int most = nmi32 ? iso::chain_tasks(ctx, H, tasks[0].F, nt) : nt;
+    const int most = nmi32 ? iso::chain_tasks(ctx, H, tasks[0].F, nt, pack16 ? 2048 : 512) : nt;
     if (nmi32) ISO_TRY(iso::chain_get(ctx, most, H, tasks[0].F, ba.chains));
     auto launch = [&](const BatchTask *d_tasks) -> int {
       for (int i0 = 0; i0 < nt; i0 += most) {

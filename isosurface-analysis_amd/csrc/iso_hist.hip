@@ -446,8 +446,8 @@ int nmi_logs(iso_ctx *ctx, const float **out) {
   return ISO_OK;
 }
 
-int chain_tasks(const iso_ctx *ctx, int H, int64_t F, int64_t ntasks) {
-  size_t limit = kChainBytes;
+int chain_tasks(const iso_ctx *ctx, int H, int64_t F, int64_t ntasks, int limit_mib) {
+  size_t limit = (size_t)limit_mib << 20;
   if (const char *e = std::getenv("ISO_NMI_CHAIN_MIB")) {  // read per call
     const long v = std::atol(e);
     if (v > 0) limit = (size_t)std::min<long>(v, 65536) << 20;
@@ -510,7 +510,7 @@ int hist_nmi_tasks(iso_ctx *ctx, const float *d_fields, int n, int64_t F, int H,
   HistBufs b;
   int most = kMaxTasksPerLaunch;
   if (nmi32) {
-    most = std::min(most, chain_tasks(ctx, H, F, ntasks));
+    most = std::min(most, chain_tasks(ctx, H, F, ntasks, pack16 ? 2048 : 1024));
     ISO_TRY(chain_get(ctx, most, H, F, b.chains));
   }
   const int64_t processed = processed_voxels(F, flags);

@@ -709,11 +709,16 @@ int nmi_logs(iso_ctx *ctx, const float **out);
 int nmi_logs_fill(iso_ctx *ctx, float *d_logs);
 
 // Tasks of a launch in the reference's float order, ntasks at most: as many whole
-// rounds of workgroups as kChainBytes of the chains' inputs hold (F: the tasks'
-// largest), one task in any case.  ISO_NMI_CHAIN_MIB in the environment sets
-// another limit.
-constexpr size_t kChainBytes = (size_t)2 << 30;
-int chain_tasks(const iso_ctx *ctx, int H, int64_t F, int64_t ntasks);
+// rounds of workgroups as limit_mib MiB of the chains' inputs hold (F: the tasks'
+// largest), one task in any case.  ISO_NMI_CHAIN_MIB in the environment sets another
+// limit.  Every launch ends with its last pairs and its folds, so few large ones are
+// better, until their inputs no longer stay in the caches.  One volume's pairs: 2
+// GiB, 1 GiB up to 128 bins (600x248x248 front, 256 bins, by 2 GiB, 1 GiB, 512 MiB:
+// 2.04, 2.13, 2.24 ms; 256 isovalues of 60,000 voxels, 128 bins: 1.89, 1.86, 1.92).
+// A batch, whose pairs come from queues: 2 GiB, 512 MiB up to 128 bins (48 volumes,
+// 186,551 pairs, 128 bins, by 2 GiB, 1 GiB, 512 MiB: 57.4, 55.7, 53.3 ms; 256 bins:
+// 66.6, 68.8, 73.8).
+int chain_tasks(const iso_ctx *ctx, int H, int64_t F, int64_t ntasks, int limit_mib);
 
 // The context's ChainBufs for a launch of ntasks tasks.
 int chain_get(iso_ctx *ctx, int64_t ntasks, int H, int64_t F, ChainBufs &b);
