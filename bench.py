@@ -31,8 +31,8 @@ VALU_LANES_PER_S = FP32_PEAK_TFLOPS * 1e12 / 2
 # (FETCH_SIZE x 1.9998, WRITE_SIZE x 1.0); commands and per-kernel table in
 # profiles/ism_c2_600x248x248_k100_hbm_traffic.md.  The profiler cannot run
 # inside this process, so the measured figures are carried here.
-HIST_TRAFFIC_DEFAULT = 7359920930
-WALK_TRAFFIC_DEFAULT = 5823908397
+HIST_TRAFFIC_DEFAULT = 7370948841
+WALK_TRAFFIC_DEFAULT = 5583217873
 
 
 def log(*a):

@@ -271,13 +271,14 @@ typedef struct {
 } iso_ism_job;
 
 /* The ISMs of several volumes (any sizes) in one call: extraction and fields
- * volume by volume, then every pair of every ISM in one persistent histogram
- * + NMI launch that pulls pair tasks from a device queue, largest fields
- * first.  Each map equals what iso_ism_volume returns for the same job.
+ * volume by volume, then every pair of every ISM in persistent histogram + NMI
+ * launches that pull pair tasks from device queues, largest fields first (one
+ * launch, or with ISO_COMPAT_NMI32 as many as its working memory of at most 2 GiB
+ * needs).  Each map equals what iso_ism_volume returns for the same job.
  * Replaces running the reference's `single` process once per volume
  * (runtime/src/Single.cpp:193-256, one histogram launch per 1M-voxel chunk per
  * volume).  h_stats (may be NULL): ms_df covers extraction + fields of all
- * volumes, ms_hist the pair launch. */
+ * volumes, ms_hist the pair stage. */
 int iso_ism_batch(iso_ctx *ctx, iso_ism_job *jobs, int njobs, int extractor, int ds, int H,
                   int df_method, uint32_t flags, iso_ism_stats *h_stats);
 

@@ -2,10 +2,12 @@
 //
 // Per volume, extraction and distance fields run as in iso_ism_volume; the
 // fields of every volume land in one buffer.  Then all unordered pairs of
-// all ISMs go through ONE persistent histogram+NMI launch: a few workgroups
-// per CU pull pair tasks (largest field first) from a device queue until it
-// is empty, so volumes from 48^3 to 256^3 share the machine without tail
-// effects and without a launch per ISM.
+// all ISMs go through persistent histogram+NMI launches: one or two workgroups
+// per CU pull pair tasks (largest field first) from device queues until they
+// are empty, so volumes from 48^3 to 256^3 share the machine without a launch,
+// and its tail, per ISM.  One launch in the double form; in the reference's float
+// order as many as the chains' inputs need room for, each with a launch that folds
+// its chains (186,551 pairs at 128 bins: 32).
 //
 // Per-pair semantics are those of hist_nmi_kernel (JointHistogram.cu:24-162):
 // exact integer joint counts privatised in LDS; NMI in the reference's float
@@ -304,7 +306,7 @@ int iso_ism_batch(iso_ctx *ctx, iso_ism_job *jobs, int njobs, int extractor, int
     mmbase += m;
   }
   ISO_HIP_CHECK(ctx, hipEventRecord(ev[1], ctx->stream));
-  // ---- all pairs of all ISMs: one persistent launch, largest fields first
+  // ---- all pairs of all ISMs: persistent launches, largest fields first
   std::stable_sort(tasks.begin(), tasks.end(),
                    [](const BatchTask &x, const BatchTask &y) { return x.F > y.F; });
   const int nt = (int)tasks.size();

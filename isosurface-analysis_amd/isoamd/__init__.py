@@ -552,7 +552,7 @@ class Context:
 
     def ism_batch(self, vols, dims_list, isos_list, extractor: int = EXTRACT_MC, ds: int = 1,
                   H: int = 128, df_method: int = DF_LBVH, flags: int = COMPAT_ALL):
-        """ISMs of several volumes in one call (one persistent pair launch).
+        """ISMs of several volumes in one call (their pairs in persistent launches).
         Returns ([(map m x m numpy, ids (m,))] per volume, IsmStats)."""
         n = len(vols)
         jobs = (IsmJob * n)()
